@@ -125,6 +125,7 @@ def prepare(case, seed):
         d = c // h if op == "rope" else c
         angles = _randn((s, d // 2), g, std=3.0, dtype=torch.float32)
         table = torch.stack([angles.cos(), angles.sin()], dim=-1)       # built once per step, shared by all blocks
+        state["table"] = table
         if op == "rope":
             state["call"] = lambda x, weight: teletron_amd.RMSNormRopeFunction.apply(x, weight, table, EPS, h)
         else:
@@ -157,6 +158,53 @@ def run(state):
     out = state["call"](*state["inputs"])
     outs = list(out) if isinstance(out, tuple) else [out]
     return outs + list(torch.autograd.grad(outs, state["inputs"], state["grads"]))
+
+
+def exact(case, seed):
+    """What ``run`` returns, by the formulas in 64 bits (gradients by autograd)."""
+    state = prepare(case, seed)
+    op, c, h = case["op"], case["cols"], case["heads"]
+    inputs = [t.detach().double().requires_grad_(case["grad"]) for t in state["inputs"]]
+
+    def layer_norm(v):
+        d = v - v.mean(dim=-1, keepdim=True)
+        return d * torch.rsqrt(d.square().mean(dim=-1, keepdim=True) + EPS)
+
+    def rms_norm(v, weight):
+        return v * torch.rsqrt(v.square().mean(dim=-1, keepdim=True) + EPS) * weight
+
+    def rotate(v):                  # [..., tokens, D], pairs of neighbouring values
+        cos, sin = state["table"].double().unbind(-1)
+        re, im = v[..., 0::2], v[..., 1::2]
+        return torch.stack([re * cos - im * sin, re * sin + im * cos], dim=-1).flatten(-2)
+
+    if op == "adaln":
+        x, shift, scale = inputs
+        outs = [layer_norm(x) * (1 + scale) + shift]
+    elif op == "adaln_saved":
+        x, scale, shift = inputs
+        outs = [layer_norm(x) * (1 + scale) + shift]
+    elif op == "rmsnorm":
+        outs = [rms_norm(*inputs)]
+    elif op == "rope":
+        outs = [rotate(rms_norm(*inputs).unflatten(-1, (h, c // h)).transpose(1, 2)).transpose(1, 2).flatten(-2)]
+    elif op == "rope_heads":
+        outs = [rotate(rms_norm(*inputs))]
+    elif op == "gate":
+        x, gate, residual = inputs
+        outs = [x + gate * residual]
+    elif op == "residual_adaln":
+        x, residual, shift, scale = inputs
+        s = x + residual
+        outs = [s, layer_norm(s) * (1 + scale) + shift]
+    else:
+        x, residual, gate, weight, bias = inputs
+        s = x + gate * residual
+        outs = [s, layer_norm(s) * weight + bias]
+    if not case["grad"]:
+        return outs[0] if len(outs) == 1 else tuple(outs)
+    grads = torch.autograd.grad(outs, inputs, [g.double() for g in state["grads"]])
+    return [o.detach() for o in outs] + list(grads)
 
 
 def work(case):
