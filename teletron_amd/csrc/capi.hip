@@ -126,10 +126,12 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   if (idx < 0) return TT_ERR_UNSUPPORTED;
   const int slots = narrow ? kNarrowL[idx] : 64 * kWideW[idx] * kWideP[idx];
   const bool full = (slots == packs);
+  // a row of whole 128-byte lines or not: see enum Rows
+  const int mode = full ? kFull : (cols * 2) % 128 == 0 ? kMasked : kRagged;
   KernelInfo k;
   if (res) {
     if (narrow || kind != kAdaLN || dir == kBwdSaved || dir == kFwdXn) return TT_ERR_UNSUPPORTED;
-    k = res == 2 ? resnorm_gated_kernel(dir == kBwd, idx, full) : resnorm_plain_kernel(dir == kBwd, idx, full);
+    k = res == 2 ? resnorm_gated_kernel(dir == kBwd, idx, mode) : resnorm_plain_kernel(dir == kBwd, idx, mode);
   } else if (rope) {
     if (kind != kRMS || dir == kBwdSaved || dir == kFwdXn) return TT_ERR_UNSUPPORTED;
     k = rms_rope_kernel(narrow, dir == kBwd, idx, full, rope_heads);
@@ -137,13 +139,13 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
     if (kind != kAdaLN) return TT_ERR_UNSUPPORTED;
     k = adaln_fwd_xnorm_kernel(narrow, idx, full);
   } else if (kind == kAdaLN)
-    k = dir == kFwd ? adaln_fwd_kernel(narrow, idx, full)
-      : dir == kBwd ? adaln_bwd_kernel(narrow, idx, full) : adaln_bwd_saved_kernel(narrow, idx, full);
+    k = dir == kFwd ? adaln_fwd_kernel(narrow, idx, mode)
+      : dir == kBwd ? adaln_bwd_kernel(narrow, idx, mode) : adaln_bwd_saved_kernel(narrow, idx, full);
   else if (kind == kRMS)
-    k = dir == kFwd ? rms_fwd_kernel(narrow, idx, full)
-      : dir == kBwd ? rms_bwd_kernel(narrow, idx, full) : rms_bwd_saved_kernel(narrow, idx, full);
+    k = dir == kFwd ? rms_fwd_kernel(narrow, idx, mode)
+      : dir == kBwd ? rms_bwd_kernel(narrow, idx, mode) : rms_bwd_saved_kernel(narrow, idx, full);
   else
-    k = dir == kFwd ? gate_fwd_kernel(narrow, idx, full) : gate_bwd_kernel(narrow, idx, full);
+    k = dir == kFwd ? gate_fwd_kernel(narrow, idx, mode) : gate_bwd_kernel(narrow, idx, mode);
   if (!k.fn) return TT_ERR_UNSUPPORTED;
 
   int cus = 0, per_cu = 0;

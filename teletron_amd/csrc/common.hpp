@@ -44,6 +44,59 @@ __device__ __forceinline__ u32x4 load_cached(const void* base, size_t elem_off) 
   return *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(base) + elem_off);
 }
 
+// How the rows of a wide kernel lie on its lane slots and in memory.
+enum Rows : int {
+  kMasked = 0,   // fewer packs than lane slots; a row is a whole number of 128-byte lines
+  kFull = 1,     // every lane slot holds a pack
+  kRagged = 2,   // as kMasked, but rows start anywhere inside a line (cols % 64 != 0)
+};
+// Where rows are not whole lines, the segments of neighbouring waves and rows share the lines at
+// their ends.  A written-through store sends its part of such a line to memory on its own, and
+// memory turns a part of a 64-byte sector into a read and a write; those lines have to meet in
+// the L2 first.  Two ways (SHORT of the kernels):
+//   short rows (at most 6 segments of 64 packs, norm and ungated residual + norm kernels): every
+//     store is a plain "nt" store that the L2 writes back, and the loads, which share lines in the
+//     same way, are cached ones.
+//   otherwise: only the lanes whose line is shared do that, the others write through (written back
+//     whole, the backward kernels lose 20 %: 80000 x 4416, 352 -> 419 us); nt loads.
+// us forward / backward of 60000 rows, everything written through | all written back | shared lines only:
+//   AdaLN 1000 columns 52 / 79 | 45 / 62 | 44 / 71;  2200: 154 / 198 | 98 / 162 | 117 / 184
+//         3688: 185 / 290 | 162 / 233 | 139 / 226;  4424: 264 / 337 | 181 / 334 | 185 / 263
+//   RMS   1544: 88 / 151 | 66 / 103 | 64 / 102;  2200: 139 / 226 | 97 / 147 | 97 / 155;  4600: 257 / 349 | 191 / 299 | 185 / 277
+//   gate  1000: 73 / 75 | 66 / 58 | 61 / 64;  3000: 246 / 247 | 188 / 192 | 179 / 182
+//   residual + norm 1544: 179 / 187 | 133 / 137 | 128 / 142;  gated: 179 / 232 | 134 / 207 | 129 / 192
+constexpr bool short_rows(int W, int P) { return W * P <= 6; }
+
+template <int ROWS, bool SHORT>
+__device__ __forceinline__ u32x4 load_row(const void* base, size_t elem_off) {
+  if constexpr (ROWS == kRagged && SHORT) return load_cached(base, elem_off);
+  else return load_stream(base, elem_off);
+}
+// Stores the pack of slot `seg + lane` (seg: first slot of the wave's segment, a multiple of 64) of a row.
+template <int ROWS, bool SHORT>
+__device__ __forceinline__ void store_row(void* base, int64_t row, int packs, int seg, int lane, u32x4 v) {
+  const int64_t pack = row * packs + seg + lane;
+  u32x4* p = reinterpret_cast<u32x4*>(base) + pack;
+  if constexpr (ROWS != kFull) {
+    if (seg + lane >= packs) return;
+  }
+  if constexpr (ROWS == kRagged) {
+    bool shared = true;
+    if constexpr (!SHORT) {
+      // position of the pack inside its 128-byte line, and whether the segment holds that whole line
+      const int at = (static_cast<int>(reinterpret_cast<uintptr_t>(p) >> 4)) & 7;
+      const int last = packs - seg < 64 ? packs - seg - 1 : 63;
+      shared = lane < at || lane + 7 - at > last;
+    }
+    if (shared) {
+      if constexpr (SHORT) __builtin_nontemporal_store(v, p);
+      else *p = v;
+      return;
+    }
+  }
+  store_stream(p, 0, v);
+}
+
 // ---------------------------------------------------------------- bf16 <-> fp32
 __device__ __forceinline__ void unpack8(u32x4 raw, float (&f)[8]) {
 #pragma unroll

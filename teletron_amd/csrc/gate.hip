@@ -2,6 +2,6 @@
 #include "kernel_table.hpp"
 
 namespace tt {
-KernelInfo gate_fwd_kernel(bool narrow, int idx, bool full) { return lookup_gate<kGateFwd>(narrow, idx, full); }
-KernelInfo gate_bwd_kernel(bool narrow, int idx, bool full) { return lookup_gate<kGateBwd>(narrow, idx, full); }
+KernelInfo gate_fwd_kernel(bool narrow, int idx, int rows) { return lookup_gate<kGateFwd>(narrow, idx, rows); }
+KernelInfo gate_bwd_kernel(bool narrow, int idx, int rows) { return lookup_gate<kGateBwd>(narrow, idx, rows); }
 }  // namespace tt

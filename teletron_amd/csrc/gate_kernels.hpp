@@ -22,8 +22,9 @@ struct GateArgs {
 
 enum GateMode : int { kGateFwd = 0, kGateBwd = 1 };
 
-template <int MODE, int W, int P, int R, int Q, bool FULL>
+template <int MODE, int W, int P, int R, int Q, int ROWS>
 __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
+  constexpr bool FULL = ROWS == kFull, SHORT = false;   // SHORT: see enum Rows
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int q = wave / W;
@@ -58,8 +59,8 @@ __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
         rawb[r][p] = u32x4{0, 0, 0, 0};
         if (r0 + r < S && act[p]) {
           const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
-          rawa[r][p] = load_stream(a.a, off);
-          rawb[r][p] = load_stream(a.b, off);
+          rawa[r][p] = load_row<ROWS, SHORT>(a.a, off);
+          rawb[r][p] = load_row<ROWS, SHORT>(a.b, off);
         }
       }
   };
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
             acc0[p][j] = fmaf(af[r][p][j], bf[r][p][j], acc0[p][j]);
           }
         }
-        if (row0 + r < S && act[p]) store_stream(a.out, (size_t)(row * C + col[p]), pack8(o));
+        if (row0 + r < S) store_row<ROWS, SHORT>(a.out, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
       }
     }
   }

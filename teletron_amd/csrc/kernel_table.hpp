@@ -62,8 +62,10 @@ constexpr int bwd_wide_R(int W, int P) { return 1; }
 // 150000 x 2048: 300.9 -> 290.0; 118800 x 3072: 358.4 -> 348.9; 60000 x 6144: 381.2 -> 355.4;
 // 300000 x 1024: 290.7 -> 288.5.  Worse with R = 2: 512 columns (156.9 -> 169.0), 4096
 // (356.6 -> 368.8), 8192 (358.0 -> 399.5), and 5120 (ten waves: spills).  RMSNorm (one reduction
-// per row) is 2-3 % slower with R = 2 everywhere.
-constexpr int adaln_bwd_wide_R(int W, int P) {
+// per row) is 2-3 % slower with R = 2 everywhere.  Ragged rows lose with two as well (60000 x 2200:
+// 162 -> 184 us, 1000: 71 -> 77 us).
+constexpr int adaln_bwd_wide_R(int W, int P, int rows) {
+  if (rows == kRagged) return bwd_wide_R(W, P);
   return ((P == 1 && W >= 2 && W <= 4) || (P == 2 && (W == 3 || W == 6))) ? 2 : bwd_wide_R(W, P);
 }
 constexpr int fwd_wide_Q(int W, int P) {
@@ -93,15 +95,15 @@ inline int select_narrow(int packs) {
   return -1;
 }
 
-template <int KIND, int W, int P, bool FULL>
+template <int KIND, int W, int P, int ROWS>
 KernelInfo info_fwd_wide() {
   constexpr int R = fwd_wide_R(W, P), Q = fwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_fwd_wide<KIND, W, P, R, Q, FULL>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_fwd_wide<KIND, W, P, R, Q, ROWS>), 64 * W * Q, Q * R, P * R};
 }
-template <int KIND, int W, int P, bool FULL>
+template <int KIND, int W, int P, int ROWS>
 KernelInfo info_bwd_wide() {
-  constexpr int R = KIND == kAdaLN ? adaln_bwd_wide_R(W, P) : bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_bwd_wide<KIND, W, P, R, Q, FULL>), 64 * W * Q, Q * R, P * R};
+  constexpr int R = KIND == kAdaLN ? adaln_bwd_wide_R(W, P, ROWS) : bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
+  return {reinterpret_cast<const void*>(&norm_bwd_wide<KIND, W, P, R, Q, ROWS>), 64 * W * Q, Q * R, P * R};
 }
 template <int KIND, int W, int P, bool FULL>
 KernelInfo info_bwd_saved_wide() {
@@ -137,7 +139,7 @@ constexpr int fwd_xn_wide_Q(int W, int P) { return 1; }
 template <int W, int P, bool FULL>
 KernelInfo info_fwd_xn_wide() {
   constexpr int R = fwd_wide_R(W, P), Q = fwd_xn_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_fwd_wide<kAdaLN, W, P, R, Q, FULL, false, true>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_fwd_wide<kAdaLN, W, P, R, Q, FULL ? kFull : kMasked, false, true>), 64 * W * Q, Q * R, P * R};
 }
 template <int L, bool FULL>
 KernelInfo info_fwd_xn_narrow() {
@@ -161,17 +163,22 @@ inline KernelInfo lookup_fwd_xn(bool narrow, int idx, bool full) {
   return {nullptr, 0, 0, 0};
 }
 
+// Picks the instantiation of a wide kernel for the row mode `rows` (enum Rows).
+#define TT_ROWS(INFO, ...)                                     \
+  return rows == kFull     ? INFO<__VA_ARGS__, kFull>()        \
+         : rows == kRagged ? INFO<__VA_ARGS__, kRagged>()      \
+                           : INFO<__VA_ARGS__, kMasked>();
 template <int KIND>
-KernelInfo lookup_fwd(bool narrow, int idx, bool full) {
+KernelInfo lookup_fwd(bool narrow, int idx, int rows) {
   if (narrow) {
     switch (idx) {
-#define X(i, L) case i: return full ? info_fwd_narrow<KIND, L, true>() : info_fwd_narrow<KIND, L, false>();
+#define X(i, L) case i: return rows == kFull ? info_fwd_narrow<KIND, L, true>() : info_fwd_narrow<KIND, L, false>();
       TT_NARROW_LIST(X)
 #undef X
     }
   } else {
     switch (idx) {
-#define X(i, W, P) case i: return full ? info_fwd_wide<KIND, W, P, true>() : info_fwd_wide<KIND, W, P, false>();
+#define X(i, W, P) case i: TT_ROWS(info_fwd_wide, KIND, W, P)
       TT_WIDE_LIST(X)
 #undef X
     }
@@ -179,16 +186,16 @@ KernelInfo lookup_fwd(bool narrow, int idx, bool full) {
   return {nullptr, 0, 0, 0};
 }
 template <int KIND>
-KernelInfo lookup_bwd(bool narrow, int idx, bool full) {
+KernelInfo lookup_bwd(bool narrow, int idx, int rows) {
   if (narrow) {
     switch (idx) {
-#define X(i, L) case i: return full ? info_bwd_narrow<KIND, L, true>() : info_bwd_narrow<KIND, L, false>();
+#define X(i, L) case i: return rows == kFull ? info_bwd_narrow<KIND, L, true>() : info_bwd_narrow<KIND, L, false>();
       TT_NARROW_LIST(X)
 #undef X
     }
   } else {
     switch (idx) {
-#define X(i, W, P) case i: return full ? info_bwd_wide<KIND, W, P, true>() : info_bwd_wide<KIND, W, P, false>();
+#define X(i, W, P) case i: TT_ROWS(info_bwd_wide, KIND, W, P)
       TT_WIDE_LIST(X)
 #undef X
     }
@@ -200,12 +207,12 @@ KernelInfo lookup_bwd(bool narrow, int idx, bool full) {
 template <int W, int P, bool FULL>
 KernelInfo info_fwd_rope_wide() {
   constexpr int R = fwd_wide_R(W, P), Q = fwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_fwd_wide<kRMS, W, P, R, Q, FULL, true>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_fwd_wide<kRMS, W, P, R, Q, FULL ? kFull : kMasked, true>), 64 * W * Q, Q * R, P * R};
 }
 template <int W, int P, bool FULL>
 KernelInfo info_bwd_rope_wide() {
   constexpr int R = bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_bwd_wide<kRMS, W, P, R, Q, FULL, true>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_bwd_wide<kRMS, W, P, R, Q, FULL ? kFull : kMasked, true>), 64 * W * Q, Q * R, P * R};
 }
 template <int L, bool FULL>
 KernelInfo info_fwd_rope_narrow() {
@@ -258,10 +265,10 @@ inline KernelInfo lookup_rope(bool narrow, bool backward, int idx, bool full, in
   return {nullptr, 0, 0, 0};
 }
 
-template <int MODE, int W, int P, bool FULL>
+template <int MODE, int W, int P, int ROWS>
 KernelInfo info_gate_wide() {
   constexpr int R = bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&gate_wide<MODE, W, P, R, Q, FULL>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&gate_wide<MODE, W, P, R, Q, ROWS>), 64 * W * Q, Q * R, P * R};
 }
 template <int MODE, int L, bool FULL>
 KernelInfo info_gate_narrow() {
@@ -269,16 +276,16 @@ KernelInfo info_gate_narrow() {
   return {reinterpret_cast<const void*>(&gate_narrow<MODE, L, R, NW, FULL>), 64 * NW, NW * R * (64 / L), R};
 }
 template <int MODE>
-KernelInfo lookup_gate(bool narrow, int idx, bool full) {
+KernelInfo lookup_gate(bool narrow, int idx, int rows) {
   if (narrow) {
     switch (idx) {
-#define X(i, L) case i: return full ? info_gate_narrow<MODE, L, true>() : info_gate_narrow<MODE, L, false>();
+#define X(i, L) case i: return rows == kFull ? info_gate_narrow<MODE, L, true>() : info_gate_narrow<MODE, L, false>();
       TT_NARROW_LIST(X)
 #undef X
     }
   } else {
     switch (idx) {
-#define X(i, W, P) case i: return full ? info_gate_wide<MODE, W, P, true>() : info_gate_wide<MODE, W, P, false>();
+#define X(i, W, P) case i: TT_ROWS(info_gate_wide, MODE, W, P)
       TT_WIDE_LIST(X)
 #undef X
     }
@@ -306,23 +313,25 @@ constexpr int res_fwd_Q(int W, int P) {
 constexpr int res_bwd_Q(int W, int P, bool gated) {
   return res_waves_Q(W, P);
 }
-template <int W, int P, bool FULL, bool GATED>
+template <int W, int P, int ROWS, bool GATED>
 KernelInfo info_res_fwd() {
   constexpr int R = 1, Q = res_fwd_Q(W, P);
-  return {reinterpret_cast<const void*>(&resnorm_fwd_wide<W, P, R, Q, FULL, GATED>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&resnorm_fwd_wide<W, P, R, Q, ROWS, GATED>), 64 * W * Q, Q * R, P * R};
 }
-template <int W, int P, bool FULL, bool GATED>
+template <int W, int P, int ROWS, bool GATED>
 KernelInfo info_res_bwd() {
   constexpr int R = 1, Q = res_bwd_Q(W, P, GATED);
-  return {reinterpret_cast<const void*>(&resnorm_bwd_wide<W, P, R, Q, FULL, GATED>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&resnorm_bwd_wide<W, P, R, Q, ROWS, GATED>), 64 * W * Q, Q * R, P * R};
 }
 template <bool GATED>
-KernelInfo lookup_res(bool backward, int idx, bool full) {
+KernelInfo lookup_res(bool backward, int idx, int rows) {
   switch (idx) {
-#define X(i, W, P)                                                                                        \
-  case i:                                                                                                 \
-    return backward ? (full ? info_res_bwd<W, P, true, GATED>() : info_res_bwd<W, P, false, GATED>())     \
-                    : (full ? info_res_fwd<W, P, true, GATED>() : info_res_fwd<W, P, false, GATED>());
+#define X(i, W, P)                                                                                            \
+  case i:                                                                                                     \
+    if (rows == kFull) return backward ? info_res_bwd<W, P, kFull, GATED>() : info_res_fwd<W, P, kFull, GATED>(); \
+    if (rows == kRagged)                                                                                      \
+      return backward ? info_res_bwd<W, P, kRagged, GATED>() : info_res_fwd<W, P, kRagged, GATED>();          \
+    return backward ? info_res_bwd<W, P, kMasked, GATED>() : info_res_fwd<W, P, kMasked, GATED>();
     TT_WIDE_LIST(X)
 #undef X
   }
@@ -349,17 +358,17 @@ KernelInfo lookup_bwd_saved(bool narrow, int idx, bool full) {
 
 // Defined one per translation unit (adaln_fwd.hip, adaln_fwd_xnorm.hip, adaln_bwd.hip, adaln_bwd_saved.hip, rms_fwd.hip, rms_bwd.hip, rms_bwd_saved.hip, rms_rope.hip, gate.hip,
 // resnorm_plain.hip, resnorm_gated.hip).
-KernelInfo adaln_fwd_kernel(bool narrow, int idx, bool full);
+KernelInfo adaln_fwd_kernel(bool narrow, int idx, int rows);
 KernelInfo adaln_fwd_xnorm_kernel(bool narrow, int idx, bool full);
-KernelInfo adaln_bwd_kernel(bool narrow, int idx, bool full);
-KernelInfo rms_fwd_kernel(bool narrow, int idx, bool full);
-KernelInfo rms_bwd_kernel(bool narrow, int idx, bool full);
+KernelInfo adaln_bwd_kernel(bool narrow, int idx, int rows);
+KernelInfo rms_fwd_kernel(bool narrow, int idx, int rows);
+KernelInfo rms_bwd_kernel(bool narrow, int idx, int rows);
 KernelInfo adaln_bwd_saved_kernel(bool narrow, int idx, bool full);
 KernelInfo rms_bwd_saved_kernel(bool narrow, int idx, bool full);
 KernelInfo rms_rope_kernel(bool narrow, bool backward, int idx, bool full, int64_t heads);
-KernelInfo gate_fwd_kernel(bool narrow, int idx, bool full);
-KernelInfo gate_bwd_kernel(bool narrow, int idx, bool full);
-KernelInfo resnorm_plain_kernel(bool backward, int idx, bool full);
-KernelInfo resnorm_gated_kernel(bool backward, int idx, bool full);
+KernelInfo gate_fwd_kernel(bool narrow, int idx, int rows);
+KernelInfo gate_bwd_kernel(bool narrow, int idx, int rows);
+KernelInfo resnorm_plain_kernel(bool backward, int idx, int rows);
+KernelInfo resnorm_gated_kernel(bool backward, int idx, int rows);
 
 }  // namespace tt

@@ -119,9 +119,10 @@ __device__ __forceinline__ void rowgroup_allsum(float (&v)[NV], float* buf, int 
 
 // ============================================================================ wide forward
 // XN: also store the normalised input before modulation (a.x_norm), paired with the y store.
-template <int KIND, int W, int P, int R, int Q, bool FULL, bool ROPE = false, bool XN = false>
+template <int KIND, int W, int P, int R, int Q, int ROWS, bool ROPE = false, bool XN = false>
 __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
   constexpr bool ADALN = (KIND == kAdaLN);
+  constexpr bool FULL = ROWS == kFull, SHORT = short_rows(W, P);
   static_assert(!ROPE || KIND == kRMS, "rotary embedding is fused behind RMSNorm only");
   static_assert(!XN || ADALN, "x_norm is an output of the AdaLN forward only");
   __shared__ float red[2][Q][W * R];
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
 #pragma unroll
       for (int p = 0; p < P; ++p) {
         raw[r][p] = u32x4{0, 0, 0, 0};
-        if (r0 + r < S && act[p]) raw[r][p] = load_stream(a.x, (size_t)((b * S + r0 + r) * C + col[p]));
+        if (r0 + r < S && act[p]) raw[r][p] = load_row<ROWS, SHORT>(a.x, (size_t)((b * S + r0 + r) * C + col[p]));
       }
   };
 
@@ -287,7 +288,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
               rope_rotate(o, fc);
             }
             if constexpr (XN) store_stream2(a.y, a.x_norm, (size_t)(row * C + col[p]), pack8(o), pack8(n));
-            else              store_stream(a.y, (size_t)(row * C + col[p]), pack8(o));
+            else              store_row<ROWS, SHORT>(a.y, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
           }
         }
         if (w == 0 && lane == 0) {
@@ -351,9 +352,10 @@ __device__ __forceinline__ void wide_write_partials(float (&acc0)[P][8], float (
 }
 
 // ============================================================================ wide backward
-template <int KIND, int W, int P, int R, int Q, bool FULL, bool ROPE = false>
+template <int KIND, int W, int P, int R, int Q, int ROWS, bool ROPE = false>
 __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
   constexpr bool ADALN = (KIND == kAdaLN);
+  constexpr bool FULL = ROWS == kFull, SHORT = short_rows(W, P);
   static_assert(!ROPE || KIND == kRMS, "rotary embedding is fused behind RMSNorm only");
   constexpr int NACC = ADALN ? 2 : 1;
   constexpr int NV = ADALN ? 3 : 2;  // reduced values per row in the main phase
@@ -422,8 +424,8 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
         }
         if (r0 + r < S && act[p]) {
           const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
-          rawx[r][p] = load_stream(a.x, off);
-          rawd[r][p] = load_stream(a.dy, off);
+          rawx[r][p] = load_row<ROWS, SHORT>(a.x, off);
+          rawd[r][p] = load_row<ROWS, SHORT>(a.dy, off);
           if constexpr (ROPE)
             load_freq8(a.freqs, (size_t)(pos[r] * a.head_dim + fcol[p]), fr[r][p]);
         }
@@ -518,7 +520,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
           if constexpr (ADALN) acc1[p][j] += dyv;
           o[j] = fmaf(xh, k2, fmaf(dyv * g[p][j], rstd, k1));
         }
-        if (rv[r] && act[p]) store_stream(a.dx, (size_t)(row * C + col[p]), pack8(o));
+        if (rv[r]) store_row<ROWS, SHORT>(a.dx, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
       }
     }
   }

@@ -2,5 +2,5 @@
 #include "kernel_table.hpp"
 
 namespace tt {
-KernelInfo resnorm_gated_kernel(bool backward, int idx, bool full) { return lookup_res<true>(backward, idx, full); }
+KernelInfo resnorm_gated_kernel(bool backward, int idx, int rows) { return lookup_res<true>(backward, idx, rows); }
 }  // namespace tt

@@ -106,8 +106,9 @@ __device__ __forceinline__ void wide_write_partials_n(float (&acc)[NACC][P][8], 
 }
 
 // ============================================================================ forward
-template <int W, int P, int R, int Q, bool FULL, bool GATED>
+template <int W, int P, int R, int Q, int ROWS, bool GATED>
 __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs a) {
+  constexpr bool FULL = ROWS == kFull, SHORT = !GATED && short_rows(W, P);
   __shared__ float red[2][Q][W * R];
 
   const int lane = threadIdx.x & 63;
@@ -150,8 +151,8 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs 
         rawr[r][p] = u32x4{0, 0, 0, 0};
         if (r0 + r < S && act[p]) {
           const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
-          rawx[r][p] = load_stream(a.x, off);
-          rawr[r][p] = load_stream(a.r, off);
+          rawx[r][p] = load_row<ROWS, SHORT>(a.x, off);
+          rawr[r][p] = load_row<ROWS, SHORT>(a.r, off);
         }
       }
   };
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs 
         for (int j = 0; j < 8; ++j) xf[r][p][j] = GATED ? fmaf(gt[p][j], rf[j], xf[r][p][j]) : xf[r][p][j] + rf[j];
         // the residual stream is stored as bf16, and it is that rounded value which is normalised
         const u32x4 sp = pack8(xf[r][p]);
-        if (rv[r] && act[p]) store_stream(a.s, (size_t)(row * C + col[p]), sp);
+        if (rv[r]) store_row<ROWS, SHORT>(a.s, row, a.packs, p * 64 * W + w * 64, lane, sp);
         unpack8(sp, xf[r][p]);
       }
     }
@@ -230,7 +231,7 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs 
             float o[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) o[j] = fmaf(xf[r][p][j] * rstd, g[p][j], sh[p][j]);
-            store_stream(a.y, (size_t)(row * C + col[p]), pack8(o));
+            store_row<ROWS, SHORT>(a.y, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
           }
         }
         if (w == 0 && lane == 0) {
@@ -243,8 +244,9 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs 
 }
 
 // ============================================================================ backward
-template <int W, int P, int R, int Q, bool FULL, bool GATED>
+template <int W, int P, int R, int Q, int ROWS, bool GATED>
 __global__ __launch_bounds__(64 * W * Q) void resnorm_bwd_wide(const ResBwdArgs a) {
+  constexpr bool FULL = ROWS == kFull, SHORT = !GATED && short_rows(W, P);
   constexpr int NACC = GATED ? 3 : 2;
   constexpr int NV = 3;
   __shared__ float red[2][Q][W * R * NV];
@@ -295,10 +297,10 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_bwd_wide(const ResBwdArgs 
         if constexpr (GATED) rawr[r][p] = u32x4{0, 0, 0, 0};
         if (r0 + r < S && act[p]) {
           const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
-          raws[r][p] = load_stream(a.s, off);
-          rawd[r][p] = load_stream(a.dy, off);
-          if (have_ds) rawg[r][p] = load_stream(a.ds_in, off);
-          if constexpr (GATED) rawr[r][p] = load_stream(a.r, off);
+          raws[r][p] = load_row<ROWS, SHORT>(a.s, off);
+          rawd[r][p] = load_row<ROWS, SHORT>(a.dy, off);
+          if (have_ds) rawg[r][p] = load_row<ROWS, SHORT>(a.ds_in, off);
+          if constexpr (GATED) rawr[r][p] = load_row<ROWS, SHORT>(a.r, off);
         }
       }
   };
@@ -390,9 +392,9 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_bwd_wide(const ResBwdArgs 
             o2[j] = gt[p][j] * ds;
           }
         }
-        if (rv[r] && act[p]) {
-          store_stream(a.dx, (size_t)(row * C + col[p]), pack8(o));
-          if constexpr (GATED) store_stream(a.dr, (size_t)(row * C + col[p]), pack8(o2));
+        if (rv[r]) {
+          store_row<ROWS, SHORT>(a.dx, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
+          if constexpr (GATED) store_row<ROWS, SHORT>(a.dr, row, a.packs, p * 64 * W + w * 64, lane, pack8(o2));
         }
       }
     }

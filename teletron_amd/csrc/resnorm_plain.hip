@@ -2,5 +2,5 @@
 #include "kernel_table.hpp"
 
 namespace tt {
-KernelInfo resnorm_plain_kernel(bool backward, int idx, bool full) { return lookup_res<false>(backward, idx, full); }
+KernelInfo resnorm_plain_kernel(bool backward, int idx, int rows) { return lookup_res<false>(backward, idx, rows); }
 }  // namespace tt

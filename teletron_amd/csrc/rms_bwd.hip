@@ -2,5 +2,5 @@
 #include "kernel_table.hpp"
 
 namespace tt {
-KernelInfo rms_bwd_kernel(bool narrow, int idx, bool full) { return lookup_bwd<kRMS>(narrow, idx, full); }
+KernelInfo rms_bwd_kernel(bool narrow, int idx, int rows) { return lookup_bwd<kRMS>(narrow, idx, rows); }
 }  // namespace tt

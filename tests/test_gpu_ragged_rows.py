@@ -1,0 +1,66 @@
+"""Wide rows that are not whole 128-byte lines (cols % 64 != 0): the lines that neighbouring waves and
+rows share are stored another way than the rest, so every segment edge of every variant is checked,
+and that nothing is written beside the rows.  Tolerances as in test_gpu_parity.py."""
+import pytest
+import torch
+
+from test_gpu_gate import test_gate_residual_shapes as check_gate
+from test_gpu_parity import DEV, check_adaln, check_rmsnorm, rand_bf16
+from test_gpu_resnorm import run_case as check_residual
+
+pytestmark = pytest.mark.gpu
+
+# the shortest and the longest ragged row of each variant (lane slots 64 ... 4096 packs of 8)
+SLOTS = [32, 64, 128, 192, 256, 384, 512, 640, 768, 1024, 1536, 2048, 4096]
+WIDTHS = [8 * w for lo, hi in zip(SLOTS, SLOTS[1:]) for w in (lo + 1, hi - 1)]
+
+
+@pytest.mark.parametrize("cols", WIDTHS)
+def test_ragged_widths(cols):
+    nb, rpb = 2, 19
+    x, dy = rand_bf16(nb, rpb, cols, seed=cols), rand_bf16(nb, rpb, cols, seed=cols + 1)
+    p = [rand_bf16(nb, 1, cols, seed=cols + 2 + i, scale=0.2) for i in range(2)]
+    check_adaln(x, p[0], p[1], dy, 1e-6, nb, f"cols {cols}")
+    check_rmsnorm(x, 1 + p[0][0, 0], dy, 1e-6, f"cols {cols}")
+    check_gate(cols, nb, rpb)
+    for gated in (False, True):
+        check_residual(cols, nb, rpb, gated, affine=False)
+
+
+@pytest.mark.parametrize("cols", [1000, 3688])
+@pytest.mark.parametrize("shift", range(0, 64, 8))
+def test_ragged_rows_at_any_16_byte_offset(lib, cols, shift):
+    """The same bits wherever in a line the tensors start, and the values around them untouched."""
+    rows, guard, eps = 23, 256, 1e-6
+    x, dy = (rand_bf16(rows, cols, seed=cols + i).to(DEV) for i in range(2))
+    w, b = (rand_bf16(cols, seed=cols + 2 + i, scale=0.2).to(DEV) for i in range(2))
+
+    def placed(t, s):
+        buf = torch.full((t.numel() + 2 * guard,), 7.0, dtype=t.dtype, device=DEV)
+        buf[guard + s:guard + s + t.numel()] = t.flatten()
+        return buf, buf.data_ptr() + 2 * (guard + s)
+
+    def run(s):
+        bufs = {}
+        for name, t in (("x", x), ("dy", dy), ("y", torch.zeros_like(x)), ("dx", torch.zeros_like(x)),
+                        ("s", torch.zeros_like(x)), ("g", torch.zeros_like(x))):
+            bufs[name] = placed(t, s)
+        ptr = {k: v[1] for k, v in bufs.items()}
+        grads = torch.zeros(2, cols, device=DEV)
+        ws = torch.empty(lib.tt_adaln_backward_workspace_bytes(rows, cols, rows), dtype=torch.uint8, device=DEV)
+        stream = torch.cuda.current_stream().cuda_stream
+        assert lib.tt_adaln_backward(ptr["dx"], grads[0].data_ptr(), grads[1].data_ptr(), ptr["dy"], ptr["x"], w.data_ptr(),
+                                     ws.data_ptr(), ws.numel(), rows, cols, rows, eps, stream) == 0
+        assert lib.tt_residual_norm_forward(ptr["s"], ptr["y"], ptr["x"], ptr["dy"], None, 1, w.data_ptr(), b.data_ptr(), 1, 0,
+                                            None, None, rows, cols, rows, eps, stream) == 0
+        assert lib.tt_gate_residual_forward(ptr["g"], ptr["x"], w.data_ptr(), ptr["dy"], rows, cols, rows, stream) == 0
+        torch.cuda.synchronize()
+        out = [grads]
+        for name in ("y", "dx", "s", "g"):
+            buf = bufs[name][0]
+            assert (buf[:guard + s] == 7).all() and (buf[guard + s + x.numel():] == 7).all(), name
+            out.append(buf[guard + s:guard + s + x.numel()])
+        return out
+
+    for got, want in zip(run(shift), run(0)):
+        assert torch.equal(got, want)
