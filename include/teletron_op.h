@@ -9,9 +9,9 @@
  *
  * Fast path: cols % 8 == 0 and every tensor 16-byte aligned (128-bit vector kernels).
  * tt_adaln_forward/backward, tt_rmsnorm_forward/backward and the tt_launch_*_forward entry
- * points also accept any other cols <= TT_MAX_COLS and 2-byte aligned tensors through
- * element-wise kernels (a correctness path, several times slower); the two-step backward
- * and the tt_launch_*_backward entry points return TT_ERR_UNSUPPORTED there.
+ * points also accept any other cols <= TT_MAX_COLS and 2-byte aligned tensors: more than 256
+ * columns run on vector kernels for any address, fewer on element-wise ones, several times slower; the two-step backward and the tt_launch_*_backward entry points
+ * return TT_ERR_UNSUPPORTED there.
  *
  * Two groups of entry points:
  *
@@ -85,8 +85,8 @@ TT_API int tt_adaln_forward(void* y, const void* x, const void* scale, const voi
  * `workspace` holds the per-workgroup partial column sums; it must be at least
  * tt_adaln_backward_workspace_bytes() (for the same shape, on the same device) and 16-byte
  * aligned; about 10 MB at rows 75600, cols 5120.  (With cols % 8 == 0 but a
- * misaligned tensor the element-wise path needs rows * 8 bytes instead, which can exceed
- * that figure for very short rows; TT_ERR_WORKSPACE is returned if it does not fit.)  The result is
+ * misaligned tensor at least rows * 8 bytes are needed as well, which can exceed
+ * that figure for very short rows; TT_ERR_WORKSPACE is returned if they do not fit.)  The result is
  * bitwise reproducible run to run (fixed summation order, no atomics).
  */
 TT_API int tt_adaln_backward(void* dx, float* dscale, float* dshift,
@@ -106,7 +106,7 @@ TT_API size_t tt_adaln_backward_workspace_bytes(int64_t rows, int64_t cols, int6
  * array (hipGetSymbolAddress) and the launch plan's device properties; a call with rows == 0 does
  * only that and touches no pointer, for callers that want this set-up done at a chosen moment.
  * A shape that needs more scratch than the array holds is refused with TT_ERR_STATIC_LIMIT: the
- * need is what tt_adaln_backward_workspace_bytes() returns (10.2 MB at rows 75600, cols 5120), or
+ * need is what tt_adaln_backward_workspace_bytes() returns (10.2 MB at rows 75600, cols 5120), and
  * rows * 8 bytes when cols is not a multiple of 8 or a tensor is not 16-byte aligned.  All calls
  * on one GPU share the array: two calls that overlap in time on the same GPU (different streams
  * or host threads, or two replays of graphs that captured it) race and give wrong dscale /

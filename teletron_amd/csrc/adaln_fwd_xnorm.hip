@@ -2,5 +2,5 @@
 #include "kernel_table.hpp"
 
 namespace tt {
-KernelInfo adaln_fwd_xnorm_kernel(bool narrow, int idx, bool full) { return lookup_fwd_xn(narrow, idx, full); }
+KernelInfo adaln_fwd_xnorm_kernel(bool narrow, int idx, int rows) { return lookup_fwd_xn(narrow, idx, rows); }
 }  // namespace tt

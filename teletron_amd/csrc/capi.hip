@@ -113,21 +113,23 @@ constexpr int kGateKind = 2;   // third op family next to kAdaLN / kRMS
 // Upper bound on workgroups per batch used by any plan: what the workspace is sized for.
 constexpr int kMaxWgsPerCu = 8;
 
+// `odd`: rows of any length and 2-byte aligned tensors (wide norm_fwd / norm_bwd kernels only).
 // `res`: 0, or the residual + LayerNorm fusion: 1 plain, 2 gated (wide rows, kFwd / kBwd only).
 int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_batch, Plan* plan, bool rope = false,
-              int res = 0, int64_t rope_heads = 0) {
+              int res = 0, int64_t rope_heads = 0, bool odd = false) {
   if (rows <= 0 || cols <= 0 || rows_per_batch <= 0 || rows % rows_per_batch != 0)
     return TT_ERR_INVALID_ARGUMENT;
   if (cols > TT_MAX_COLS) return TT_ERR_UNSUPPORTED;
-  if (cols % kPack != 0) return TT_ERR_UNSUPPORTED;
-  const int packs = static_cast<int>(cols / kPack);
+  if (cols % kPack != 0 && !odd) return TT_ERR_UNSUPPORTED;
+  const int packs = static_cast<int>((cols + kPack - 1) / kPack);
   const bool narrow = packs <= kNarrowMaxPacks;
+  if (odd && (narrow || res || rope || dir == kBwdSaved || kind == kGateKind)) return TT_ERR_UNSUPPORTED;
   const int idx = narrow ? select_narrow(packs) : select_wide(packs);
   if (idx < 0) return TT_ERR_UNSUPPORTED;
   const int slots = narrow ? kNarrowL[idx] : 64 * kWideW[idx] * kWideP[idx];
   const bool full = (slots == packs);
   // a row of whole 128-byte lines or not: see enum Rows
-  const int mode = full ? kFull : (cols * 2) % 128 == 0 ? kMasked : kRagged;
+  const int mode = odd ? kOdd : full ? kFull : (cols * 2) % 128 == 0 ? kMasked : kRagged;
   KernelInfo k;
   if (res) {
     if (narrow || kind != kAdaLN || dir == kBwdSaved || dir == kFwdXn) return TT_ERR_UNSUPPORTED;
@@ -137,7 +139,7 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
     k = rms_rope_kernel(narrow, dir == kBwd, idx, full, rope_heads);
   } else if (dir == kFwdXn) {
     if (kind != kAdaLN) return TT_ERR_UNSUPPORTED;
-    k = adaln_fwd_xnorm_kernel(narrow, idx, full);
+    k = adaln_fwd_xnorm_kernel(narrow, idx, odd ? kOdd : full ? kFull : kMasked);
   } else if (kind == kAdaLN)
     k = dir == kFwd ? adaln_fwd_kernel(narrow, idx, mode)
       : dir == kBwd ? adaln_bwd_kernel(narrow, idx, mode) : adaln_bwd_saved_kernel(narrow, idx, full);
@@ -192,6 +194,20 @@ size_t partial_bytes(const Plan& p, int n_acc, int64_t cols) {
   return (size_t)p.n_batches * p.grid_x * n_acc * cols * sizeof(float);
 }
 
+// Backward of rows that the 128-bit kernels do not take (cols % 8 != 0, or tensors that are only 2-byte
+// aligned).  Rows of more than 256 values take the kOdd kernels, which leave partial column sums like
+// all others, as long as those stay small: at most the size of the scratch array or of x and dy.  Beyond
+// that (a modulation vector for every few rows), and for shorter rows, the element-wise kernels run, which
+// keep two floats a row (their column sums have cols / 64 workgroups).  us forward / backward, element-wise ->
+// these: RMSNorm 5000 x 1001 12.6 / 117 -> 9.4 / 16, AdaLN 8000 x 1999 33 / 125 -> 17 / 29, 60000 x 1537
+// 283 / 2122 -> 79 / 133 (1544 columns, 16-byte aligned rows: 67 / 109).
+bool odd_plan(int kind, int64_t rows, int64_t cols, int64_t rows_per_batch, Plan* p) {
+  if (make_plan(kind, kBwd, rows, cols, rows_per_batch, p, false, 0, 0, true) != TT_OK) return false;
+  const size_t tensors = (size_t)rows * cols * 4;
+  const size_t most = tensors > TT_STATIC_WORKSPACE_BYTES ? tensors : (size_t)TT_STATIC_WORKSPACE_BYTES;
+  return partial_bytes(*p, kind == kAdaLN ? 2 : 1, cols) <= most;
+}
+
 // Workspace bound that does not depend on the launch-time occupancy query.
 size_t workspace_bound(int n_acc, int64_t rows, int64_t cols, int64_t rows_per_batch) {
   if (rows <= 0 || cols <= 0 || rows_per_batch <= 0 || rows % rows_per_batch != 0) return 0;
@@ -210,7 +226,13 @@ size_t workspace_bound(int n_acc, int64_t rows, int64_t cols, int64_t rows_per_b
 // plan-independent bound when a plan cannot be made here or a tuning override is active.
 size_t workspace_for(int kind, int n_acc, int64_t rows, int64_t cols, int64_t rows_per_batch) {
   const size_t bound = workspace_bound(n_acc, rows, cols, rows_per_batch);
-  if (bound == 0 || cols % kPack != 0) return bound;
+  if (bound == 0) return bound;
+  if (cols % kPack != 0) {
+    Plan po;
+    if (!odd_plan(kind, rows, cols, rows_per_batch, &po)) return bound;
+    const size_t need = partial_bytes(po, n_acc, cols);
+    return need > bound ? need : bound;
+  }
   if (g_wgs_per_cu_override.load() > 0 || g_grid_override.load() > 0) return bound;
   Plan p;
   if (make_plan(kind, kBwd, rows, cols, rows_per_batch, &p) != TT_OK) return bound;
@@ -260,11 +282,22 @@ int check_shape(int64_t rows, int64_t cols, int64_t rows_per_batch) {
   return TT_OK;
 }
 
+int reduce(void* out0, void* out1, const void* workspace, int n_batches, int n_partials, int n_acc,
+           int64_t cols, bool out_bf16, void* stream, void* out2 = nullptr);
+
 int forward_generic(int kind, void* y, const void* x, const void* p0, const void* p1, float* mean, float* rstd,
                     void* x_norm, int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream) {
   int rc = check_shape(rows, cols, rows_per_batch);
   if (rc != TT_OK) return rc;
   if (!aligned2(y) || !aligned2(x) || !aligned2(p0) || !aligned2(p1) || !aligned2(x_norm)) return TT_ERR_INVALID_ARGUMENT;
+  Plan p;
+  if (make_plan(kind, x_norm ? kFwdXn : kFwd, rows, cols, rows_per_batch, &p, false, 0, 0, true) == TT_OK) {
+    FwdArgs f = {};
+    f.y = y; f.x = x; f.p0 = p0; f.p1 = p1; f.mean = mean; f.rstd = rstd; f.x_norm = x_norm;
+    f.rows_per_batch = rows_per_batch; f.n_tiles = p.n_tiles;
+    f.cols = (int)cols; f.packs = p.packs; f.eps = eps; f.inv_cols = 1.0f / (float)cols;
+    return launch(p, f, stream);
+  }
   int grid = 0;
   rc = generic_grid(rows, &grid);
   if (rc != TT_OK) return rc;
@@ -290,6 +323,19 @@ int backward_generic(int kind, void* dx, void* out0, void* out1, const void* dy,
   if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 3u) != 0 ||
       workspace_bytes < (size_t)rows * 2 * sizeof(float))
     return TT_ERR_WORKSPACE;
+  Plan p;
+  if (odd_plan(kind, rows, cols, rows_per_batch, &p)) {
+    const int n_acc = kind == kAdaLN ? 2 : 1;
+    if (workspace_bytes >= partial_bytes(p, n_acc, cols)) {
+      BwdArgs b = {};
+      b.dx = dx; b.dy = dy; b.x = x; b.p0 = p0; b.partials = static_cast<float*>(workspace);
+      b.rows_per_batch = rows_per_batch; b.n_tiles = p.n_tiles;
+      b.cols = (int)cols; b.packs = p.packs; b.eps = eps; b.inv_cols = 1.0f / (float)cols;
+      rc = launch(p, b, stream);
+      if (rc != TT_OK) return rc;
+      return reduce(out0, out1, workspace, (int)p.n_batches, p.grid_x, n_acc, cols, false, stream);
+    }
+  }
   int grid = 0;
   rc = generic_grid(rows, &grid);
   if (rc != TT_OK) return rc;
@@ -407,7 +453,7 @@ int backward_saved_partials(int kind, void* dx, const void* dy, const void* xs, 
 }
 
 int reduce(void* out0, void* out1, const void* workspace, int n_batches, int n_partials, int n_acc,
-           int64_t cols, bool out_bf16, void* stream, void* out2 = nullptr) {
+           int64_t cols, bool out_bf16, void* stream, void* out2) {
   if (n_batches == 0) return TT_OK;
   if (!out0 || !workspace || n_batches < 0 || n_batches > 65535 || n_partials <= 0 || cols <= 0 ||
       cols > TT_MAX_COLS || n_acc < 1 || n_acc > 3 || (n_acc >= 2 && !out1) || (n_acc == 3 && !out2))

@@ -49,6 +49,7 @@ enum Rows : int {
   kMasked = 0,   // fewer packs than lane slots; a row is a whole number of 128-byte lines
   kFull = 1,     // every lane slot holds a pack
   kRagged = 2,   // as kMasked, but rows start anywhere inside a line (cols % 64 != 0)
+  kOdd = 3,      // any row length and 2-byte aligned tensors; the last pack may be short
 };
 // Where rows are not whole lines, the segments of neighbouring waves and rows share the lines at
 // their ends.  A written-through store sends its part of such a line to memory on its own, and
@@ -95,6 +96,31 @@ __device__ __forceinline__ void store_row(void* base, int64_t row, int packs, in
     }
   }
   store_stream(p, 0, v);
+}
+
+// ---- kOdd rows: packs at any 2-byte address (this target's vector memory instructions take them)
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+__device__ __forceinline__ u32x4 load_any(const void* base, size_t elem_off) {
+  return *reinterpret_cast<const u32x4_any*>(static_cast<const uint16_t*>(base) + elem_off);
+}
+// Stores the first n values of a pack (n <= 0: none).
+__device__ __forceinline__ void store_any(void* base, size_t elem_off, u32x4 v, int n) {
+  uint16_t* p = static_cast<uint16_t*>(base) + elem_off;
+  if (n >= kPack) {
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any*>(p));
+  } else {
+#pragma unroll
+    for (int j = 0; j < kPack - 1; ++j)
+      if (j < n) p[j] = static_cast<uint16_t>(v[j / 2] >> (16 * (j & 1)));
+  }
+}
+// A short last pack is loaded as the last eight values of its row, which is always inside the
+// tensor; this moves its own values to the front and zeros in behind them.
+__device__ __forceinline__ u32x4 drop_values(u32x4 v, int drop) {
+  if (drop & 1) v = u32x4{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+  if (drop & 2) v = u32x4{v[1], v[2], v[3], 0};
+  if (drop & 4) v = u32x4{v[2], v[3], 0, 0};
+  return v;
 }
 
 // ---------------------------------------------------------------- bf16 <-> fp32

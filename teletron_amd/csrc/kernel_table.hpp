@@ -65,7 +65,7 @@ constexpr int bwd_wide_R(int W, int P) { return 1; }
 // per row) is 2-3 % slower with R = 2 everywhere.  Ragged rows lose with two as well (60000 x 2200:
 // 162 -> 184 us, 1000: 71 -> 77 us).
 constexpr int adaln_bwd_wide_R(int W, int P, int rows) {
-  if (rows == kRagged) return bwd_wide_R(W, P);
+  if (rows == kRagged || rows == kOdd) return bwd_wide_R(W, P);
   return ((P == 1 && W >= 2 && W <= 4) || (P == 2 && (W == 3 || W == 6))) ? 2 : bwd_wide_R(W, P);
 }
 constexpr int fwd_wide_Q(int W, int P) {
@@ -136,26 +136,30 @@ KernelInfo info_bwd_narrow() {
 // the input (period 128 MiB); independent workgroups stay at 384-393 us at every placement.
 // Measured with this rule: 75600 x 5120 416 us, 131040 x 1536 213 us, 150000 x 2048 323 us.
 constexpr int fwd_xn_wide_Q(int W, int P) { return 1; }
-template <int W, int P, bool FULL>
+template <int W, int P, int ROWS>
 KernelInfo info_fwd_xn_wide() {
   constexpr int R = fwd_wide_R(W, P), Q = fwd_xn_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_fwd_wide<kAdaLN, W, P, R, Q, FULL ? kFull : kMasked, false, true>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_fwd_wide<kAdaLN, W, P, R, Q, ROWS, false, true>), 64 * W * Q, Q * R, P * R};
 }
 template <int L, bool FULL>
 KernelInfo info_fwd_xn_narrow() {
   constexpr int R = kNarrowR, NW = kNarrowNW;
   return {reinterpret_cast<const void*>(&norm_fwd_narrow<kAdaLN, L, R, NW, FULL, 0, true>), 64 * NW, NW * R * (64 / L), R};
 }
-inline KernelInfo lookup_fwd_xn(bool narrow, int idx, bool full) {
+inline KernelInfo lookup_fwd_xn(bool narrow, int idx, int rows) {
   if (narrow) {
     switch (idx) {
-#define X(i, L) case i: return full ? info_fwd_xn_narrow<L, true>() : info_fwd_xn_narrow<L, false>();
+#define X(i, L) case i: return rows == kFull ? info_fwd_xn_narrow<L, true>() : info_fwd_xn_narrow<L, false>();
       TT_NARROW_LIST(X)
 #undef X
     }
   } else {
     switch (idx) {
-#define X(i, W, P) case i: return full ? info_fwd_xn_wide<W, P, true>() : info_fwd_xn_wide<W, P, false>();
+#define X(i, W, P)                                           \
+  case i:                                                    \
+    return rows == kFull  ? info_fwd_xn_wide<W, P, kFull>()  \
+           : rows == kOdd ? info_fwd_xn_wide<W, P, kOdd>()   \
+                          : info_fwd_xn_wide<W, P, kMasked>();
       TT_WIDE_LIST(X)
 #undef X
     }
@@ -168,6 +172,9 @@ inline KernelInfo lookup_fwd_xn(bool narrow, int idx, bool full) {
   return rows == kFull     ? INFO<__VA_ARGS__, kFull>()        \
          : rows == kRagged ? INFO<__VA_ARGS__, kRagged>()      \
                            : INFO<__VA_ARGS__, kMasked>();
+#define TT_ROWS_ODD(INFO, ...)                           \
+  if (rows == kOdd) return INFO<__VA_ARGS__, kOdd>();    \
+  TT_ROWS(INFO, __VA_ARGS__)
 template <int KIND>
 KernelInfo lookup_fwd(bool narrow, int idx, int rows) {
   if (narrow) {
@@ -178,7 +185,7 @@ KernelInfo lookup_fwd(bool narrow, int idx, int rows) {
     }
   } else {
     switch (idx) {
-#define X(i, W, P) case i: TT_ROWS(info_fwd_wide, KIND, W, P)
+#define X(i, W, P) case i: TT_ROWS_ODD(info_fwd_wide, KIND, W, P)
       TT_WIDE_LIST(X)
 #undef X
     }
@@ -195,7 +202,7 @@ KernelInfo lookup_bwd(bool narrow, int idx, int rows) {
     }
   } else {
     switch (idx) {
-#define X(i, W, P) case i: TT_ROWS(info_bwd_wide, KIND, W, P)
+#define X(i, W, P) case i: TT_ROWS_ODD(info_bwd_wide, KIND, W, P)
       TT_WIDE_LIST(X)
 #undef X
     }
@@ -359,7 +366,7 @@ KernelInfo lookup_bwd_saved(bool narrow, int idx, bool full) {
 // Defined one per translation unit (adaln_fwd.hip, adaln_fwd_xnorm.hip, adaln_bwd.hip, adaln_bwd_saved.hip, rms_fwd.hip, rms_bwd.hip, rms_bwd_saved.hip, rms_rope.hip, gate.hip,
 // resnorm_plain.hip, resnorm_gated.hip).
 KernelInfo adaln_fwd_kernel(bool narrow, int idx, int rows);
-KernelInfo adaln_fwd_xnorm_kernel(bool narrow, int idx, bool full);
+KernelInfo adaln_fwd_xnorm_kernel(bool narrow, int idx, int rows);
 KernelInfo adaln_bwd_kernel(bool narrow, int idx, int rows);
 KernelInfo rms_fwd_kernel(bool narrow, int idx, int rows);
 KernelInfo rms_bwd_kernel(bool narrow, int idx, int rows);

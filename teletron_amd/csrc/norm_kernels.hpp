@@ -1,6 +1,7 @@
 // Streaming kernels for fused AdaLN / RMSNorm, forward and backward, on gfx950.
 //
-// Two shapes of kernel cover every row width that is a multiple of 8:
+// Two shapes of kernel cover every row width that is a multiple of 8 (the wide one any other width too,
+// see enum Rows):
 //
 //  * "wide"   (more than 32 packs per row): a row is owned by a *row group* of
 //    W waves; lane l of wave w owns the packs  p*64*W + w*64 + l  (p < P), so
@@ -118,11 +119,25 @@ __device__ __forceinline__ void rowgroup_allsum(float (&v)[NV], float* buf, int 
 }
 
 // ============================================================================ wide forward
+// Parameters of a lane, and its own values of a loaded pack, for any row mode; `n` as in the kernels.
+template <int ROWS>
+__device__ __forceinline__ u32x4 own_values(u32x4 v, int n) {
+  if constexpr (ROWS == kOdd) {
+    if (n > 0 && n < kPack) v = drop_values(v, kPack - n);
+  }
+  return v;
+}
+template <int ROWS>
+__device__ __forceinline__ u32x4 load_pack(const void* base, size_t elem_off, int n) {
+  if constexpr (ROWS == kOdd) return own_values<ROWS>(load_any(base, elem_off - (kPack - n)), n);
+  else return load_cached(base, elem_off);
+}
+
 // XN: also store the normalised input before modulation (a.x_norm), paired with the y store.
 template <int KIND, int W, int P, int R, int Q, int ROWS, bool ROPE = false, bool XN = false>
 __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
   constexpr bool ADALN = (KIND == kAdaLN);
-  constexpr bool FULL = ROWS == kFull, SHORT = short_rows(W, P);
+  constexpr bool FULL = ROWS == kFull, SHORT = short_rows(W, P), ODD = ROWS == kOdd;
   static_assert(!ROPE || KIND == kRMS, "rotary embedding is fused behind RMSNorm only");
   static_assert(!XN || ADALN, "x_norm is an output of the AdaLN forward only");
   __shared__ float red[2][Q][W * R];
@@ -135,18 +150,20 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
   const int64_t S = a.rows_per_batch;
   const int C = a.cols;
 
-  int col[P];
+  int col[P], n[P];            // n: values of the pack that exist
   bool act[P];
   float g[P][8], sh[P][8];
+  const int drop = ODD ? a.packs * kPack - C : 0;   // values that the last pack is short of
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     const int pk = p * 64 * W + w * 64 + lane;
     act[p] = FULL || pk < a.packs;
     col[p] = pk * kPack;
+    n[p] = !act[p] ? 0 : pk == a.packs - 1 ? kPack - drop : kPack;
     u32x4 r0 = {0, 0, 0, 0}, r1 = {0, 0, 0, 0};
     if (act[p]) {
-      r0 = load_cached(a.p0, (ADALN ? b * C : 0) + col[p]);
-      if constexpr (ADALN) r1 = load_cached(a.p1, b * C + col[p]);
+      r0 = load_pack<ROWS>(a.p0, (ADALN ? b * C : 0) + col[p], n[p]);
+      if constexpr (ADALN) r1 = load_pack<ROWS>(a.p1, b * C + col[p], n[p]);
     }
     unpack8(r0, g[p]);
     unpack8(r1, sh[p]);
@@ -196,7 +213,11 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
 #pragma unroll
       for (int p = 0; p < P; ++p) {
         raw[r][p] = u32x4{0, 0, 0, 0};
-        if (r0 + r < S && act[p]) raw[r][p] = load_row<ROWS, SHORT>(a.x, (size_t)((b * S + r0 + r) * C + col[p]));
+        if (r0 + r < S && act[p]) {
+          const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
+          if constexpr (ODD) raw[r][p] = load_any(a.x, off - (kPack - n[p]));
+          else               raw[r][p] = load_row<ROWS, SHORT>(a.x, off);
+        }
       }
   };
 
@@ -213,7 +234,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
     for (int r = 0; r < R; ++r) {
       rv[r] = row0 + r < S;
 #pragma unroll
-      for (int p = 0; p < P; ++p) unpack8(raw[r][p], xf[r][p]);
+      for (int p = 0; p < P; ++p) unpack8(own_values<ROWS>(raw[r][p], n[p]), xf[r][p]);
     }
     if constexpr (ROPE) {
       if (floader) {
@@ -254,7 +275,8 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
           float d = xf[r][p][j];
           if constexpr (ADALN) {
             d -= mean[r];
-            if constexpr (!FULL) d = act[p] ? d : 0.f;
+            if constexpr (ODD) d = j < n[p] ? d : 0.f;
+            else if constexpr (!FULL) d = act[p] ? d : 0.f;
             xf[r][p][j] = d;
           }
           t = fmaf(d, d, t);
@@ -272,11 +294,11 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
 #pragma unroll
         for (int p = 0; p < P; ++p) {
           if (act[p]) {
-            float o[8], n[8];
+            float o[8], xn[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
               const float xh = xf[r][p][j] * rstd;
-              n[j] = xh;
+              xn[j] = xh;
               o[j] = ADALN ? fmaf(xh, g[p][j], sh[p][j]) : xh * g[p][j];
             }
             if constexpr (ROPE) {
@@ -287,7 +309,10 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
               fc[4] = f1[0]; fc[5] = f1[1]; fc[6] = f1[2]; fc[7] = f1[3];
               rope_rotate(o, fc);
             }
-            if constexpr (XN) store_stream2(a.y, a.x_norm, (size_t)(row * C + col[p]), pack8(o), pack8(n));
+            if constexpr (ODD) {
+              store_any(a.y, (size_t)(row * C + col[p]), pack8(o), n[p]);
+              if constexpr (XN) store_any(a.x_norm, (size_t)(row * C + col[p]), pack8(xn), n[p]);
+            } else if constexpr (XN) store_stream2(a.y, a.x_norm, (size_t)(row * C + col[p]), pack8(o), pack8(xn));
             else              store_row<ROWS, SHORT>(a.y, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
           }
         }
@@ -302,7 +327,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
 
 // Epilogue of the wide backward kernels: fold the Q row groups of the workgroup into
 // group 0 (in group order, through LDS) and write the workgroup's partial column sums.
-template <bool ADALN, int W, int P, int Q>
+template <bool ADALN, int W, int P, int Q, bool ODD = false>
 __device__ __forceinline__ void wide_write_partials(float (&acc0)[P][8], float (&acc1)[P][8], const bool (&act)[P],
                                                     const int (&col)[P], float* partials, int64_t b, int C,
                                                     int q, int w, int lane) {
@@ -337,7 +362,14 @@ __device__ __forceinline__ void wide_write_partials(float (&acc0)[P][8], float (
     float* base = partials + ((size_t)(b * gridDim.x + blockIdx.x) * NACC) * C;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      if (act[p]) {
+      if constexpr (ODD) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (col[p] + j < C) {
+            base[col[p] + j] = acc0[p][j];
+            if constexpr (ADALN) base[C + col[p] + j] = acc1[p][j];
+          }
+      } else if (act[p]) {
         f32x4* d0 = reinterpret_cast<f32x4*>(base + col[p]);
         d0[0] = f32x4{acc0[p][0], acc0[p][1], acc0[p][2], acc0[p][3]};
         d0[1] = f32x4{acc0[p][4], acc0[p][5], acc0[p][6], acc0[p][7]};
@@ -355,7 +387,7 @@ __device__ __forceinline__ void wide_write_partials(float (&acc0)[P][8], float (
 template <int KIND, int W, int P, int R, int Q, int ROWS, bool ROPE = false>
 __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
   constexpr bool ADALN = (KIND == kAdaLN);
-  constexpr bool FULL = ROWS == kFull, SHORT = short_rows(W, P);
+  constexpr bool FULL = ROWS == kFull, SHORT = short_rows(W, P), ODD = ROWS == kOdd;
   static_assert(!ROPE || KIND == kRMS, "rotary embedding is fused behind RMSNorm only");
   constexpr int NACC = ADALN ? 2 : 1;
   constexpr int NV = ADALN ? 3 : 2;  // reduced values per row in the main phase
@@ -369,8 +401,9 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
   const int64_t S = a.rows_per_batch;
   const int C = a.cols;
 
-  int col[P];
+  int col[P], n[P];
   bool act[P];
+  const int drop = ODD ? a.packs * kPack - C : 0;   // as in the forward kernel
   float g[P][8];
   float acc0[P][8];  // dscale / dgamma
   float acc1[P][8];  // dshift (AdaLN only)
@@ -379,8 +412,9 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
     const int pk = p * 64 * W + w * 64 + lane;
     act[p] = FULL || pk < a.packs;
     col[p] = pk * kPack;
+    n[p] = !act[p] ? 0 : pk == a.packs - 1 ? kPack - drop : kPack;
     u32x4 r0 = {0, 0, 0, 0};
-    if (act[p]) r0 = load_cached(a.p0, (ADALN ? b * C : 0) + col[p]);
+    if (act[p]) r0 = load_pack<ROWS>(a.p0, (ADALN ? b * C : 0) + col[p], n[p]);
     unpack8(r0, g[p]);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -424,8 +458,13 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
         }
         if (r0 + r < S && act[p]) {
           const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
-          rawx[r][p] = load_row<ROWS, SHORT>(a.x, off);
-          rawd[r][p] = load_row<ROWS, SHORT>(a.dy, off);
+          if constexpr (ODD) {
+            rawx[r][p] = load_any(a.x, off - (kPack - n[p]));
+            rawd[r][p] = load_any(a.dy, off - (kPack - n[p]));
+          } else {
+            rawx[r][p] = load_row<ROWS, SHORT>(a.x, off);
+            rawd[r][p] = load_row<ROWS, SHORT>(a.dy, off);
+          }
           if constexpr (ROPE)
             load_freq8(a.freqs, (size_t)(pos[r] * a.head_dim + fcol[p]), fr[r][p]);
         }
@@ -445,8 +484,8 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
       rv[r] = row0 + r < S;
 #pragma unroll
       for (int p = 0; p < P; ++p) {
-        unpack8(rawx[r][p], xf[r][p]);
-        unpack8(rawd[r][p], df[r][p]);
+        unpack8(own_values<ROWS>(rawx[r][p], n[p]), xf[r][p]);
+        unpack8(own_values<ROWS>(rawd[r][p], n[p]), df[r][p]);
         // the incoming gradient is that of the rotated output: undo the rotation first
         if constexpr (ROPE) rope_unrotate(df[r][p], fr[r][p]);
       }
@@ -485,7 +524,8 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
           float d = xf[r][p][j];
           if constexpr (ADALN) {
             d -= mean[r];
-            if constexpr (!FULL) d = act[p] ? d : 0.f;
+            if constexpr (ODD) d = j < n[p] ? d : 0.f;
+            else if constexpr (!FULL) d = act[p] ? d : 0.f;
             xf[r][p][j] = d;
           }
           const float gg = df[r][p][j] * g[p][j];
@@ -520,12 +560,14 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
           if constexpr (ADALN) acc1[p][j] += dyv;
           o[j] = fmaf(xh, k2, fmaf(dyv * g[p][j], rstd, k1));
         }
-        if (rv[r]) store_row<ROWS, SHORT>(a.dx, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
+        if constexpr (ODD) {
+          if (rv[r]) store_any(a.dx, (size_t)(row * C + col[p]), pack8(o), n[p]);
+        } else if (rv[r]) store_row<ROWS, SHORT>(a.dx, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
       }
     }
   }
 
-  wide_write_partials<ADALN, W, P, Q>(acc0, acc1, act, col, a.partials, b, C, q, w, lane);
+  wide_write_partials<ADALN, W, P, Q, ODD>(acc0, acc1, act, col, a.partials, b, C, q, w, lane);
 }
 
 // Position of a row for the narrow ROPE kernels: one row is one head, `rows_per_pos` consecutive

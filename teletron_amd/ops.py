@@ -115,8 +115,7 @@ def clear_workspaces() -> None:
 def _workspace(lib_bytes: int, rows: int, *tensors: torch.Tensor) -> torch.Tensor:
     """Backward workspace (partial column sums), kept per device and stream and reused from call to
     call: launches on one stream run in order, so consecutive backward calls never overlap in it.
-    Tensors that are not 16-byte aligned take the element-wise kernels, which keep two floats of
-    statistics per row there."""
+    Tensors that are not 16-byte aligned need at least two floats per row there."""
     need = lib_bytes
     if any(t.data_ptr() % 16 for t in tensors):
         need = max(need, rows * 8)

@@ -64,3 +64,51 @@ def test_ragged_rows_at_any_16_byte_offset(lib, cols, shift):
 
     for got, want in zip(run(shift), run(0)):
         assert torch.equal(got, want)
+
+
+# one value more than a variant of the kernels holds, one less, and a short last pack of every length
+ODD = [257, 511, 513, 1001, 1023, 1535, 1537, 2049, 3073, 4095, 5121, 6143, 8193, 16383, 32767] + list(range(521, 528))
+
+
+@pytest.mark.parametrize("cols", ODD)
+def test_odd_widths(cols):
+    for nb, rpb in ((1, 1), (2, 37), (41, 1)):
+        x, dy = rand_bf16(nb, rpb, cols, seed=cols), rand_bf16(nb, rpb, cols, seed=cols + 1)
+        p = [rand_bf16(nb, 1, cols, seed=cols + 2 + i, scale=0.2) for i in range(2)]
+        check_adaln(3 + x, p[0], p[1], dy, 1e-6, nb, f"cols {cols}")
+        check_rmsnorm(x, 1 + p[0][0, 0], dy, 1e-6, f"cols {cols}")
+
+
+@pytest.mark.parametrize("cols", [1001, 1000, 1536])
+@pytest.mark.parametrize("shift", [1, 3, 8, 13])
+def test_backward_at_any_address_and_workspace(lib, cols, shift):
+    """Nothing beside the rows and gradients is written; the smallest workspace (two floats a row, with
+    which the element-wise kernels run) gives the same gradients."""
+    rows, guard = 2500, 64
+    x, dy, w = rand_bf16(rows, cols, seed=1), rand_bf16(rows, cols, seed=2), rand_bf16(cols, seed=3, scale=0.2)
+    from oracle import norm_oracle as O
+    from test_gpu_parity import assert_bf16_close, assert_grad_close
+    dxo, dso, dho = O.adaln_backward(dy, x, w, 1e-6, 1)
+
+    def placed(t):
+        buf = torch.full((t.numel() + 2 * guard,), 7.0, dtype=t.dtype, device=DEV)
+        buf[guard + shift:guard + shift + t.numel()] = t.flatten().to(DEV)
+        return buf, buf.data_ptr() + 2 * (guard + shift)
+
+    (xb, xp), (db, dp), (wb, wp), (ob, op) = (placed(t) for t in (x, dy, w, torch.zeros_like(x)))
+    stream = torch.cuda.current_stream().cuda_stream
+    need = max(lib.tt_adaln_backward_workspace_bytes(rows, cols, rows), rows * 8)
+    for size, status in ((need, 0), (rows * 8, 0), (rows * 8 - 4, 3)):
+        if shift == 8 and cols % 8 == 0 and size != need:
+            continue                                   # 16-byte aligned: the ordinary kernels, which need it all
+        ws = torch.full((size // 4 + guard,), 5.0, device=DEV)
+        grads = torch.full((2, cols + guard), 5.0, device=DEV)
+        assert lib.tt_adaln_backward(op, grads[0].data_ptr(), grads[1].data_ptr(), dp, xp, wp, ws.data_ptr(), size,
+                                     rows, cols, rows, 1e-6, stream) == status
+        torch.cuda.synchronize()
+        assert (ws[size // 4:] == 5).all() and (grads[:, cols:] == 5).all()
+        assert (ob[:guard + shift] == 7).all() and (ob[guard + shift + x.numel():] == 7).all()
+        if status == 0:
+            assert_bf16_close(ob[guard + shift:guard + shift + x.numel()], dxo, "dx")
+            assert_grad_close(grads[0, :cols], dso, rows, "dscale")
+            assert_grad_close(grads[1, :cols], dho, rows, "dshift")
