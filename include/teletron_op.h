@@ -255,6 +255,53 @@ TT_API int tt_residual_norm_backward(void* dx, void* dr, float* dscale, float* d
                                      int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream);
 TT_API size_t tt_residual_norm_backward_workspace_bytes(int64_t rows, int64_t cols, int64_t rows_per_batch, int gated);
 
+/* ------------------------------------------------------------------ parameters and gradients as a model holds them
+ * The entry points above with the memory layout and types of the parameters spelled out, so that
+ * no copy or cast has to be launched around them.  No counterparts in the reference.
+ *   *_strided: consecutive batches' scale / shift / gate vectors lie *_stride elements apart (a chunk
+ *     of a [B, 6, C] modulation tensor).  scale_copy / gate_copy (optional) receive the vectors
+ *     without gaps, which is what backward reads.
+ *   tt_rmsnorm_forward_f32_weight: the weight is fp32 and is rounded to bf16 as it is read;
+ *     weight_copy (optional) receives the rounded weight.
+ *   *_typed: parameter gradients are rounded once to bf16 where grads_bf16 is set, else fp32.
+ *     tt_rmsnorm_backward_typed: freqs NULL: no rotary embedding; heads 0: all heads in one row, as
+ *     tt_rmsnorm_rope_backward, else as tt_rmsnorm_rope_heads_backward.
+ * TT_ERR_UNSUPPORTED where only the element-wise kernels could run (at most 256 columns, and
+ * cols % 8 != 0 or an address or stride that is not a multiple of 16 bytes) and wherever the entry
+ * points above return it. */
+TT_API int tt_adaln_forward_strided(void* y, const void* x, const void* scale, int64_t scale_stride,
+                                    const void* shift, int64_t shift_stride, void* scale_copy,
+                                    int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream);
+TT_API int tt_adaln_backward_typed(void* dx, void* dscale, void* dshift, int grads_bf16,
+                                   const void* dy, const void* x, const void* scale,
+                                   void* workspace, size_t workspace_bytes,
+                                   int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream);
+TT_API int tt_rmsnorm_forward_f32_weight(void* y, const void* x, const float* weight, void* weight_copy,
+                                         int64_t rows, int64_t cols, float eps, void* stream);
+TT_API int tt_rmsnorm_backward_typed(void* dx, void* dweight, int grads_bf16,
+                                     const void* dy, const void* x, const void* weight,
+                                     const float* freqs, int64_t head_dim, int64_t heads, int64_t seq_len,
+                                     void* workspace, size_t workspace_bytes,
+                                     int64_t rows, int64_t cols, float eps, void* stream);
+TT_API int tt_gate_residual_forward_strided(void* out, const void* x, const void* gate, int64_t gate_stride,
+                                            void* gate_copy, const void* residual,
+                                            int64_t rows, int64_t cols, int64_t rows_per_batch, void* stream);
+TT_API int tt_gate_residual_backward_typed(void* dresidual, void* dgate, int grads_bf16,
+                                           const void* dout, const void* gate, const void* residual,
+                                           void* workspace, size_t workspace_bytes,
+                                           int64_t rows, int64_t cols, int64_t rows_per_batch, void* stream);
+TT_API int tt_residual_norm_forward_strided(void* s, void* y, const void* x, const void* r,
+                                            const void* gate, int64_t n_gate, int64_t gate_stride, void* gate_copy,
+                                            const void* scale, int64_t scale_stride, void* scale_copy,
+                                            const void* shift, int64_t shift_stride, int64_t n_param, int affine,
+                                            float* mean, float* rstd,
+                                            int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream);
+TT_API int tt_residual_norm_backward_typed(void* dx, void* dr, void* dscale, void* dshift, void* dgate, int grads_bf16,
+                                           const void* dy, const void* ds_in, const void* s, const void* r,
+                                           const void* gate, int64_t n_gate, const void* scale, int64_t n_param, int affine,
+                                           void* workspace, size_t workspace_bytes,
+                                           int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream);
+
 /* ------------------------------------------------------------------ bare streaming probe
  * Measurement aid without a counterpart in the reference.  Over `bytes` bytes, with the
  * load/store policy of the kernels above, one workgroup per compute unit and no arithmetic:

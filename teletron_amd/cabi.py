@@ -76,6 +76,27 @@ PROTOTYPES = {
                                           c_void_p, c_int64, c_void_p, c_int64, c_int,
                                           c_void_p, c_size_t, c_int64, c_int64, c_int64, c_float, c_void_p]),
     "tt_residual_norm_backward_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int]),
+    "tt_adaln_forward_strided": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p,
+                                         c_int64, c_int64, c_int64, c_float, c_void_p]),
+    "tt_adaln_backward_typed": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
+                                        c_void_p, c_size_t, c_int64, c_int64, c_int64, c_float, c_void_p]),
+    "tt_rmsnorm_forward_f32_weight": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p,
+                                              c_int64, c_int64, c_float, c_void_p]),
+    "tt_rmsnorm_backward_typed": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
+                                          c_void_p, c_int64, c_int64, c_int64, c_void_p, c_size_t,
+                                          c_int64, c_int64, c_float, c_void_p]),
+    "tt_gate_residual_forward_strided": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p,
+                                                 c_int64, c_int64, c_int64, c_void_p]),
+    "tt_gate_residual_backward_typed": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
+                                                c_void_p, c_size_t, c_int64, c_int64, c_int64, c_void_p]),
+    "tt_residual_norm_forward_strided": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p,
+                                                 c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_void_p,
+                                                 c_void_p, c_int64, c_int64, c_int, c_void_p, c_void_p,
+                                                 c_int64, c_int64, c_int64, c_float, c_void_p]),
+    "tt_residual_norm_backward_typed": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
+                                                c_void_p, c_void_p, c_void_p, c_void_p,
+                                                c_void_p, c_int64, c_void_p, c_int64, c_int,
+                                                c_void_p, c_size_t, c_int64, c_int64, c_int64, c_float, c_void_p]),
     "tt_stream_probe": (c_int, [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "tt_stream_probe_two_outputs": (c_int, [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "tt_launch_adaln_forward": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,

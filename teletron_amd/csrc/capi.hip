@@ -99,6 +99,13 @@ struct Rope {
   int64_t heads = 0;   // 0: a row holds every head of a token; > 0: one head per row, `heads` rows per token
 };
 
+// How the parameters of a norm forward lie in memory, where not as dense bf16 (see FwdArgs).
+struct Params {
+  int64_t stride0, stride1;
+  int f32;
+  void* copy;
+};
+
 struct Plan {
   KernelInfo k;
   int64_t n_batches = 0;
@@ -265,6 +272,7 @@ int launch(const Plan& p, Args& args, void* stream) {
 }
 
 // ---------------------------------------------------------------- element-wise fallback
+bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
 bool aligned2(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 1u) == 0; }
 
 int generic_grid(int64_t rows, int* grid) {
@@ -286,18 +294,23 @@ int reduce(void* out0, void* out1, const void* workspace, int n_batches, int n_p
            int64_t cols, bool out_bf16, void* stream, void* out2 = nullptr);
 
 int forward_generic(int kind, void* y, const void* x, const void* p0, const void* p1, float* mean, float* rstd,
-                    void* x_norm, int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream) {
+                    void* x_norm, int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream,
+                    const Params* params) {
   int rc = check_shape(rows, cols, rows_per_batch);
   if (rc != TT_OK) return rc;
   if (!aligned2(y) || !aligned2(x) || !aligned2(p0) || !aligned2(p1) || !aligned2(x_norm)) return TT_ERR_INVALID_ARGUMENT;
+  if (params && (!aligned2(params->copy) || (params->f32 && !aligned4(p0)))) return TT_ERR_INVALID_ARGUMENT;
   Plan p;
   if (make_plan(kind, x_norm ? kFwdXn : kFwd, rows, cols, rows_per_batch, &p, false, 0, 0, true) == TT_OK) {
     FwdArgs f = {};
+    f.p0_stride = params ? params->stride0 : cols; f.p1_stride = params ? params->stride1 : cols;
+    f.p0_f32 = params ? params->f32 : 0; f.p0_copy = params ? params->copy : nullptr;
     f.y = y; f.x = x; f.p0 = p0; f.p1 = p1; f.mean = mean; f.rstd = rstd; f.x_norm = x_norm;
     f.rows_per_batch = rows_per_batch; f.n_tiles = p.n_tiles;
     f.cols = (int)cols; f.packs = p.packs; f.eps = eps; f.inv_cols = 1.0f / (float)cols;
     return launch(p, f, stream);
   }
+  if (params) return TT_ERR_UNSUPPORTED;   // the element-wise kernels read dense bf16 parameters only
   int grid = 0;
   rc = generic_grid(rows, &grid);
   if (rc != TT_OK) return rc;
@@ -315,7 +328,7 @@ int forward_generic(int kind, void* y, const void* x, const void* p0, const void
 
 int backward_generic(int kind, void* dx, void* out0, void* out1, const void* dy, const void* x, const void* p0,
                      void* workspace, size_t workspace_bytes, int64_t rows, int64_t cols, int64_t rows_per_batch,
-                     float eps, void* stream) {
+                     float eps, void* stream, bool out_bf16) {
   int rc = check_shape(rows, cols, rows_per_batch);
   if (rc != TT_OK) return rc;
   if (!dx || !dy || !x || !p0 || !out0 || (kind == kAdaLN && !out1)) return TT_ERR_INVALID_ARGUMENT;
@@ -333,7 +346,7 @@ int backward_generic(int kind, void* dx, void* out0, void* out1, const void* dy,
       b.cols = (int)cols; b.packs = p.packs; b.eps = eps; b.inv_cols = 1.0f / (float)cols;
       rc = launch(p, b, stream);
       if (rc != TT_OK) return rc;
-      return reduce(out0, out1, workspace, (int)p.n_batches, p.grid_x, n_acc, cols, false, stream);
+      return reduce(out0, out1, workspace, (int)p.n_batches, p.grid_x, n_acc, cols, out_bf16, stream);
     }
   }
   int grid = 0;
@@ -343,7 +356,7 @@ int backward_generic(int kind, void* dx, void* out0, void* out1, const void* dy,
   a.dx = static_cast<uint16_t*>(dx); a.dy = static_cast<const uint16_t*>(dy); a.x = static_cast<const uint16_t*>(x);
   a.p0 = static_cast<const uint16_t*>(p0); a.stats = static_cast<float*>(workspace); a.out0 = out0; a.out1 = out1;
   a.rows = rows; a.rows_per_batch = rows_per_batch; a.cols = (int)cols; a.eps = eps; a.inv_cols = 1.0f / (float)cols;
-  a.out_bf16 = 0;
+  a.out_bf16 = out_bf16 ? 1 : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 cgrid((unsigned)((cols + 63) / 64), (unsigned)(rows / rows_per_batch), 1);
   if (kind == kAdaLN) {
@@ -379,15 +392,19 @@ int check_rope(const Rope& rope, int64_t rows, int64_t cols) {
 }
 
 int forward(int kind, void* y, const void* x, const void* p0, const void* p1, float* mean, float* rstd, void* x_norm,
-            int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream, const Rope* rope = nullptr) {
+            int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream, const Rope* rope = nullptr,
+            const Params* params = nullptr) {
   if (rows == 0) return TT_OK;
   if (!y || !x || !p0 || (kind == kAdaLN && !p1)) return TT_ERR_INVALID_ARGUMENT;
+  const Params dense{cols, cols, 0, nullptr};
+  const Params& pm = params ? *params : dense;
+  const bool aligned = vector_path(cols, {y, x, p0, p1, x_norm, pm.copy}) && (pm.stride0 | pm.stride1) % kPack == 0;
   if (rope) {
-    if (!vector_path(cols, {y, x, p0})) return TT_ERR_UNSUPPORTED;
+    if (!aligned) return TT_ERR_UNSUPPORTED;
     const int rrc = check_rope(*rope, rows, cols);
     if (rrc != TT_OK) return rrc;
-  } else if (!vector_path(cols, {y, x, p0, p1, x_norm})) {
-    return forward_generic(kind, y, x, p0, p1, mean, rstd, x_norm, rows, cols, rows_per_batch, eps, stream);
+  } else if (!aligned) {
+    return forward_generic(kind, y, x, p0, p1, mean, rstd, x_norm, rows, cols, rows_per_batch, eps, stream, params);
   }
   Plan p;
   if (x_norm && (kind != kAdaLN || rope)) return TT_ERR_UNSUPPORTED;
@@ -397,6 +414,7 @@ int forward(int kind, void* y, const void* x, const void* p0, const void* p1, fl
   FwdArgs a;
   a.freqs = rope ? rope->freqs : nullptr; a.seq_len = rope ? rope->seq_len : 1; a.head_dim = rope ? (int)rope->head_dim : 8;
   a.rows_per_pos = rope && rope->heads > 0 ? rope->heads : 1;
+  a.p0_stride = pm.stride0; a.p1_stride = pm.stride1; a.p0_f32 = pm.f32; a.p0_copy = pm.copy;
   a.y = y; a.x = x; a.p0 = p0; a.p1 = p1; a.mean = mean; a.rstd = rstd; a.x_norm = x_norm;
   a.rows_per_batch = rows_per_batch; a.n_tiles = p.n_tiles;
   a.cols = (int)cols; a.packs = p.packs; a.eps = eps; a.inv_cols = 1.0f / (float)cols;
@@ -536,19 +554,26 @@ int tt_reduce_partials(float* out0, float* out1, const void* workspace,
   return reduce(out0, out1, workspace, n_batches, n_partials, n_acc, cols, false, stream);
 }
 
-int tt_adaln_backward(void* dx, float* dscale, float* dshift, const void* dy, const void* x, const void* scale,
-                      void* workspace, size_t workspace_bytes,
-                      int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream) {
+int tt_adaln_backward_typed(void* dx, void* dscale, void* dshift, int grads_bf16, const void* dy, const void* x,
+                            const void* scale, void* workspace, size_t workspace_bytes,
+                            int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream) {
   if (rows == 0) return TT_OK;
   if (!dscale || !dshift) return TT_ERR_INVALID_ARGUMENT;
   if (!vector_path(cols, {dx, dy, x, scale, workspace}))
     return backward_generic(kAdaLN, dx, dscale, dshift, dy, x, scale, workspace, workspace_bytes,
-                            rows, cols, rows_per_batch, eps, stream);
+                            rows, cols, rows_per_batch, eps, stream, grads_bf16 != 0);
   int n_partials = 0;
   int rc = backward_partials(kAdaLN, dx, dy, x, scale, workspace, workspace_bytes, &n_partials,
                              rows, cols, rows_per_batch, eps, stream);
   if (rc != TT_OK) return rc;
-  return reduce(dscale, dshift, workspace, (int)(rows / rows_per_batch), n_partials, 2, cols, false, stream);
+  return reduce(dscale, dshift, workspace, (int)(rows / rows_per_batch), n_partials, 2, cols, grads_bf16 != 0, stream);
+}
+
+int tt_adaln_backward(void* dx, float* dscale, float* dshift, const void* dy, const void* x, const void* scale,
+                      void* workspace, size_t workspace_bytes,
+                      int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream) {
+  return tt_adaln_backward_typed(dx, dscale, dshift, 0, dy, x, scale, workspace, workspace_bytes,
+                                 rows, cols, rows_per_batch, eps, stream);
 }
 
 int tt_adaln_backward_static(void* dx, float* dscale, float* dshift, const void* dy, const void* x,
@@ -563,19 +588,43 @@ int tt_adaln_backward_static(void* dx, float* dscale, float* dshift, const void*
   return rc == TT_ERR_WORKSPACE ? TT_ERR_STATIC_LIMIT : rc;
 }
 
+int tt_rmsnorm_backward_typed(void* dx, void* dweight, int grads_bf16, const void* dy, const void* x, const void* weight,
+                              const float* freqs, int64_t head_dim, int64_t heads, int64_t seq_len,
+                              void* workspace, size_t workspace_bytes,
+                              int64_t rows, int64_t cols, float eps, void* stream) {
+  if (rows == 0) return TT_OK;
+  if (!dweight) return TT_ERR_INVALID_ARGUMENT;
+  Rope rope;
+  rope.freqs = freqs; rope.head_dim = head_dim; rope.seq_len = seq_len; rope.heads = heads;
+  if (!freqs && !vector_path(cols, {dx, dy, x, weight, workspace}))
+    return backward_generic(kRMS, dx, dweight, nullptr, dy, x, weight, workspace, workspace_bytes,
+                            rows, cols, rows, eps, stream, grads_bf16 != 0);
+  int n_partials = 0;
+  int rc = backward_partials(kRMS, dx, dy, x, weight, workspace, workspace_bytes, &n_partials,
+                             rows, cols, rows, eps, stream, freqs ? &rope : nullptr);
+  if (rc != TT_OK) return rc;
+  return reduce(dweight, nullptr, workspace, 1, n_partials, 1, cols, grads_bf16 != 0, stream);
+}
+
 int tt_rmsnorm_backward(void* dx, float* dweight, const void* dy, const void* x, const void* weight,
                         void* workspace, size_t workspace_bytes,
                         int64_t rows, int64_t cols, float eps, void* stream) {
-  if (rows == 0) return TT_OK;
-  if (!dweight) return TT_ERR_INVALID_ARGUMENT;
-  if (!vector_path(cols, {dx, dy, x, weight, workspace}))
-    return backward_generic(kRMS, dx, dweight, nullptr, dy, x, weight, workspace, workspace_bytes,
-                            rows, cols, rows, eps, stream);
-  int n_partials = 0;
-  int rc = backward_partials(kRMS, dx, dy, x, weight, workspace, workspace_bytes, &n_partials,
-                             rows, cols, rows, eps, stream);
-  if (rc != TT_OK) return rc;
-  return reduce(dweight, nullptr, workspace, 1, n_partials, 1, cols, false, stream);
+  return tt_rmsnorm_backward_typed(dx, dweight, 0, dy, x, weight, nullptr, 0, 0, 0, workspace, workspace_bytes,
+                                   rows, cols, eps, stream);
+}
+
+int tt_adaln_forward_strided(void* y, const void* x, const void* scale, int64_t scale_stride,
+                             const void* shift, int64_t shift_stride, void* scale_copy,
+                             int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream) {
+  if (scale_stride < 0 || shift_stride < 0) return TT_ERR_INVALID_ARGUMENT;
+  const Params pm{scale_stride, shift_stride, 0, scale_copy};
+  return forward(kAdaLN, y, x, scale, shift, nullptr, nullptr, nullptr, rows, cols, rows_per_batch, eps, stream, nullptr, &pm);
+}
+
+int tt_rmsnorm_forward_f32_weight(void* y, const void* x, const float* weight, void* weight_copy,
+                                  int64_t rows, int64_t cols, float eps, void* stream) {
+  const Params pm{0, 0, 1, weight_copy};
+  return forward(kRMS, y, x, weight, nullptr, nullptr, nullptr, nullptr, rows, cols, rows, eps, stream, nullptr, &pm);
 }
 
 // ---------------------------------------------------------------- RMSNorm + rotary embedding
@@ -621,27 +670,34 @@ int tt_rmsnorm_rope_heads_backward(void* dx, float* dweight, const void* dy, con
 }
 
 // ---------------------------------------------------------------- gated residual add
-int tt_gate_residual_forward(void* out, const void* x, const void* gate, const void* residual,
-                             int64_t rows, int64_t cols, int64_t rows_per_batch, void* stream) {
+int tt_gate_residual_forward_strided(void* out, const void* x, const void* gate, int64_t gate_stride, void* gate_copy,
+                                     const void* residual, int64_t rows, int64_t cols, int64_t rows_per_batch,
+                                     void* stream) {
   if (rows == 0) return TT_OK;
-  if (!out || !x || !gate || !residual) return TT_ERR_INVALID_ARGUMENT;
-  if (!vector_path(cols, {out, x, gate, residual})) return TT_ERR_UNSUPPORTED;
+  if (!out || !x || !gate || !residual || gate_stride < 0) return TT_ERR_INVALID_ARGUMENT;
+  if (!vector_path(cols, {out, x, gate, residual, gate_copy}) || gate_stride % kPack != 0) return TT_ERR_UNSUPPORTED;
   Plan p;
   int rc = make_plan(kGateKind, kFwd, rows, cols, rows_per_batch, &p);
   if (rc != TT_OK) return rc;
   GateArgs a;
   a.out = out; a.a = x; a.b = residual; a.gate = gate; a.partials = nullptr;
+  a.gate_stride = gate_stride; a.gate_copy = gate_copy;
   a.rows_per_batch = rows_per_batch; a.n_tiles = p.n_tiles; a.cols = (int)cols; a.packs = p.packs;
   return launch(p, a, stream);
+}
+
+int tt_gate_residual_forward(void* out, const void* x, const void* gate, const void* residual,
+                             int64_t rows, int64_t cols, int64_t rows_per_batch, void* stream) {
+  return tt_gate_residual_forward_strided(out, x, gate, cols, nullptr, residual, rows, cols, rows_per_batch, stream);
 }
 
 size_t tt_gate_residual_backward_workspace_bytes(int64_t rows, int64_t cols, int64_t rows_per_batch) {
   return cols % kPack == 0 ? workspace_for(kGateKind, 1, rows, cols, rows_per_batch) : 0;
 }
 
-int tt_gate_residual_backward(void* dresidual, float* dgate, const void* dout, const void* gate,
-                              const void* residual, void* workspace, size_t workspace_bytes,
-                              int64_t rows, int64_t cols, int64_t rows_per_batch, void* stream) {
+int tt_gate_residual_backward_typed(void* dresidual, void* dgate, int grads_bf16, const void* dout, const void* gate,
+                                    const void* residual, void* workspace, size_t workspace_bytes,
+                                    int64_t rows, int64_t cols, int64_t rows_per_batch, void* stream) {
   if (rows == 0) return TT_OK;
   if (!dresidual || !dgate || !dout || !gate || !residual) return TT_ERR_INVALID_ARGUMENT;
   if (!vector_path(cols, {dresidual, dout, gate, residual})) return TT_ERR_UNSUPPORTED;
@@ -651,23 +707,36 @@ int tt_gate_residual_backward(void* dresidual, float* dgate, const void* dout, c
   if (!workspace || !aligned16(workspace) || workspace_bytes < partial_bytes(p, 1, cols)) return TT_ERR_WORKSPACE;
   GateArgs a;
   a.out = dresidual; a.a = dout; a.b = residual; a.gate = gate; a.partials = static_cast<float*>(workspace);
+  a.gate_stride = cols; a.gate_copy = nullptr;
   a.rows_per_batch = rows_per_batch; a.n_tiles = p.n_tiles; a.cols = (int)cols; a.packs = p.packs;
   rc = launch(p, a, stream);
   if (rc != TT_OK) return rc;
-  return reduce(dgate, nullptr, workspace, (int)(rows / rows_per_batch), p.grid_x, 1, cols, false, stream);
+  return reduce(dgate, nullptr, workspace, (int)(rows / rows_per_batch), p.grid_x, 1, cols, grads_bf16 != 0, stream);
+}
+
+int tt_gate_residual_backward(void* dresidual, float* dgate, const void* dout, const void* gate,
+                              const void* residual, void* workspace, size_t workspace_bytes,
+                              int64_t rows, int64_t cols, int64_t rows_per_batch, void* stream) {
+  return tt_gate_residual_backward_typed(dresidual, dgate, 0, dout, gate, residual, workspace, workspace_bytes,
+                                         rows, cols, rows_per_batch, stream);
 }
 
 // ---------------------------------------------------------------- residual update + LayerNorm
 // scale / shift / gate hold either one vector for all batches or one per batch.
 static bool stride_ok(int64_t n_vectors, int64_t n_batches) { return n_vectors == 1 || n_vectors == n_batches; }
 
-int tt_residual_norm_forward(void* s, void* y, const void* x, const void* r, const void* gate, int64_t n_gate,
-                             const void* scale, const void* shift, int64_t n_param, int affine,
-                             float* mean, float* rstd, int64_t rows, int64_t cols, int64_t rows_per_batch,
-                             float eps, void* stream) {
+int tt_residual_norm_forward_strided(void* s, void* y, const void* x, const void* r,
+                                     const void* gate, int64_t n_gate, int64_t gate_stride, void* gate_copy,
+                                     const void* scale, int64_t scale_stride, void* scale_copy,
+                                     const void* shift, int64_t shift_stride, int64_t n_param, int affine,
+                                     float* mean, float* rstd, int64_t rows, int64_t cols, int64_t rows_per_batch,
+                                     float eps, void* stream) {
   if (rows == 0) return TT_OK;
   if (!s || !y || !x || !r || !scale || !shift) return TT_ERR_INVALID_ARGUMENT;
-  if (!vector_path(cols, {s, y, x, r, gate, scale, shift})) return TT_ERR_UNSUPPORTED;
+  if (gate_stride < 0 || scale_stride < 0 || shift_stride < 0) return TT_ERR_INVALID_ARGUMENT;
+  if (!vector_path(cols, {s, y, x, r, gate, scale, shift, gate_copy, scale_copy}) ||
+      (gate_stride | scale_stride | shift_stride) % kPack != 0)
+    return TT_ERR_UNSUPPORTED;
   Plan p;
   int rc = make_plan(kAdaLN, kFwd, rows, cols, rows_per_batch, &p, false, gate ? 2 : 1);
   if (rc != TT_OK) return rc;
@@ -675,9 +744,19 @@ int tt_residual_norm_forward(void* s, void* y, const void* x, const void* r, con
   ResFwdArgs a;
   a.s = s; a.y = y; a.x = x; a.r = r; a.gate = gate; a.scale = scale; a.shift = shift; a.mean = mean; a.rstd = rstd;
   a.rows_per_batch = rows_per_batch; a.n_tiles = p.n_tiles;
-  a.gate_stride = n_gate == 1 ? 0 : cols; a.param_stride = n_param == 1 ? 0 : cols;
+  a.gate_stride = n_gate == 1 ? 0 : gate_stride; a.gate_copy = gate_copy; a.scale_copy = scale_copy;
+  a.gate_copy_stride = n_gate == 1 ? 0 : cols; a.scale_copy_stride = n_param == 1 ? 0 : cols;
+  a.scale_stride = n_param == 1 ? 0 : scale_stride; a.shift_stride = n_param == 1 ? 0 : shift_stride;
   a.cols = (int)cols; a.packs = p.packs; a.eps = eps; a.inv_cols = 1.0f / (float)cols; a.one = affine ? 0.f : 1.f;
   return launch(p, a, stream);
+}
+
+int tt_residual_norm_forward(void* s, void* y, const void* x, const void* r, const void* gate, int64_t n_gate,
+                             const void* scale, const void* shift, int64_t n_param, int affine,
+                             float* mean, float* rstd, int64_t rows, int64_t cols, int64_t rows_per_batch,
+                             float eps, void* stream) {
+  return tt_residual_norm_forward_strided(s, y, x, r, gate, n_gate, cols, nullptr, scale, cols, nullptr, shift, cols,
+                                          n_param, affine, mean, rstd, rows, cols, rows_per_batch, eps, stream);
 }
 
 size_t tt_residual_norm_backward_workspace_bytes(int64_t rows, int64_t cols, int64_t rows_per_batch, int gated) {
@@ -690,7 +769,7 @@ size_t tt_residual_norm_backward_workspace_bytes(int64_t rows, int64_t cols, int
   return need < 16 ? 16 : need;
 }
 
-int tt_residual_norm_backward(void* dx, void* dr, float* dscale, float* dshift, float* dgate,
+int tt_residual_norm_backward_typed(void* dx, void* dr, void* dscale, void* dshift, void* dgate, int grads_bf16,
                               const void* dy, const void* ds_in, const void* s, const void* r,
                               const void* gate, int64_t n_gate, const void* scale, int64_t n_param, int affine,
                               void* workspace, size_t workspace_bytes,
@@ -714,7 +793,16 @@ int tt_residual_norm_backward(void* dx, void* dr, float* dscale, float* dshift, 
   a.cols = (int)cols; a.packs = p.packs; a.eps = eps; a.inv_cols = 1.0f / (float)cols; a.one = affine ? 0.f : 1.f;
   rc = launch(p, a, stream);
   if (rc != TT_OK) return rc;
-  return reduce(dscale, dshift, workspace, (int)p.n_batches, p.grid_x, n_acc, cols, false, stream, dgate);
+  return reduce(dscale, dshift, workspace, (int)p.n_batches, p.grid_x, n_acc, cols, grads_bf16 != 0, stream, dgate);
+}
+
+int tt_residual_norm_backward(void* dx, void* dr, float* dscale, float* dshift, float* dgate,
+                              const void* dy, const void* ds_in, const void* s, const void* r,
+                              const void* gate, int64_t n_gate, const void* scale, int64_t n_param, int affine,
+                              void* workspace, size_t workspace_bytes,
+                              int64_t rows, int64_t cols, int64_t rows_per_batch, float eps, void* stream) {
+  return tt_residual_norm_backward_typed(dx, dr, dscale, dshift, dgate, 0, dy, ds_in, s, r, gate, n_gate, scale, n_param,
+                                         affine, workspace, workspace_bytes, rows, cols, rows_per_batch, eps, stream);
 }
 
 // ---------------------------------------------------------------- bare streaming probe

@@ -13,6 +13,8 @@ struct GateArgs {
   const void* a;     // forward: x;              backward: dout
   const void* b;     // forward: residual;       backward: residual
   const void* gate;  // [B, C] bf16
+  int64_t gate_stride;   // elements between the gate vectors of consecutive batches
+  void* gate_copy;   // optional (forward): the gate vectors without gaps, as FwdArgs::p0_copy
   float* partials;   // backward: [B][gridDim.x][1][C]
   int64_t rows_per_batch;
   int64_t n_tiles;
@@ -42,7 +44,10 @@ __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
     act[p] = FULL || pk < a.packs;
     col[p] = pk * kPack;
     u32x4 r0 = {0, 0, 0, 0};
-    if (act[p]) r0 = load_cached(a.gate, b * C + col[p]);
+    if (act[p]) {
+      r0 = load_cached(a.gate, b * a.gate_stride + col[p]);
+      if (a.gate_copy && blockIdx.x == 0 && q == 0) store_any(a.gate_copy, b * C + col[p], r0, kPack);
+    }
     unpack8(r0, g[p]);
 #pragma unroll
     for (int j = 0; j < 8; ++j) { acc0[p][j] = 0.f; acc1[p][j] = 0.f; }
@@ -121,7 +126,10 @@ __global__ __launch_bounds__(64 * NW) void gate_narrow(const GateArgs a) {
   float g[8], acc0[8], acc1[8];
   {
     u32x4 r0 = {0, 0, 0, 0};
-    if (act) r0 = load_cached(a.gate, b * C + col);
+    if (act) {
+      r0 = load_cached(a.gate, b * a.gate_stride + col);
+      if (a.gate_copy && blockIdx.x == 0 && wave == 0 && ri == 0) store_any(a.gate_copy, b * C + col, r0, kPack);
+    }
     unpack8(r0, g);
 #pragma unroll
     for (int j = 0; j < 8; ++j) { acc0[j] = 0.f; acc1[j] = 0.f; }

@@ -48,6 +48,13 @@ struct FwdArgs {
   int64_t seq_len;
   int head_dim;
   int64_t rows_per_pos;   // narrow ROPE kernels: consecutive rows (heads) that share one position
+  // AdaLN: elements between the scale (shift) vectors of consecutive batches; RMSNorm: 0
+  int64_t p0_stride, p1_stride;
+  int p0_f32;             // p0 holds fp32, rounded to bf16 as it is read (RMSNorm)
+  void* p0_copy;          // optional: p0 as bf16 [B, C] without gaps, written for the backward to read.
+                          // It and the strides take the place of the copy and cast launches that a slice
+                          // of a modulation tensor or an fp32 weight cost in front of every forward
+                          // (about 4 us each on the GPU, next to 4 us for 512 x 5120).
 };
 
 struct BwdArgs {
@@ -119,7 +126,7 @@ __device__ __forceinline__ void rowgroup_allsum(float (&v)[NV], float* buf, int 
 }
 
 // ============================================================================ wide forward
-// Parameters of a lane, and its own values of a loaded pack, for any row mode; `n` as in the kernels.
+// A lane's own values of a loaded pack, and its pack of a parameter, for any row mode; `n` as in the kernels.
 template <int ROWS>
 __device__ __forceinline__ u32x4 own_values(u32x4 v, int n) {
   if constexpr (ROWS == kOdd) {
@@ -128,7 +135,14 @@ __device__ __forceinline__ u32x4 own_values(u32x4 v, int n) {
   return v;
 }
 template <int ROWS>
-__device__ __forceinline__ u32x4 load_pack(const void* base, size_t elem_off, int n) {
+__device__ __forceinline__ u32x4 load_pack(const void* base, size_t elem_off, int n, bool f32 = false) {
+  if (f32) {
+    const float* p = static_cast<const float*>(base) + elem_off;
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = j < n ? p[j] : 0.f;
+    return pack8(v);
+  }
   if constexpr (ROWS == kOdd) return own_values<ROWS>(load_any(base, elem_off - (kPack - n)), n);
   else return load_cached(base, elem_off);
 }
@@ -162,8 +176,9 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
     n[p] = !act[p] ? 0 : pk == a.packs - 1 ? kPack - drop : kPack;
     u32x4 r0 = {0, 0, 0, 0}, r1 = {0, 0, 0, 0};
     if (act[p]) {
-      r0 = load_pack<ROWS>(a.p0, (ADALN ? b * C : 0) + col[p], n[p]);
-      if constexpr (ADALN) r1 = load_pack<ROWS>(a.p1, b * C + col[p], n[p]);
+      r0 = load_pack<ROWS>(a.p0, (ADALN ? b * a.p0_stride : 0) + col[p], n[p], !ADALN && a.p0_f32);
+      if constexpr (ADALN) r1 = load_pack<ROWS>(a.p1, b * a.p1_stride + col[p], n[p]);
+      if (a.p0_copy && blockIdx.x == 0 && q == 0) store_any(a.p0_copy, b * C + col[p], r0, n[p]);
     }
     unpack8(r0, g[p]);
     unpack8(r1, sh[p]);
@@ -618,8 +633,9 @@ __global__ __launch_bounds__(64 * NW) void norm_fwd_narrow(const FwdArgs a) {
   {
     u32x4 r0 = {0, 0, 0, 0}, r1 = {0, 0, 0, 0};
     if (act) {
-      r0 = load_cached(a.p0, (ADALN ? b * C : 0) + col);
-      if constexpr (ADALN) r1 = load_cached(a.p1, b * C + col);
+      r0 = load_pack<kMasked>(a.p0, (ADALN ? b * a.p0_stride : 0) + col, kPack, !ADALN && a.p0_f32);
+      if constexpr (ADALN) r1 = load_cached(a.p1, b * a.p1_stride + col);
+      if (a.p0_copy && blockIdx.x == 0 && wave == 0 && ri == 0) store_any(a.p0_copy, b * C + col, r0, kPack);
     }
     unpack8(r0, g);
     unpack8(r1, sh);

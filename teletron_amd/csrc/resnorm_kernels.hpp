@@ -34,7 +34,10 @@ struct ResFwdArgs {
   int64_t rows_per_batch;
   int64_t n_tiles;
   int64_t gate_stride;   // elements between the gate vectors of consecutive batches: cols or 0
-  int64_t param_stride;  // same for scale / shift
+  int64_t scale_stride, shift_stride;   // same for scale / shift
+  void* gate_copy;       // optional: as FwdArgs::p0_copy
+  void* scale_copy;
+  int64_t gate_copy_stride, scale_copy_stride;   // cols, or 0 for one vector shared by all batches
   int cols;
   int packs;
   float eps;
@@ -129,9 +132,13 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs 
     col[p] = pk * kPack;
     u32x4 r0 = {0, 0, 0, 0}, r1 = {0, 0, 0, 0}, r2 = {0, 0, 0, 0};
     if (act[p]) {
-      r0 = load_cached(a.scale, b * a.param_stride + col[p]);
-      r1 = load_cached(a.shift, b * a.param_stride + col[p]);
+      r0 = load_cached(a.scale, b * a.scale_stride + col[p]);
+      r1 = load_cached(a.shift, b * a.shift_stride + col[p]);
       if constexpr (GATED) r2 = load_cached(a.gate, b * a.gate_stride + col[p]);
+      if (blockIdx.x == 0 && q == 0) {
+        if (a.scale_copy && (b == 0 || a.scale_copy_stride)) store_any(a.scale_copy, b * C + col[p], r0, kPack);
+        if (GATED && a.gate_copy && (b == 0 || a.gate_copy_stride)) store_any(a.gate_copy, b * C + col[p], r2, kPack);
+      }
     }
     unpack8(r0, g[p]);
     unpack8(r1, sh[p]);

@@ -45,18 +45,21 @@ def _adaln_forward(ctx, x, scale, shift, epsilon, cols):
     ctx.scale_meta = (scale.shape, scale.dtype)
     ctx.shift_meta = (shift.shape, shift.dtype)
     x = x.contiguous()
-    scale_c = scale.detach().to(torch.bfloat16).contiguous()
-    y = ops.adaln_forward(x, scale_c, shift.detach(), ctx.eps)
-    ctx.save_for_backward(x, scale_c)
+    save = any(ctx.needs_input_grad)
+    y, scale_c = ops.adaln_forward_saving(x, scale.detach(), shift.detach(), ctx.eps, save)
+    if save:
+        ctx.save_for_backward(x, scale_c)
     return y
 
 
 def _adaln_backward(ctx, grad_output, grad_reduce=None):
     x, scale_c = ctx.saved_tensors
-    dx, grads = ops.adaln_backward_packed(grad_output.contiguous(), x, scale_c, ctx.eps)
+    (sc_shape, sc_dtype), (sh_shape, sh_dtype) = ctx.scale_meta, ctx.shift_meta
+    # one rounding to the parameters' dtype in the kernel, unless an exchange in fp32 comes first
+    dtype = ops._grad_dtype(sc_dtype) if grad_reduce is None and sc_dtype == sh_dtype else torch.float32
+    dx, grads = ops.adaln_backward_packed(grad_output.contiguous(), x, scale_c, ctx.eps, dtype)
     if grad_reduce is not None:
         grad_reduce(grads)                  # fp32 [2, n_batches, C]: dscale and dshift in ONE exchange, before the cast
-    (sc_shape, sc_dtype), (sh_shape, sh_dtype) = ctx.scale_meta, ctx.shift_meta
     if sc_dtype == sh_dtype:
         grads = grads.to(sc_dtype)          # both parameter gradients in one cast
     dx = dx if ctx.needs_input_grad[0] else None
@@ -103,9 +106,10 @@ class RMSNormModelFunction(Function):
         ctx.weight_meta = (weight.shape, weight.dtype)
         if ops.memory_order_view(x)[0] is None:      # dense permuted views are handled without a copy
             x = x.contiguous()
-        weight_c = weight.detach().to(torch.bfloat16).contiguous()
-        y = ops.rmsnorm_forward(x, weight_c, ctx.eps)
-        ctx.save_for_backward(x, weight_c)
+        save = any(ctx.needs_input_grad)
+        y, weight_c = ops.rmsnorm_forward_saving(x, weight.detach(), ctx.eps, save)
+        if save:
+            ctx.save_for_backward(x, weight_c)
         return y
 
     @staticmethod
@@ -113,8 +117,8 @@ class RMSNormModelFunction(Function):
         x, weight_c = ctx.saved_tensors
         if x.is_contiguous():
             grad_output = grad_output.contiguous()
-        dx, dweight = ops.rmsnorm_backward(grad_output, x, weight_c, ctx.eps)
         w_shape, w_dtype = ctx.weight_meta
+        dx, dweight = ops.rmsnorm_backward(grad_output, x, weight_c, ctx.eps, ops._grad_dtype(w_dtype))
         dx = dx if ctx.needs_input_grad[0] else None
         dweight = dweight.to(w_dtype).reshape(w_shape) if ctx.needs_input_grad[1] else None
         return dx, dweight, None, None
@@ -141,8 +145,9 @@ class RMSNormRopeFunction(Function):
     @staticmethod
     def backward(ctx, grad_output):
         x, weight_c, freqs_c = ctx.saved_tensors
-        dx, dweight = ops.rmsnorm_rope_backward(grad_output.contiguous(), x, weight_c, freqs_c, ctx.eps, ctx.head_dim)
         w_shape, w_dtype = ctx.weight_meta
+        dx, dweight = ops.rmsnorm_rope_backward(grad_output.contiguous(), x, weight_c, freqs_c, ctx.eps, ctx.head_dim,
+                                                ops._grad_dtype(w_dtype))
         return (dx if ctx.needs_input_grad[0] else None,
                 dweight.to(w_dtype).reshape(w_shape) if ctx.needs_input_grad[1] else None, None, None, None)
 
@@ -167,8 +172,8 @@ class RMSNormRopeHeadsFunction(Function):
     @staticmethod
     def backward(ctx, grad_output):
         x, weight_c, freqs_c = ctx.saved_tensors
-        dx, dweight = ops.rmsnorm_rope_heads_backward(grad_output, x, weight_c, freqs_c, ctx.eps)
         w_shape, w_dtype = ctx.weight_meta
+        dx, dweight = ops.rmsnorm_rope_heads_backward(grad_output, x, weight_c, freqs_c, ctx.eps, ops._grad_dtype(w_dtype))
         return (dx if ctx.needs_input_grad[0] else None,
                 dweight.to(w_dtype).reshape(w_shape) if ctx.needs_input_grad[1] else None, None, None)
 
@@ -188,10 +193,12 @@ def rope_table_from_cos_sin(cos: torch.Tensor, sin: torch.Tensor, extra_tokens: 
 def _gate_forward(ctx, x, gate, residual):
     _check_row_groups(x, gate)
     ctx.gate_meta = (gate.shape, gate.dtype)
-    gate_c = gate.detach().to(torch.bfloat16).contiguous()
     residual = residual.contiguous()
-    ctx.save_for_backward(gate_c, residual)
-    return ops.gate_residual_forward(x.contiguous(), gate_c, residual)
+    save = any(ctx.needs_input_grad)
+    out, gate_c = ops.gate_residual_forward_saving(x.contiguous(), gate.detach(), residual, save)
+    if save:
+        ctx.save_for_backward(gate_c, residual)
+    return out
 
 
 def _gate_backward(ctx, grad_output, grad_reduce=None):
@@ -199,7 +206,8 @@ def _gate_backward(ctx, grad_output, grad_reduce=None):
     g_shape, g_dtype = ctx.gate_meta
     if not (ctx.needs_input_grad[1] or ctx.needs_input_grad[2]):
         return grad_output, None, None
-    dres, dgate = ops.gate_residual_backward(grad_output.contiguous(), gate_c, residual)
+    dres, dgate = ops.gate_residual_backward(grad_output.contiguous(), gate_c, residual,
+                                             ops._grad_dtype(g_dtype) if grad_reduce is None else torch.float32)
     if grad_reduce is not None and ctx.needs_input_grad[1]:
         grad_reduce(dgate)                  # fp32 [n_batches, C], before the cast
     return (grad_output if ctx.needs_input_grad[0] else None,
@@ -253,12 +261,13 @@ class ResidualNormFunction(Function):
         _check_row_groups(x, gate, scale, shift)
         ctx.set_materialize_grads(False)
         ctx.metas = [None if t is None else (t.shape, t.dtype) for t in (gate, scale, shift)]
-        bf = torch.bfloat16
-        gate_c = None if gate is None else gate.detach().to(bf).contiguous()
-        scale_c = scale.detach().to(bf).contiguous()
+        save = any(ctx.needs_input_grad)
         residual = residual.contiguous()
-        s, y = ops.residual_norm_forward(x.contiguous(), residual, gate_c, scale_c, shift.detach(), ctx.eps, ctx.affine)
-        ctx.save_for_backward(s, residual if gate is not None else None, gate_c, scale_c)
+        s, y, gate_c, scale_c = ops.residual_norm_forward_saving(
+            x.contiguous(), residual, None if gate is None else gate.detach(), scale.detach(), shift.detach(),
+            ctx.eps, ctx.affine, save)
+        if save:
+            ctx.save_for_backward(s, residual if gate is not None else None, gate_c, scale_c)
         return s, y
 
     @staticmethod
@@ -266,9 +275,13 @@ class ResidualNormFunction(Function):
         s, residual, gate_c, scale_c = ctx.saved_tensors
         if grad_y is None:
             grad_y = torch.zeros_like(s)
+        # one rounding in the kernel where every gradient leaves as it is: bf16, one vector per batch
+        n = max(c.numel() for c in (gate_c, scale_c) if c is not None)
+        direct = ctx.grad_reduce is None and all(
+            m is None or (m[1] == torch.bfloat16 and m[0].numel() == n) for m in ctx.metas)
         dx, dr, dscale, dshift, dgate = ops.residual_norm_backward(
             grad_y.contiguous(), None if grad_s is None else grad_s.contiguous(), s, residual, gate_c, scale_c,
-            ctx.eps, ctx.affine)
+            ctx.eps, ctx.affine, torch.bfloat16 if direct else torch.float32)
         if ctx.grad_reduce is not None:
             parts = [g for g in ((dgate,) if ctx.affine else (dscale, dshift, dgate)) if g is not None]
             if parts:

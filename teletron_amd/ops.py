@@ -98,6 +98,76 @@ def _batches(x: torch.Tensor, scale: torch.Tensor, cols: int) -> Tuple[int, int,
     return rows, nb, (rows // nb if nb else rows)
 
 
+def _vectors(p: torch.Tensor, cols: int):
+    """Elements between consecutive vectors of a parameter, or None where they are not evenly spaced
+    ([B, 1, C] slices of a [B, 6, C] modulation tensor are)."""
+    if p.dtype != BF16 or p.stride(-1) != 1:
+        return None
+    outer = [(n, st) for n, st in zip(p.shape[:-1], p.stride()[:-1]) if n != 1]
+    return outer[0][1] if len(outer) == 1 else cols if not outer else None
+
+
+def _grad_dtype(dtype: torch.dtype) -> torch.dtype:
+    """Type in which parameter gradients leave the kernels: the parameter's own where that is bf16."""
+    return BF16 if dtype == BF16 else torch.float32
+
+
+def adaln_forward_saving(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor, eps: float, save: bool):
+    """``(adaln_forward(x, scale, shift, eps), scale as dense bf16)``, the latter for backward (undefined
+    without ``save``).  Slices of a modulation tensor are read in place and the dense scale is written by the
+    same launch."""
+    cols = x.shape[-1]
+    if scale.is_contiguous() and shift.is_contiguous():
+        scale = scale.to(BF16)
+        return adaln_forward(x, scale, shift, eps), scale
+    st, sh = _vectors(scale, cols), _vectors(shift, cols)
+    if (st is None or sh is None or scale.shape[-1] != cols or shift.shape != scale.shape
+            or scale.device != x.device or shift.device != x.device):
+        scale = scale.to(BF16).contiguous()
+        return adaln_forward(x, scale, shift, eps), scale
+    x = _check_act("x", x, cols)
+    rows, nb, rpb = _batches(x, scale, cols)
+    y = torch.empty_like(x)
+    kept = torch.empty(nb, cols, dtype=BF16, device=x.device) if save else scale
+    if rows:
+        with torch.cuda.device(x.device):
+            rc = cabi.load().tt_adaln_forward_strided(
+                y.data_ptr(), x.data_ptr(), scale.data_ptr(), st, shift.data_ptr(), sh, kept.data_ptr() if save else None,
+                rows, cols, rpb, float(eps), _stream(x))
+        if rc == cabi.TT_ERR_UNSUPPORTED:          # element-wise kernels: dense parameters only
+            scale = scale.contiguous()
+            return adaln_forward(x, scale, shift, eps), scale
+        cabi.check("tt_adaln_forward_strided", rc)
+    return y, kept
+
+
+def rmsnorm_forward_saving(x: torch.Tensor, weight: torch.Tensor, eps: float, save: bool):
+    """``(rmsnorm_forward(x, weight, eps), weight as bf16)``, the latter for backward (undefined without
+    ``save``).  An fp32 weight is rounded by the same launch."""
+    cols = x.shape[-1]
+    if (weight.dtype != torch.float32 or weight.device != x.device or weight.numel() != cols or weight.dim() < 1
+            or weight.shape[-1] != cols or not weight.is_contiguous()):
+        weight = weight.to(BF16).contiguous()
+        return rmsnorm_forward(x, weight, eps), weight
+    view, perm = memory_order_view(x)
+    xm = _check_act("x", x if view is None else view, cols)
+    rows = xm.numel() // cols
+    y = torch.empty_like(xm)
+    kept = torch.empty(cols, dtype=BF16, device=x.device) if save else weight
+    if rows:
+        with torch.cuda.device(x.device):
+            rc = cabi.load().tt_rmsnorm_forward_f32_weight(
+                y.data_ptr(), xm.data_ptr(), weight.data_ptr(), kept.data_ptr() if save else None,
+                rows, cols, float(eps), _stream(x))
+        if rc == cabi.TT_ERR_UNSUPPORTED:
+            weight = weight.to(BF16)
+            return rmsnorm_forward(x, weight, eps), weight
+        cabi.check("tt_rmsnorm_forward_f32_weight", rc)
+    elif save:
+        kept = weight.to(BF16)
+    return (y if view is None else y.permute(_inverse(perm))), kept
+
+
 _WORKSPACES = {}   # (device index, stream handle) -> uint8 tensor, grown on demand
 _WORKSPACES_LOCK = threading.Lock()   # backward runs on autograd's threads, one per device
 # the element-wise path's row statistics (rows * 8 bytes) are only kept between calls up to this size
@@ -164,9 +234,10 @@ def adaln_forward(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor, eps
     return (y, mean, rstd) if return_stats else y
 
 
-def adaln_backward_packed(dy: torch.Tensor, x: torch.Tensor, scale: torch.Tensor, eps: float):
-    """Returns (dx bf16 like x, grads fp32 [2, n_batches, C]) with grads[0] = dscale, grads[1] = dshift:
-    one tensor, so that a caller casting both to the parameters' dtype needs one launch for it."""
+def adaln_backward_packed(dy: torch.Tensor, x: torch.Tensor, scale: torch.Tensor, eps: float,
+                          dtype: torch.dtype = torch.float32):
+    """Returns (dx bf16 like x, grads [2, n_batches, C] in ``dtype``, fp32 or bf16, rounded once) with
+    grads[0] = dscale, grads[1] = dshift."""
     cols = x.shape[-1]
     x = _check_act("x", x, cols)
     dy = _check_act("dy", dy, cols)
@@ -175,11 +246,11 @@ def adaln_backward_packed(dy: torch.Tensor, x: torch.Tensor, scale: torch.Tensor
     rows, nb, rpb = _batches(x, scale, cols)
     dx = torch.empty_like(x)
     if rows == 0:
-        return dx, torch.zeros(2, nb, cols, dtype=torch.float32, device=x.device)
-    grads = torch.empty(2, nb, cols, dtype=torch.float32, device=x.device)
+        return dx, torch.zeros(2, nb, cols, dtype=dtype, device=x.device)
+    grads = torch.empty(2, nb, cols, dtype=dtype, device=x.device)
     with torch.cuda.device(x.device):
         ws = _workspace(cabi.load().tt_adaln_backward_workspace_bytes(rows, cols, rpb), rows, x, dy, dx, scale)
-        cabi.call("tt_adaln_backward", dx.data_ptr(), grads[0].data_ptr(), grads[1].data_ptr(),
+        cabi.call("tt_adaln_backward_typed", dx.data_ptr(), grads[0].data_ptr(), grads[1].data_ptr(), int(dtype == BF16),
                   dy.data_ptr(), x.data_ptr(), scale.data_ptr(), ws.data_ptr(), ws.numel(),
                   rows, cols, rpb, float(eps), _stream(x))
     return dx, grads
@@ -215,11 +286,12 @@ def rmsnorm_forward(x: torch.Tensor, weight: torch.Tensor, eps: float, return_st
     return (y, rstd) if return_stats else y
 
 
-def rmsnorm_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, eps: float):
-    """Returns (dx bf16 like x, dweight fp32 [C]).  Dense permuted ``x`` as in ``rmsnorm_forward``."""
+def rmsnorm_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, eps: float,
+                     dtype: torch.dtype = torch.float32):
+    """Returns (dx bf16 like x, dweight [C] in ``dtype``, fp32 or bf16).  Dense permuted ``x`` as in ``rmsnorm_forward``."""
     view, perm = memory_order_view(x) if isinstance(x, torch.Tensor) else (None, None)
     if view is not None and isinstance(dy, torch.Tensor) and dy.shape == x.shape:
-        dx, dweight = rmsnorm_backward(dy.permute(perm), view, weight, eps)
+        dx, dweight = rmsnorm_backward(dy.permute(perm), view, weight, eps, dtype)
         return dx.permute(_inverse(perm)), dweight
     cols = x.shape[-1]
     x = _check_act("x", x, cols)
@@ -230,12 +302,12 @@ def rmsnorm_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, ep
     rows = x.numel() // cols
     dx = torch.empty_like(x)
     if rows == 0:
-        return dx, torch.zeros(cols, dtype=torch.float32, device=x.device)
-    dweight = torch.empty(cols, dtype=torch.float32, device=x.device)
+        return dx, torch.zeros(cols, dtype=dtype, device=x.device)
+    dweight = torch.empty(cols, dtype=dtype, device=x.device)
     with torch.cuda.device(x.device):
         ws = _workspace(cabi.load().tt_rmsnorm_backward_workspace_bytes(rows, cols), rows, x, dy, dx, weight)
-        cabi.call("tt_rmsnorm_backward", dx.data_ptr(), dweight.data_ptr(), dy.data_ptr(), x.data_ptr(),
-                  weight.data_ptr(), ws.data_ptr(), ws.numel(), rows, cols, float(eps), _stream(x))
+        cabi.call("tt_rmsnorm_backward_typed", dx.data_ptr(), dweight.data_ptr(), int(dtype == BF16), dy.data_ptr(),
+                  x.data_ptr(), weight.data_ptr(), None, 0, 0, 0, ws.data_ptr(), ws.numel(), rows, cols, float(eps), _stream(x))
     return dx, dweight
 
 
@@ -256,8 +328,35 @@ def gate_residual_forward(x: torch.Tensor, gate: torch.Tensor, residual: torch.T
     return out
 
 
-def gate_residual_backward(dout: torch.Tensor, gate: torch.Tensor, residual: torch.Tensor):
-    """Returns (dresidual bf16 like residual, dgate fp32 [n_batches, C]); dx is dout itself."""
+def gate_residual_forward_saving(x: torch.Tensor, gate: torch.Tensor, residual: torch.Tensor, save: bool):
+    """``(gate_residual_forward(x, gate, residual), gate as dense bf16)``; as ``adaln_forward_saving``."""
+    cols = x.shape[-1]
+    st = None if gate.is_contiguous() else _vectors(gate, cols)
+    if st is None or gate.shape[-1] != cols or gate.device != x.device:
+        gate = gate.to(BF16).contiguous()
+        return gate_residual_forward(x, gate, residual), gate
+    x = _check_act("x", x, cols)
+    residual = _check_act("residual", residual, cols)
+    _require(residual.numel() == x.numel() and residual.device == x.device, ValueError,
+             "residual must match x in size and device")
+    rows, nb, rpb = _batches(x, gate, cols)
+    out = torch.empty_like(x)
+    kept = torch.empty(nb, cols, dtype=BF16, device=x.device) if save else gate
+    if rows:
+        with torch.cuda.device(x.device):
+            rc = cabi.load().tt_gate_residual_forward_strided(
+                out.data_ptr(), x.data_ptr(), gate.data_ptr(), st, kept.data_ptr() if save else None, residual.data_ptr(),
+                rows, cols, rpb, _stream(x))
+        if rc == cabi.TT_ERR_UNSUPPORTED:
+            gate = gate.contiguous()
+            return gate_residual_forward(x, gate, residual), gate
+        cabi.check("tt_gate_residual_forward_strided", rc)
+    return out, kept
+
+
+def gate_residual_backward(dout: torch.Tensor, gate: torch.Tensor, residual: torch.Tensor,
+                           dtype: torch.dtype = torch.float32):
+    """Returns (dresidual bf16 like residual, dgate [n_batches, C] in ``dtype``, fp32 or bf16); dx is dout itself."""
     cols = dout.shape[-1]
     dout = _check_act("dout", dout, cols)
     residual = _check_act("residual", residual, cols)
@@ -267,11 +366,11 @@ def gate_residual_backward(dout: torch.Tensor, gate: torch.Tensor, residual: tor
     rows, nb, rpb = _batches(dout, gate, cols)
     dres = torch.empty_like(residual)
     if rows == 0:
-        return dres, torch.zeros(nb, cols, dtype=torch.float32, device=dout.device)
-    dgate = torch.empty(nb, cols, dtype=torch.float32, device=dout.device)
+        return dres, torch.zeros(nb, cols, dtype=dtype, device=dout.device)
+    dgate = torch.empty(nb, cols, dtype=dtype, device=dout.device)
     with torch.cuda.device(dout.device):
         ws = _workspace(cabi.load().tt_gate_residual_backward_workspace_bytes(rows, cols, rpb), 0, dout)
-        cabi.call("tt_gate_residual_backward", dres.data_ptr(), dgate.data_ptr(), dout.data_ptr(), gate.data_ptr(),
+        cabi.call("tt_gate_residual_backward_typed", dres.data_ptr(), dgate.data_ptr(), int(dtype == BF16), dout.data_ptr(), gate.data_ptr(),
                   residual.data_ptr(), ws.data_ptr(), ws.numel(), rows, cols, rpb, _stream(dout))
     return dres, dgate
 
@@ -306,8 +405,8 @@ def rmsnorm_rope_forward(x: torch.Tensor, weight: torch.Tensor, freqs: torch.Ten
 
 
 def rmsnorm_rope_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, freqs: torch.Tensor,
-                          eps: float, head_dim: int):
-    """Returns (dx bf16 like x, dweight fp32 [C]) for y = rope(rmsnorm(x) * weight)."""
+                          eps: float, head_dim: int, dtype: torch.dtype = torch.float32):
+    """Returns (dx bf16 like x, dweight [C] in ``dtype``, fp32 or bf16) for y = rope(rmsnorm(x) * weight)."""
     cols = x.shape[-1]
     x = _check_act("x", x, cols)
     dy = _check_act("dy", dy, cols)
@@ -317,13 +416,13 @@ def rmsnorm_rope_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tenso
     rows, seq = x.numel() // cols, freqs.shape[0]
     dx = torch.empty_like(x)
     if rows == 0:
-        return dx, torch.zeros(cols, dtype=torch.float32, device=x.device)
-    dweight = torch.empty(cols, dtype=torch.float32, device=x.device)
+        return dx, torch.zeros(cols, dtype=dtype, device=x.device)
+    dweight = torch.empty(cols, dtype=dtype, device=x.device)
     with torch.cuda.device(x.device):
         ws = _workspace(cabi.load().tt_rmsnorm_backward_workspace_bytes(rows, cols), 0, x)
-        cabi.call("tt_rmsnorm_rope_backward", dx.data_ptr(), dweight.data_ptr(), dy.data_ptr(), x.data_ptr(),
-                  weight.data_ptr(), freqs.data_ptr(), ws.data_ptr(), ws.numel(), rows, cols, head_dim, seq,
-                  float(eps), _stream(x))
+        cabi.call("tt_rmsnorm_backward_typed", dx.data_ptr(), dweight.data_ptr(), int(dtype == BF16), dy.data_ptr(),
+                  x.data_ptr(), weight.data_ptr(), freqs.data_ptr(), head_dim, 0, seq, ws.data_ptr(), ws.numel(),
+                  rows, cols, float(eps), _stream(x))
     return dx, dweight
 
 
@@ -360,8 +459,9 @@ def rmsnorm_rope_heads_forward(x: torch.Tensor, weight: torch.Tensor, freqs: tor
     return y if perm is None else y.permute(_inverse(perm))
 
 
-def rmsnorm_rope_heads_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, freqs: torch.Tensor, eps: float):
-    """Returns (dx like x, dweight fp32 [D]) for ``rmsnorm_rope_heads_forward``; dy in x's layout."""
+def rmsnorm_rope_heads_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, freqs: torch.Tensor, eps: float,
+                                dtype: torch.dtype = torch.float32):
+    """Returns (dx like x, dweight [D] in ``dtype``, fp32 or bf16) for ``rmsnorm_rope_heads_forward``; dy in x's layout."""
     xm, perm, weight, freqs, heads, d, seq = _heads_layout(x, weight, freqs)
     _require(isinstance(dy, torch.Tensor) and dy.shape == x.shape and dy.device == x.device, ValueError,
              "dy must match x in shape and device")
@@ -370,13 +470,13 @@ def rmsnorm_rope_heads_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch
     rows = xm.numel() // d
     dx = torch.empty_like(xm)
     if rows == 0:
-        return (dx if perm is None else dx.permute(_inverse(perm))), torch.zeros(d, dtype=torch.float32, device=xm.device)
-    dweight = torch.empty(d, dtype=torch.float32, device=xm.device)
+        return (dx if perm is None else dx.permute(_inverse(perm))), torch.zeros(d, dtype=dtype, device=xm.device)
+    dweight = torch.empty(d, dtype=dtype, device=xm.device)
     with torch.cuda.device(xm.device):
         ws = _workspace(cabi.load().tt_rmsnorm_backward_workspace_bytes(rows, d), 0, xm)
-        cabi.call("tt_rmsnorm_rope_heads_backward", dx.data_ptr(), dweight.data_ptr(), dym.data_ptr(), xm.data_ptr(),
-                  weight.data_ptr(), freqs.data_ptr(), ws.data_ptr(), ws.numel(), rows, d, heads, seq,
-                  float(eps), _stream(xm))
+        cabi.call("tt_rmsnorm_backward_typed", dx.data_ptr(), dweight.data_ptr(), int(dtype == BF16), dym.data_ptr(),
+                  xm.data_ptr(), weight.data_ptr(), freqs.data_ptr(), d, heads, seq, ws.data_ptr(), ws.numel(),
+                  rows, d, float(eps), _stream(xm))
     return (dx if perm is None else dx.permute(_inverse(perm))), dweight
 
 
@@ -425,13 +525,52 @@ def residual_norm_forward(x: torch.Tensor, residual: torch.Tensor, gate: Optiona
     return s, y
 
 
+def residual_norm_forward_saving(x: torch.Tensor, residual: torch.Tensor, gate: Optional[torch.Tensor],
+                                 scale: torch.Tensor, shift: torch.Tensor, eps: float, affine: bool, save: bool):
+    """``(s, y, gate, scale)``: ``residual_norm_forward`` and its gate and scale as dense bf16; as
+    ``adaln_forward_saving``."""
+    cols = x.shape[-1]
+    params = [p for p in (gate, scale, shift) if p is not None]
+    if all(p.is_contiguous() for p in params):
+        gate, scale = None if gate is None else gate.to(BF16), scale.to(BF16)
+        return (*residual_norm_forward(x, residual, gate, scale, shift, eps, affine), gate, scale)
+    strides = [_vectors(p, cols) for p in params]
+    if (any(st is None for st in strides) or shift.shape != scale.shape
+            or any(p.shape[-1] != cols or p.device != x.device for p in params)):
+        gate = None if gate is None else gate.to(BF16).contiguous()
+        scale = scale.to(BF16).contiguous()
+        return (*residual_norm_forward(x, residual, gate, scale, shift, eps, affine), gate, scale)
+    x = _check_act("x", x, cols)
+    residual = _check_act("residual", residual, cols)
+    _require(residual.numel() == x.numel() and residual.device == x.device, ValueError,
+             "residual must match x in size and device")
+    rows = x.numel() // cols
+    s, y = torch.empty_like(x), torch.empty_like(x)
+    dense = [p if p is None or not save or p.is_contiguous() else torch.empty(p.numel() // cols, cols, dtype=BF16, device=x.device)
+             for p in (gate, scale)]
+    if rows:
+        nb, rpb, n_gate, n_param = _res_batches(rows, cols, gate, scale)
+        with torch.cuda.device(x.device):
+            rc = cabi.load().tt_residual_norm_forward_strided(
+                s.data_ptr(), y.data_ptr(), x.data_ptr(), residual.data_ptr(),
+                _ptr(gate), n_gate, strides[0] if gate is not None else cols, _ptr(None if dense[0] is gate else dense[0]),
+                scale.data_ptr(), strides[-2], _ptr(None if dense[1] is scale else dense[1]), shift.data_ptr(), strides[-1],
+                n_param, int(bool(affine)), None, None, rows, cols, rpb, float(eps), _stream(x))
+        if rc == cabi.TT_ERR_UNSUPPORTED:
+            gate = None if gate is None else gate.contiguous()
+            scale = scale.contiguous()
+            return (*residual_norm_forward(x, residual, gate, scale, shift, eps, affine), gate, scale)
+        cabi.check("tt_residual_norm_forward_strided", rc)
+    return s, y, dense[0], dense[1]
+
+
 def residual_norm_backward(dy: torch.Tensor, ds_in: Optional[torch.Tensor], s: torch.Tensor,
                            residual: Optional[torch.Tensor], gate: Optional[torch.Tensor], scale: torch.Tensor,
-                           eps: float, affine: bool = False):
+                           eps: float, affine: bool = False, dtype: torch.dtype = torch.float32):
     """Backward of ``residual_norm_forward`` from the saved ``s``.  ``ds_in`` is the gradient that
     reaches ``s`` from its other consumers (None = none).  Returns
     ``(dx, dresidual, dscale, dshift, dgate)``: dx / dresidual bf16 (the same tensor when there is
-    no gate), the parameter gradients fp32 ``[n_batches, C]`` (dgate None without a gate)."""
+    no gate), the parameter gradients ``[n_batches, C]`` in ``dtype``, fp32 or bf16 (dgate None without a gate)."""
     cols = s.shape[-1]
     s = _check_act("s", s, cols)
     dy = _check_act("dy", dy, cols)
@@ -448,16 +587,16 @@ def residual_norm_backward(dy: torch.Tensor, ds_in: Optional[torch.Tensor], s: t
     nb, rpb, n_gate, n_param = _res_batches(rows, cols, gate, scale) if rows else (max(scale.numel() // cols, 1), 0, 1, 1)
     dx = torch.empty_like(s)
     dr = torch.empty_like(s) if gate is not None else dx
-    f32 = dict(dtype=torch.float32, device=s.device)
+    like = dict(dtype=dtype, device=s.device)
     if rows == 0:
-        return dx, dr, torch.zeros(nb, cols, **f32), torch.zeros(nb, cols, **f32), \
-            (torch.zeros(nb, cols, **f32) if gate is not None else None)
-    dscale, dshift = torch.empty(nb, cols, **f32), torch.empty(nb, cols, **f32)
-    dgate = torch.empty(nb, cols, **f32) if gate is not None else None
+        return dx, dr, torch.zeros(nb, cols, **like), torch.zeros(nb, cols, **like), \
+            (torch.zeros(nb, cols, **like) if gate is not None else None)
+    dscale, dshift = torch.empty(nb, cols, **like), torch.empty(nb, cols, **like)
+    dgate = torch.empty(nb, cols, **like) if gate is not None else None
     with torch.cuda.device(s.device):
         ws = _workspace(cabi.load().tt_residual_norm_backward_workspace_bytes(rows, cols, rpb, int(gate is not None)), 0, s)
-        cabi.call("tt_residual_norm_backward", dx.data_ptr(), _ptr(dr if gate is not None else None),
-                  dscale.data_ptr(), dshift.data_ptr(), _ptr(dgate), dy.data_ptr(), _ptr(ds_in), s.data_ptr(),
+        cabi.call("tt_residual_norm_backward_typed", dx.data_ptr(), _ptr(dr if gate is not None else None),
+                  dscale.data_ptr(), dshift.data_ptr(), _ptr(dgate), int(dtype == BF16), dy.data_ptr(), _ptr(ds_in), s.data_ptr(),
                   _ptr(residual if gate is not None else None), _ptr(gate), n_gate, scale.data_ptr(), n_param,
                   int(bool(affine)), ws.data_ptr(), ws.numel(), rows, cols, rpb, float(eps), _stream(s))
     return dx, dr, dscale, dshift, dgate
