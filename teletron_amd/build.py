@@ -74,7 +74,7 @@ def build_library(force: bool = True, defines=(), jobs: int = 8, verbose: bool =
     return LIB_PATH
 
 
-TORCH_EXT_MODULES = ["fused_adaln", "fused_rmsnorm"]
+TORCH_EXT_MODULES = ["fused_adaln", "fused_rmsnorm", "native_ops"]
 
 
 def torch_ext_path(name: str) -> Path:
@@ -127,7 +127,7 @@ def build_torch_extensions(force: bool = True, verbose: bool = True):
         _run(cmd)
         return out
 
-    with ThreadPoolExecutor(max_workers=2) as pool:
+    with ThreadPoolExecutor(max_workers=3) as pool:
         return list(pool.map(compile_one, TORCH_EXT_MODULES))
 
 

@@ -32,6 +32,8 @@ def _check_row_groups(x, *params):
     A parameter with the input's rank is shaped for broadcasting, and must then mean the same thing
     ([B, 1, C] for x [B, S, C] does; [1, S, C] with B > 1 does not): refused rather than misread."""
     for p in params:
+        if p is not None and p.dim() == 3 == x.dim() and p.shape == (x.shape[0], 1, x.shape[2]):
+            continue
         if p is not None and x.dim() >= 3 and p.dim() == x.dim() and ops.row_groups(x, p) is None:
             raise ValueError(f"a parameter of shape {tuple(p.shape)} does not broadcast over consecutive groups of rows "
                              f"of an input of shape {tuple(x.shape)}")
@@ -46,7 +48,9 @@ def _adaln_forward(ctx, x, scale, shift, epsilon, cols):
     ctx.shift_meta = (shift.shape, shift.dtype)
     x = x.contiguous()
     save = any(ctx.needs_input_grad)
-    y, scale_c = ops.adaln_forward_saving(x, scale.detach(), shift.detach(), ctx.eps, save)
+    native = ops.native(x)
+    y, scale_c = (native and native.adaln_forward(x, scale, shift, ctx.eps, save)) or \
+        ops.adaln_forward_saving(x, scale.detach(), shift.detach(), ctx.eps, save)
     if save:
         ctx.save_for_backward(x, scale_c)
     return y
@@ -57,7 +61,15 @@ def _adaln_backward(ctx, grad_output, grad_reduce=None):
     (sc_shape, sc_dtype), (sh_shape, sh_dtype) = ctx.scale_meta, ctx.shift_meta
     # one rounding to the parameters' dtype in the kernel, unless an exchange in fp32 comes first
     dtype = ops._grad_dtype(sc_dtype) if grad_reduce is None and sc_dtype == sh_dtype else torch.float32
-    dx, grads = ops.adaln_backward_packed(grad_output.contiguous(), x, scale_c, ctx.eps, dtype)
+    grad_output = grad_output.contiguous()
+    native = ops.native(x)
+    if native and grad_reduce is None and sc_dtype == sh_dtype:
+        done = native.adaln_backward(grad_output, x, scale_c, ctx.eps, dtype == torch.bfloat16, sc_shape, sh_shape)
+        if done:
+            dx, dscale, dshift = done
+            need = ctx.needs_input_grad
+            return dx if need[0] else None, dscale.to(sc_dtype) if need[1] else None, dshift.to(sh_dtype) if need[2] else None
+    dx, grads = ops.adaln_backward_packed(grad_output, x, scale_c, ctx.eps, dtype)
     if grad_reduce is not None:
         grad_reduce(grads)                  # fp32 [2, n_batches, C]: dscale and dshift in ONE exchange, before the cast
     if sc_dtype == sh_dtype:
@@ -97,6 +109,12 @@ class AdaLNGradReduceFunction(Function):
         return (*_adaln_backward(ctx, grad_output, ctx.grad_reduce), None, None, None)
 
 
+def _rmsnorm_backward(grad_output, x, weight, freqs, eps, head_dim, heads, w_shape, w_dtype):
+    native = ops.native(x)
+    return native and native.rmsnorm_backward(grad_output, x, weight, freqs, eps, head_dim, heads,
+                                              w_dtype == torch.bfloat16, w_shape)
+
+
 class RMSNormModelFunction(Function):
     @staticmethod
     def forward(ctx, x, weight, epsilon, cols):
@@ -107,7 +125,9 @@ class RMSNormModelFunction(Function):
         if ops.memory_order_view(x)[0] is None:      # dense permuted views are handled without a copy
             x = x.contiguous()
         save = any(ctx.needs_input_grad)
-        y, weight_c = ops.rmsnorm_forward_saving(x, weight.detach(), ctx.eps, save)
+        native = ops.native(x)               # (not for permuted views: it takes dense ones)
+        y, weight_c = (native and native.rmsnorm_forward(x, weight, ctx.eps, save)) or \
+            ops.rmsnorm_forward_saving(x, weight.detach(), ctx.eps, save)
         if save:
             ctx.save_for_backward(x, weight_c)
         return y
@@ -118,7 +138,8 @@ class RMSNormModelFunction(Function):
         if x.is_contiguous():
             grad_output = grad_output.contiguous()
         w_shape, w_dtype = ctx.weight_meta
-        dx, dweight = ops.rmsnorm_backward(grad_output, x, weight_c, ctx.eps, ops._grad_dtype(w_dtype))
+        dx, dweight = _rmsnorm_backward(grad_output, x, weight_c, None, ctx.eps, 0, 0, w_shape, w_dtype) or \
+            ops.rmsnorm_backward(grad_output, x, weight_c, ctx.eps, ops._grad_dtype(w_dtype))
         dx = dx if ctx.needs_input_grad[0] else None
         dweight = dweight.to(w_dtype).reshape(w_shape) if ctx.needs_input_grad[1] else None
         return dx, dweight, None, None
@@ -140,14 +161,17 @@ class RMSNormRopeFunction(Function):
         weight_c = weight.detach().to(torch.bfloat16).contiguous()
         freqs_c = ops._check_freqs(freqs.detach(), x, ctx.head_dim)
         ctx.save_for_backward(x, weight_c, freqs_c)
-        return ops.rmsnorm_rope_forward(x, weight_c, freqs_c, ctx.eps, ctx.head_dim)
+        native = ops.native(x)
+        y = native.rope_forward(x, weight_c, freqs_c, ctx.eps, ctx.head_dim, 0) if native else None
+        return ops.rmsnorm_rope_forward(x, weight_c, freqs_c, ctx.eps, ctx.head_dim) if y is None else y
 
     @staticmethod
     def backward(ctx, grad_output):
         x, weight_c, freqs_c = ctx.saved_tensors
         w_shape, w_dtype = ctx.weight_meta
-        dx, dweight = ops.rmsnorm_rope_backward(grad_output.contiguous(), x, weight_c, freqs_c, ctx.eps, ctx.head_dim,
-                                                ops._grad_dtype(w_dtype))
+        grad_output = grad_output.contiguous()
+        dx, dweight = _rmsnorm_backward(grad_output, x, weight_c, freqs_c, ctx.eps, ctx.head_dim, 0, w_shape, w_dtype) or \
+            ops.rmsnorm_rope_backward(grad_output, x, weight_c, freqs_c, ctx.eps, ctx.head_dim, ops._grad_dtype(w_dtype))
         return (dx if ctx.needs_input_grad[0] else None,
                 dweight.to(w_dtype).reshape(w_shape) if ctx.needs_input_grad[1] else None, None, None, None)
 
@@ -195,7 +219,10 @@ def _gate_forward(ctx, x, gate, residual):
     ctx.gate_meta = (gate.shape, gate.dtype)
     residual = residual.contiguous()
     save = any(ctx.needs_input_grad)
-    out, gate_c = ops.gate_residual_forward_saving(x.contiguous(), gate.detach(), residual, save)
+    x = x.contiguous()
+    native = ops.native(x)
+    out, gate_c = (native and native.gate_forward(x, gate, residual, save)) or \
+        ops.gate_residual_forward_saving(x, gate.detach(), residual, save)
     if save:
         ctx.save_for_backward(gate_c, residual)
     return out
@@ -206,8 +233,12 @@ def _gate_backward(ctx, grad_output, grad_reduce=None):
     g_shape, g_dtype = ctx.gate_meta
     if not (ctx.needs_input_grad[1] or ctx.needs_input_grad[2]):
         return grad_output, None, None
-    dres, dgate = ops.gate_residual_backward(grad_output.contiguous(), gate_c, residual,
-                                             ops._grad_dtype(g_dtype) if grad_reduce is None else torch.float32)
+    dtype = ops._grad_dtype(g_dtype) if grad_reduce is None else torch.float32
+    dout = grad_output.contiguous()
+    native = ops.native(dout)
+    vectors = (gate_c.numel() // gate_c.shape[-1], gate_c.shape[-1])
+    dres, dgate = (native and native.gate_backward(dout, gate_c, residual, dtype == torch.bfloat16, vectors)) or \
+        ops.gate_residual_backward(dout, gate_c, residual, dtype)
     if grad_reduce is not None and ctx.needs_input_grad[1]:
         grad_reduce(dgate)                  # fp32 [n_batches, C], before the cast
     return (grad_output if ctx.needs_input_grad[0] else None,
@@ -263,9 +294,12 @@ class ResidualNormFunction(Function):
         ctx.metas = [None if t is None else (t.shape, t.dtype) for t in (gate, scale, shift)]
         save = any(ctx.needs_input_grad)
         residual = residual.contiguous()
-        s, y, gate_c, scale_c = ops.residual_norm_forward_saving(
-            x.contiguous(), residual, None if gate is None else gate.detach(), scale.detach(), shift.detach(),
-            ctx.eps, ctx.affine, save)
+        x = x.contiguous()
+        native = ops.native(x)
+        s, y, gate_c, scale_c = \
+            (native and native.residual_norm_forward(x, residual, gate, scale, shift, ctx.eps, ctx.affine, save)) or \
+            ops.residual_norm_forward_saving(x, residual, None if gate is None else gate.detach(), scale.detach(),
+                                             shift.detach(), ctx.eps, ctx.affine, save)
         if save:
             ctx.save_for_backward(s, residual if gate is not None else None, gate_c, scale_c)
         return s, y
@@ -279,9 +313,12 @@ class ResidualNormFunction(Function):
         n = max(c.numel() for c in (gate_c, scale_c) if c is not None)
         direct = ctx.grad_reduce is None and all(
             m is None or (m[1] == torch.bfloat16 and m[0].numel() == n) for m in ctx.metas)
-        dx, dr, dscale, dshift, dgate = ops.residual_norm_backward(
-            grad_y.contiguous(), None if grad_s is None else grad_s.contiguous(), s, residual, gate_c, scale_c,
-            ctx.eps, ctx.affine, torch.bfloat16 if direct else torch.float32)
+        grad_y, grad_s = grad_y.contiguous(), None if grad_s is None else grad_s.contiguous()
+        native = ops.native(s)
+        dx, dr, dscale, dshift, dgate = \
+            (native and native.residual_norm_backward(grad_y, grad_s, s, residual, gate_c, scale_c, ctx.eps, ctx.affine, direct)) or \
+            ops.residual_norm_backward(grad_y, grad_s, s, residual, gate_c, scale_c, ctx.eps, ctx.affine,
+                                       torch.bfloat16 if direct else torch.float32)
         if ctx.grad_reduce is not None:
             parts = [g for g in ((dgate,) if ctx.affine else (dscale, dshift, dgate)) if g is not None]
             if parts:

@@ -20,6 +20,22 @@ from . import cabi
 BF16 = torch.bfloat16
 
 
+_native = None
+
+
+def native(x: torch.Tensor):
+    """The module that makes an operator one native call (csrc/torch_ext/native_ops.cpp) if ``x`` is an ordinary
+    GPU tensor, else None.  Its functions return None for arguments they do not cover: the functions below
+    then take the call."""
+    global _native
+    if type(x) not in (torch.Tensor, torch.nn.Parameter) or not x.is_cuda:
+        return None
+    if _native is None:
+        from . import native_ops      # built by `python -m teletron_amd.build`
+        _native = native_ops
+    return _native
+
+
 def _require(cond: bool, exc, msg: str):
     if not cond:
         raise exc(msg)
@@ -180,6 +196,8 @@ def clear_workspaces() -> None:
     until they finish (the caching allocator frees in stream order)."""
     with _WORKSPACES_LOCK:
         _WORKSPACES.clear()
+    if _native is not None:
+        _native.clear_workspaces()
 
 
 def _workspace(lib_bytes: int, rows: int, *tensors: torch.Tensor) -> torch.Tensor:
@@ -451,6 +469,10 @@ def rmsnorm_rope_heads_forward(x: torch.Tensor, weight: torch.Tensor, freqs: tor
     result has the input's shape and strides).  freqs: [S, D/2, 2] (cos, sin) or complex [S, 1, D/2]."""
     xm, perm, weight, freqs, heads, d, seq = _heads_layout(x, weight, freqs)
     rows = xm.numel() // d
+    n = native(xm)
+    y = n.rope_forward(xm, weight, freqs, eps, d, heads) if n else None
+    if y is not None:
+        return y if perm is None else y.permute(_inverse(perm))
     y = torch.empty_like(xm)
     if rows:
         with torch.cuda.device(xm.device):
@@ -468,6 +490,10 @@ def rmsnorm_rope_heads_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch
     dym = dy if perm is None else dy.permute(perm)
     dym = _check_act("dy", dym, d)          # contiguous copy only if dy is not laid out like x
     rows = xm.numel() // d
+    n = native(xm)
+    done = n and n.rmsnorm_backward(dym, xm, weight, freqs, eps, d, heads, dtype == BF16, (d,))
+    if done:
+        return (done[0] if perm is None else done[0].permute(_inverse(perm))), done[1]
     dx = torch.empty_like(xm)
     if rows == 0:
         return (dx if perm is None else dx.permute(_inverse(perm))), torch.zeros(d, dtype=dtype, device=xm.device)

@@ -85,3 +85,33 @@ def test_bf16_gradients_are_the_fp32_ones_rounded(op):
         w, args, fn = rand_bf16(d, seed=3).to(DEV), (1e-6,), ops.rmsnorm_rope_heads_backward
     (dx, g), (dx16, g16) = fn(dy, x, w, table, *args), fn(dy, x, w, table, *args, dtype=torch.bfloat16)
     assert torch.equal(dx, dx16) and g.dtype == torch.float32 and torch.equal(g.to(torch.bfloat16), g16)
+
+
+@pytest.mark.parametrize("cols", [7, 100, 128, 1000, 1001, 1536])
+def test_native_calls_equal_the_python_ones(cols, monkeypatch):
+    """ops.native() covers the ordinary calls; what it declines, and other tensor classes, take ops.py."""
+    from teletron_amd import functional as T, ops
+
+    class Tagged(torch.Tensor):
+        pass
+
+    x, r = (rand_bf16(2, 29, cols, seed=i).to(DEV).requires_grad_(True) for i in range(2))
+    assert ops.native(x) is not None and ops.native(x.detach().as_subclass(Tagged)) is None and ops.native(x.cpu()) is None
+    assert ops.native(x).adaln_forward(x.float(), x[:, :1], x[:, :1], 1e-6, False) is None
+    p = [t.detach().requires_grad_(True) for t in modulation(2, cols, "chunks")]
+    w = p[0].detach()[0, 0].clone().requires_grad_(True)
+    calls = [(lambda: T.adaln_modulate(x, p[0], p[1]), [x, p[0], p[1]]), (lambda: T.rms_norm(x, w), [x, w])]
+    if cols % 8 == 0:
+        calls.append((lambda: T.gate_residual(x, p[2], r), [x, p[2], r]))
+        table = torch.randn(29, cols // 2, 2, device=DEV)
+        heads = x.detach().reshape(2, 29, 1, cols).expand(2, 29, 3, cols).contiguous().requires_grad_(True)
+        if cols <= 256:
+            calls.append((lambda: T.RMSNormRopeHeadsFunction.apply(heads.transpose(1, 2), w, table, 1e-6), [heads, w]))
+    if cols == 1536:
+        calls += [(lambda: T.residual_adaln(x, r, p[2], p[0], p[1]), [x, r, *p]),
+                  (lambda: T.RMSNormRopeFunction.apply(x, w, table[:, :64].contiguous(), 1e-6, 12), [x, w])]
+    native = [grads(call(), inputs, 3) for call, inputs in calls]
+    monkeypatch.setattr(ops, "native", lambda x: None)
+    for (call, inputs), got in zip(calls, native):
+        for a, b in zip(got, grads(call(), inputs, 3)):
+            assert torch.equal(a, b)
