@@ -120,10 +120,12 @@ constexpr int kGateKind = 2;   // third op family next to kAdaLN / kRMS
 // Upper bound on workgroups per batch used by any plan: what the workspace is sized for.
 constexpr int kMaxWgsPerCu = 8;
 
-// `odd`: rows of any length and 2-byte aligned tensors (wide norm_fwd / norm_bwd kernels only).
+// `force`: kOdd for rows of any length and 2-byte aligned tensors (wide norm_fwd / norm_bwd kernels only),
+// kMasked for the plan that ragged rows would have on the kernels of whole-line rows.
 // `res`: 0, or the residual + LayerNorm fusion: 1 plain, 2 gated (wide rows, kFwd / kBwd only).
 int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_batch, Plan* plan, bool rope = false,
-              int res = 0, int64_t rope_heads = 0, bool odd = false) {
+              int res = 0, int64_t rope_heads = 0, int force = -1) {
+  const bool odd = force == kOdd;
   if (rows <= 0 || cols <= 0 || rows_per_batch <= 0 || rows % rows_per_batch != 0)
     return TT_ERR_INVALID_ARGUMENT;
   if (cols > TT_MAX_COLS) return TT_ERR_UNSUPPORTED;
@@ -136,7 +138,7 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   const int slots = narrow ? kNarrowL[idx] : 64 * kWideW[idx] * kWideP[idx];
   const bool full = (slots == packs);
   // a row of whole 128-byte lines or not: see enum Rows
-  const int mode = odd ? kOdd : full ? kFull : (cols * 2) % 128 == 0 ? kMasked : kRagged;
+  const int mode = odd ? kOdd : full ? kFull : (cols * 2) % 128 == 0 || force == kMasked ? kMasked : kRagged;
   KernelInfo k;
   if (res) {
     if (narrow || kind != kAdaLN || dir == kBwdSaved || dir == kFwdXn) return TT_ERR_UNSUPPORTED;
@@ -209,7 +211,7 @@ size_t partial_bytes(const Plan& p, int n_acc, int64_t cols) {
 // these: RMSNorm 5000 x 1001 12.6 / 117 -> 9.4 / 16, AdaLN 8000 x 1999 33 / 125 -> 17 / 29, 60000 x 1537
 // 283 / 2122 -> 79 / 133 (1544 columns, 16-byte aligned rows: 67 / 109).
 bool odd_plan(int kind, int64_t rows, int64_t cols, int64_t rows_per_batch, Plan* p) {
-  if (make_plan(kind, kBwd, rows, cols, rows_per_batch, p, false, 0, 0, true) != TT_OK) return false;
+  if (make_plan(kind, kBwd, rows, cols, rows_per_batch, p, false, 0, 0, kOdd) != TT_OK) return false;
   const size_t tensors = (size_t)rows * cols * 4;
   const size_t most = tensors > TT_STATIC_WORKSPACE_BYTES ? tensors : (size_t)TT_STATIC_WORKSPACE_BYTES;
   return partial_bytes(*p, kind == kAdaLN ? 2 : 1, cols) <= most;
@@ -301,7 +303,7 @@ int forward_generic(int kind, void* y, const void* x, const void* p0, const void
   if (!aligned2(y) || !aligned2(x) || !aligned2(p0) || !aligned2(p1) || !aligned2(x_norm)) return TT_ERR_INVALID_ARGUMENT;
   if (params && (!aligned2(params->copy) || (params->f32 && !aligned4(p0)))) return TT_ERR_INVALID_ARGUMENT;
   Plan p;
-  if (make_plan(kind, x_norm ? kFwdXn : kFwd, rows, cols, rows_per_batch, &p, false, 0, 0, true) == TT_OK) {
+  if (make_plan(kind, x_norm ? kFwdXn : kFwd, rows, cols, rows_per_batch, &p, false, 0, 0, kOdd) == TT_OK) {
     FwdArgs f = {};
     f.p0_stride = params ? params->stride0 : cols; f.p1_stride = params ? params->stride1 : cols;
     f.p0_f32 = params ? params->f32 : 0; f.p0_copy = params ? params->copy : nullptr;
@@ -437,6 +439,14 @@ int backward_partials(int kind, void* dx, const void* dy, const void* x, const v
   int rc = make_plan(kind, kBwd, rows, cols, rows_per_batch, &p, rope != nullptr, 0, rope ? rope->heads : 0);
   if (rc != TT_OK) return rc;
   const int n_acc = kind == kAdaLN ? 2 : 1;
+  if (!rope && workspace_bytes < partial_bytes(p, n_acc, cols)) {
+    // The kernels of ragged rows keep more workgroups resident, hence more partial sums, than those of
+    // whole-line rows.  A workspace (the scratch array above all) that would do for the latter gets their grid.
+    Plan pm;
+    if (make_plan(kind, kBwd, rows, cols, rows_per_batch, &pm, false, 0, 0, kMasked) == TT_OK &&
+        pm.grid_x < p.grid_x && workspace_bytes >= partial_bytes(pm, n_acc, cols))
+      p.grid_x = pm.grid_x;
+  }
   if (!workspace || !aligned16(workspace) || workspace_bytes < partial_bytes(p, n_acc, cols)) return TT_ERR_WORKSPACE;
   BwdArgs a;
   a.freqs = rope ? rope->freqs : nullptr; a.seq_len = rope ? rope->seq_len : 1; a.head_dim = rope ? (int)rope->head_dim : 8;
