@@ -231,25 +231,44 @@ KernelInfo info_bwd_rope_narrow() {
   constexpr int R = kNarrowR, NW = kNarrowNW;
   return {reinterpret_cast<const void*>(&norm_bwd_narrow<kRMS, L, R, NW, FULL, true>), 64 * NW, NW * R * (64 / L), R};
 }
-// Token mode of the narrow ROPE kernels (ROPE = 2: the rows a wave takes per tile are the heads of
-// one token, so the (cos, sin) entries are loaded once per tile and lane).  Instantiated for rows of
-// 16 lanes (head_dim 72 ... 128) and 24 heads per token, HunyuanVideo's layout: 24 rows / 4 rows per
-// load = 6 loads per lane.
-constexpr int kRopeTokenL = 16, kRopeTokenR = 6, kRopeTokenHeads = kRopeTokenR * (64 / kRopeTokenL);
-// Four waves in one workgroup per CU (24 loads per lane column and tensor in flight) measured best:
-// forward 245 us, backward + reduction 356 us at 118800 x 24 x 128; 5 / 6 / 8 waves: 277 / 265 / 267 us
-// forward, 378 / 368 / 380 us backward; 2 and 3 waves need 2-3 workgroups per CU and reach 259-265 us.
-constexpr int kRopeTokenNW = 4;
-template <bool FULL>
+// Token mode of the narrow ROPE kernels (ROPE = 2: the rows a wave takes per tile are heads of one
+// token, so the (cos, sin) entries are loaded once per tile and lane).  R loads of 64 / L rows each have to
+// divide a token's heads: instantiated for rows of 8 and 16 lanes (head_dim 40 ... 128), the largest of
+// R = 6, 4, 3 that divides (24 heads of 128: 6, 16: 4, 12: 3; 24 heads of 64: 3).  Other head counts
+// look every row up (ROPE = 1, two loads).  us forward / backward + reduction, per row -> per token:
+// 2 x 60000 x 12 x 128 137 / 190 -> 127 / 184, 60000 x 16 x 128 92 / 128 -> 89 / 127, 2 x 60000 x 24 x 64
+// 133 / 189 -> 127 / 183.  R = 5 is slower (60000 x 40 x 128 221 / 318 -> 227 / 321).
+// One workgroup per CU with about 24 loads per lane column and tensor in flight measured best (24
+// heads of 128, four waves of six: forward 245 us, backward + reduction 356 us at 118800 tokens; 5 / 6 / 8
+// waves: 277 / 265 / 267 us forward, 378 / 368 / 380 us backward; 2 and 3 waves need 2-3 workgroups per
+// CU and reach 259-265 us).
+constexpr int kRopeTokenMinL = 8, kRopeTokenMaxL = 16, kRopeTokenHeads = 24;   // 24 x 128: HunyuanVideo, at every size
+constexpr int rope_token_NW(int R) { return (24 + R / 2) / R; }
+template <int L, int R, bool FULL>
 KernelInfo info_rope_token(bool backward) {
-  constexpr int L = kRopeTokenL, R = kRopeTokenR, NF = kRopeTokenNW, NB = kRopeTokenNW;
+  constexpr int NW = rope_token_NW(R);
   if (backward)
-    return {reinterpret_cast<const void*>(&norm_bwd_narrow<kRMS, L, R, NB, FULL, 2>), 64 * NB, NB * R * (64 / L), R};
-  return {reinterpret_cast<const void*>(&norm_fwd_narrow<kRMS, L, R, NF, FULL, 2>), 64 * NF, NF * R * (64 / L), R};
+    return {reinterpret_cast<const void*>(&norm_bwd_narrow<kRMS, L, R, NW, FULL, 2>), 64 * NW, NW * R * (64 / L), R};
+  return {reinterpret_cast<const void*>(&norm_fwd_narrow<kRMS, L, R, NW, FULL, 2>), 64 * NW, NW * R * (64 / L), R};
+}
+// Loads per wave and tile in token mode, or 0 where `heads` rows per token do not allow it.
+inline int rope_token_R(int L, int64_t heads) {
+  if (L < kRopeTokenMinL || L > kRopeTokenMaxL || heads <= 0) return 0;
+  for (int r : {6, 4, 3})
+    if (heads % (r * (64 / L)) == 0) return r;
+  return 0;
+}
+template <int L, bool FULL>
+KernelInfo lookup_rope_token(int R, bool backward) {
+  return R == 6   ? info_rope_token<L, 6, FULL>(backward)
+         : R == 4 ? info_rope_token<L, 4, FULL>(backward)
+                  : info_rope_token<L, 3, FULL>(backward);
 }
 inline KernelInfo lookup_rope(bool narrow, bool backward, int idx, bool full, int64_t heads) {
-  if (narrow && kNarrowL[idx] == kRopeTokenL && heads == kRopeTokenHeads)
-    return full ? info_rope_token<true>(backward) : info_rope_token<false>(backward);
+  if (const int r = narrow ? rope_token_R(kNarrowL[idx], heads) : 0) {
+    if (kNarrowL[idx] == 16) return full ? lookup_rope_token<16, true>(r, backward) : lookup_rope_token<16, false>(r, backward);
+    return full ? lookup_rope_token<8, true>(r, backward) : lookup_rope_token<8, false>(r, backward);
+  }
   if (narrow) {
     switch (idx) {
 #define X(i, L)                                                                                       \

@@ -610,7 +610,7 @@ struct RowPos {
 // L lanes per row (one pack each), 64/L rows per wave per load, R loads in flight,
 // NW independent waves per workgroup.  A tile is NW*R*(64/L) consecutive rows.
 // ROPE: 0 none; 1 every row looks up its own position; 2 the R * 64/L rows a wave takes per tile
-// are exactly the heads of ONE token (the caller guarantees rows_per_pos == R * 64/L), so a lane
+// are heads of ONE token (the caller guarantees that R * 64/L divides rows_per_pos), so a lane
 // loads its (cos, sin) entries once per tile instead of once per row.
 template <int KIND, int L, int R, int NW, bool FULL, int ROPE = 0, bool XN = false>   // XN as in norm_fwd_wide
 __global__ __launch_bounds__(64 * NW) void norm_fwd_narrow(const FwdArgs a) {
