@@ -207,6 +207,8 @@ size_t partial_bytes(const Plan& p, int n_acc, int64_t cols) {
   return (size_t)p.n_batches * p.grid_x * n_acc * cols * sizeof(float);
 }
 
+size_t workspace_for(int kind, int n_acc, int64_t rows, int64_t cols, int64_t rows_per_batch);
+
 // Backward of rows that the 128-bit kernels do not take (cols % 8 != 0, or tensors that are only 2-byte
 // aligned).  Rows of more than 256 values take the kOdd kernels, which leave partial column sums like
 // all others, as long as those stay small: at most the size of the scratch array or of x and dy.  Beyond
@@ -214,11 +216,22 @@ size_t partial_bytes(const Plan& p, int n_acc, int64_t cols) {
 // keep two floats a row (their column sums have cols / 64 workgroups).  us forward / backward, element-wise ->
 // these: RMSNorm 5000 x 1001 12.6 / 117 -> 9.4 / 16, AdaLN 8000 x 1999 33 / 125 -> 17 / 29, 60000 x 1537
 // 283 / 2122 -> 79 / 133 (1544 columns, 16-byte aligned rows: 67 / 109).
+// Where cols % 8 == 0 the size query does not know of the misaligned tensor and answers for the aligned
+// kernels, which may want less (two rows a tile: half the workgroups).  The grid is then what the answer
+// holds, so that which kernels run, and the order of their sums, depends on the shape and not on what else
+// the workspace has room for.
 bool odd_plan(int kind, int64_t rows, int64_t cols, int64_t rows_per_batch, Plan* p) {
   if (make_plan(kind, kBwd, rows, cols, rows_per_batch, p, false, 0, 0, kOdd) != TT_OK) return false;
+  const int n_acc = kind == kAdaLN ? 2 : 1;
+  if (cols % kPack == 0) {
+    const size_t per_wg = partial_bytes(*p, n_acc, cols) / p->grid_x;   // one workgroup of every batch
+    const size_t fit = workspace_for(kind, n_acc, rows, cols, rows_per_batch) / per_wg;
+    if (fit < 1) return false;
+    if (fit < (size_t)p->grid_x) p->grid_x = (int)fit;
+  }
   const size_t tensors = (size_t)rows * cols * 4;
   const size_t most = tensors > TT_STATIC_WORKSPACE_BYTES ? tensors : (size_t)TT_STATIC_WORKSPACE_BYTES;
-  return partial_bytes(*p, kind == kAdaLN ? 2 : 1, cols) <= most;
+  return partial_bytes(*p, n_acc, cols) <= most;
 }
 
 // Workspace bound that does not depend on the launch-time occupancy query.

@@ -1,0 +1,50 @@
+"""Rows of any length and tensors at any 2-byte address: which kernels a call runs on, and that this and
+every bit of the result depend on its arguments alone.  Tolerances as in test_gpu_parity.py."""
+import pytest
+import torch
+
+from test_gpu_parity import DEV, rand_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+def shifted(t, by):
+    """The values of ``t`` in a buffer of their own, ``by`` values behind a 16-byte boundary."""
+    buf = torch.empty(t.numel() + by, dtype=t.dtype, device=DEV)
+    buf[by:] = t.flatten().to(DEV)
+    return buf[by:].view(t.shape)
+
+
+# shapes whose aligned AdaLN kernel takes two rows a tile and so asks for fewer partial sums, and one that does not
+@pytest.mark.parametrize("nb,rpb,cols", [(2, 512, 1536), (1, 2500, 1536), (3, 700, 1000), (1, 1500, 3072), (1, 900, 5120)])
+def test_misaligned_backward_does_not_depend_on_earlier_calls(lib, nb, rpb, cols):
+    from teletron_amd import ops
+    rows = nb * rpb
+    x, dy = (shifted(rand_bf16(rows, cols, seed=i), 3) for i in range(2))
+    w = shifted(rand_bf16(nb, cols, seed=2, scale=0.2), 5)
+    calls = [lambda: ops.adaln_backward(dy, x, w, 1e-6), lambda: ops.rmsnorm_backward(dy, x, w[0], 1e-6)]
+    ops.clear_workspaces()
+    first = [call() for call in calls]
+    big = rand_bf16(8000, 8192, seed=3).to(DEV)
+    ops.adaln_backward(big, big, big[0], 1e-6)              # leaves a workspace with room to spare
+    for call, want in zip(calls, first):
+        for a, b in zip(call(), want):
+            assert torch.equal(a, b)
+
+    # the workspace that the queries ask for holds the partial sums of the vector kernels: they are
+    # written behind the two floats a row that the element-wise kernels keep
+    st = torch.cuda.current_stream().cuda_stream
+    dx, g = torch.empty_like(x), torch.empty(2, nb, cols, device=DEV)
+    for name, need in (("adaln", lib.tt_adaln_backward_workspace_bytes(rows, cols, rpb)),
+                       ("rms", lib.tt_rmsnorm_backward_workspace_bytes(rows, cols))):
+        assert need > 2 * rows * 8
+        ws = torch.full((need // 4,), 1e30, device=DEV)
+        if name == "adaln":
+            rc = lib.tt_adaln_backward(dx.data_ptr(), g[0].data_ptr(), g[1].data_ptr(), dy.data_ptr(), x.data_ptr(),
+                                       w.data_ptr(), ws.data_ptr(), need, rows, cols, rpb, 1e-6, st)
+        else:
+            rc = lib.tt_rmsnorm_backward(dx.data_ptr(), g[0].data_ptr(), dy.data_ptr(), x.data_ptr(), w.data_ptr(),
+                                         ws.data_ptr(), need, rows, cols, 1e-6, st)
+        assert rc == 0
+        torch.cuda.synchronize()
+        assert (ws[rows * 2:] != 1e30).any(), name
