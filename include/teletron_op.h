@@ -10,8 +10,9 @@
  * Fast path: cols % 8 == 0 and every tensor 16-byte aligned (128-bit vector kernels).
  * tt_adaln_forward/backward, tt_rmsnorm_forward/backward and the tt_launch_*_forward entry
  * points also accept any other cols <= TT_MAX_COLS and 2-byte aligned tensors: more than 256
- * columns run on vector kernels for any address, fewer on element-wise ones, several times slower; the two-step backward and the tt_launch_*_backward entry points
- * return TT_ERR_UNSUPPORTED there.
+ * columns run on vector kernels for any address, fewer (and the backward of more than 16384) on
+ * element-wise ones, several times slower; the two-step backward and the tt_launch_*_backward
+ * entry points return TT_ERR_UNSUPPORTED there.
  *
  * Two groups of entry points:
  *

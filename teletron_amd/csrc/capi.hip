@@ -215,13 +215,17 @@ size_t workspace_for(int kind, int n_acc, int64_t rows, int64_t cols, int64_t ro
 // that (a modulation vector for every few rows), and for shorter rows, the element-wise kernels run, which
 // keep two floats a row (their column sums have cols / 64 workgroups).  us forward / backward, element-wise ->
 // these: RMSNorm 5000 x 1001 12.6 / 117 -> 9.4 / 16, AdaLN 8000 x 1999 33 / 125 -> 17 / 29, 60000 x 1537
-// 283 / 2122 -> 79 / 133 (1544 columns, 16-byte aligned rows: 67 / 109).
+// 283 / 2122 -> 79 / 133 (1544 columns, 16-byte aligned rows: 67 / 109).  Rows of more than 16384 values stay
+// element-wise: their wide kernel (16 waves of four packs a lane) spills its column sums and is the slower one,
+// AdaLN / RMSNorm 10485 x 20001 1080 / 904 -> 2256 / 1738, 2047 x 16391 128 / 103 -> 453 / 337, against
+// 12800 x 16383 1085 / 919 -> 907 / 420.
 // Where cols % 8 == 0 the size query does not know of the misaligned tensor and answers for the aligned
 // kernels, which may want less (two rows a tile: half the workgroups).  The grid is then what the answer
 // holds, so that which kernels run, and the order of their sums, depends on the shape and not on what else
 // the workspace has room for.
+constexpr int64_t kOddBwdMaxCols = 16384;
 bool odd_plan(int kind, int64_t rows, int64_t cols, int64_t rows_per_batch, Plan* p) {
-  if (make_plan(kind, kBwd, rows, cols, rows_per_batch, p, false, 0, 0, kOdd) != TT_OK) return false;
+  if (cols > kOddBwdMaxCols || make_plan(kind, kBwd, rows, cols, rows_per_batch, p, false, 0, 0, kOdd) != TT_OK) return false;
   const int n_acc = kind == kAdaLN ? 2 : 1;
   if (cols % kPack == 0) {
     const size_t per_wg = partial_bytes(*p, n_acc, cols) / p->grid_x;   // one workgroup of every batch

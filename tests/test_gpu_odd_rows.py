@@ -48,3 +48,25 @@ def test_misaligned_backward_does_not_depend_on_earlier_calls(lib, nb, rpb, cols
         assert rc == 0
         torch.cuda.synchronize()
         assert (ws[rows * 2:] != 1e30).any(), name
+
+
+@pytest.mark.parametrize("cols", [250, 257, 1001, 16383, 16385, 32767])
+def test_odd_widths_run_on_the_faster_kernels(lib, cols):
+    """The vector kernels leave partial sums in the workspace, the element-wise ones two floats a row."""
+    rows, st = 700, torch.cuda.current_stream().cuda_stream
+    x, dy = (rand_bf16(rows, cols, seed=i).to(DEV) for i in range(2))
+    w = rand_bf16(cols, seed=2, scale=0.2).to(DEV)
+    vector = 256 < cols <= 16384
+    dx, g = torch.empty_like(x), torch.empty(2, cols, device=DEV)
+    for adaln, need in ((True, lib.tt_adaln_backward_workspace_bytes(rows, cols, rows)),
+                        (False, lib.tt_rmsnorm_backward_workspace_bytes(rows, cols))):
+        assert (need > rows * 8) == vector
+        ws = torch.full((1 << 24,), 1e30, device=DEV)
+        args = [dy.data_ptr(), x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel() * 4, rows, cols]
+        if adaln:
+            assert lib.tt_adaln_backward(dx.data_ptr(), g[0].data_ptr(), g[1].data_ptr(), *args, rows, 1e-6, st) == 0
+        else:
+            assert lib.tt_rmsnorm_backward(dx.data_ptr(), g[0].data_ptr(), *args, 1e-6, st) == 0
+        torch.cuda.synchronize()
+        assert (ws[:rows * 2] != 1e30).all() and (ws[rows * 2:need // 4] != 1e30).any() == vector
+        assert (ws[need // 4:] == 1e30).all()
