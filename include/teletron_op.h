@@ -88,7 +88,9 @@ TT_API int tt_adaln_forward(void* y, const void* x, const void* scale, const voi
  * aligned; about 10 MB at rows 75600, cols 5120.  (With cols % 8 == 0 but a
  * misaligned tensor at least rows * 8 bytes are needed as well, which can exceed
  * that figure for very short rows; TT_ERR_WORKSPACE is returned if they do not fit.)  The result is
- * bitwise reproducible run to run (fixed summation order, no atomics).
+ * bitwise reproducible run to run (fixed summation order, no atomics), and the same with any workspace of
+ * at least the queried size.  Some smaller ones are taken too (cols % 64 != 0, or the element-wise
+ * kernels' rows * 8 bytes): dscale and dshift are then summed in another order.
  */
 TT_API int tt_adaln_backward(void* dx, float* dscale, float* dshift,
                       const void* dy, const void* x, const void* scale,
@@ -99,15 +101,16 @@ TT_API size_t tt_adaln_backward_workspace_bytes(int64_t rows, int64_t cols, int6
 
 /* tt_adaln_backward for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc): same arguments without the
- * workspace, same kernels, same results bit for bit.  No counterpart in the reference.  The
- * scratch memory (partial column sums) is a device array inside the library,
- * TT_STATIC_WORKSPACE_BYTES (16 MiB); every GPU on which the library's code is loaded holds its
- * own copy until the process ends, whether or not this entry point is ever called.  The call
+ * workspace, same kernels, same results bit for bit (as with a workspace of the queried size).  No
+ * counterpart in the reference.  The scratch memory (partial column sums) is a device array inside the
+ * library, 2 * TT_STATIC_WORKSPACE_BYTES (32 MiB); every GPU on which the library's code is loaded holds
+ * its own copy until the process ends, whether or not this entry point is ever called.  The call
  * performs no hipMalloc / hipFree.  The first call on a GPU looks up that GPU's address of the
  * array (hipGetSymbolAddress) and the launch plan's device properties; a call with rows == 0 does
  * only that and touches no pointer, for callers that want this set-up done at a chosen moment.
- * A shape that needs more scratch than the array holds is refused with TT_ERR_STATIC_LIMIT: the
- * need is what tt_adaln_backward_workspace_bytes() returns (10.2 MB at rows 75600, cols 5120), and
+ * A shape that needs more than TT_STATIC_WORKSPACE_BYTES (16 MiB) is refused with TT_ERR_STATIC_LIMIT.
+ * The need is what tt_adaln_backward_workspace_bytes() returns (10.2 MB at rows 75600, cols 5120; where
+ * cols % 64 != 0, whose kernels keep more workgroups resident, up to twice the limit may still be taken), or
  * rows * 8 bytes when cols is not a multiple of 8 or a tensor is not 16-byte aligned.  All calls
  * on one GPU share the array: two calls that overlap in time on the same GPU (different streams
  * or host threads, or two replays of graphs that captured it) race and give wrong dscale /

@@ -66,7 +66,10 @@ int resident_wgs_per_cu(const KernelInfo& k, int* out) {
 // Backward workspace of tt_adaln_backward_static: a file-scope device array, so that the entry
 // point never allocates.  Every device the library runs on holds its own copy at its own address;
 // the host-side name below is only a handle for hipGetSymbolAddress, never a kernel argument.
-static __device__ __align__(256) unsigned char scratch[TT_STATIC_WORKSPACE_BYTES];
+// The entry point takes what the kernels of whole-line rows (or the element-wise ones) do within
+// TT_STATIC_WORKSPACE_BYTES; those of ragged rows keep up to twice the workgroups resident.
+constexpr size_t kScratchBytes = 2 * (size_t)TT_STATIC_WORKSPACE_BYTES;
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 // Device address of `scratch` on the current device, looked up once per device.
 int static_scratch(void** out) {
@@ -207,6 +210,32 @@ size_t partial_bytes(const Plan& p, int n_acc, int64_t cols) {
   return (size_t)p.n_batches * p.grid_x * n_acc * cols * sizeof(float);
 }
 
+// Caps the grid so that the partial sums fit `bytes`; false if one workgroup a batch does not.
+bool fit_grid(Plan* p, int n_acc, int64_t cols, size_t bytes) {
+  const size_t fit = bytes / ((size_t)p->n_batches * n_acc * cols * sizeof(float));
+  if (fit < 1) return false;
+  if (fit < (size_t)p->grid_x) p->grid_x = (int)fit;
+  return true;
+}
+
+// Whether tt_adaln_backward_static takes an aligned tensor.
+bool static_takes(int64_t rows, int64_t cols, int64_t rows_per_batch) {
+  Plan p;
+  return make_plan(kAdaLN, kBwd, rows, cols, rows_per_batch, &p, false, 0, 0, kMasked) == TT_OK &&
+         partial_bytes(p, 2, cols) <= TT_STATIC_WORKSPACE_BYTES;
+}
+
+// Plan of the backward of aligned rows.  tt_adaln_backward_static runs what tt_adaln_backward does, so where it
+// takes the shape the partial sums have to fit its array (they do without the cap while ragged rows have no more
+// than twice the workgroups of whole-line rows).
+int backward_plan(int kind, int64_t rows, int64_t cols, int64_t rows_per_batch, Plan* p, bool rope = false,
+                  int64_t rope_heads = 0) {
+  const int rc = make_plan(kind, kBwd, rows, cols, rows_per_batch, p, rope, 0, rope_heads);
+  if (rc == TT_OK && kind == kAdaLN && partial_bytes(*p, 2, cols) > kScratchBytes && static_takes(rows, cols, rows_per_batch))
+    fit_grid(p, 2, cols, kScratchBytes);
+  return rc;
+}
+
 size_t workspace_for(int kind, int n_acc, int64_t rows, int64_t cols, int64_t rows_per_batch);
 
 // Backward of rows that the 128-bit kernels do not take (cols % 8 != 0, or tensors that are only 2-byte
@@ -222,20 +251,18 @@ size_t workspace_for(int kind, int n_acc, int64_t rows, int64_t cols, int64_t ro
 // Where cols % 8 == 0 the size query does not know of the misaligned tensor and answers for the aligned
 // kernels, which may want less (two rows a tile: half the workgroups).  The grid is then what the answer
 // holds, so that which kernels run, and the order of their sums, depends on the shape and not on what else
-// the workspace has room for.
+// the workspace has room for.  For the same reason AdaLN's partial sums fit the scratch array, with which
+// tt_adaln_backward_static gives the same bits (300 x 10 x 16383 472 -> 343 us; element-wise where one
+// workgroup a batch does not fit: 5000 x 10 x 1001 338 -> 353).
 constexpr int64_t kOddBwdMaxCols = 16384;
 bool odd_plan(int kind, int64_t rows, int64_t cols, int64_t rows_per_batch, Plan* p) {
   if (cols > kOddBwdMaxCols || make_plan(kind, kBwd, rows, cols, rows_per_batch, p, false, 0, 0, kOdd) != TT_OK) return false;
   const int n_acc = kind == kAdaLN ? 2 : 1;
-  if (cols % kPack == 0) {
-    const size_t per_wg = partial_bytes(*p, n_acc, cols) / p->grid_x;   // one workgroup of every batch
-    const size_t fit = workspace_for(kind, n_acc, rows, cols, rows_per_batch) / per_wg;
-    if (fit < 1) return false;
-    if (fit < (size_t)p->grid_x) p->grid_x = (int)fit;
-  }
   const size_t tensors = (size_t)rows * cols * 4;
   const size_t most = tensors > TT_STATIC_WORKSPACE_BYTES ? tensors : (size_t)TT_STATIC_WORKSPACE_BYTES;
-  return partial_bytes(*p, n_acc, cols) <= most;
+  if (partial_bytes(*p, n_acc, cols) > most) return false;
+  if (kind == kAdaLN && !fit_grid(p, n_acc, cols, kScratchBytes)) return false;
+  return cols % kPack != 0 || fit_grid(p, n_acc, cols, workspace_for(kind, n_acc, rows, cols, rows_per_batch));
 }
 
 // Workspace bound that does not depend on the launch-time occupancy query.
@@ -265,7 +292,7 @@ size_t workspace_for(int kind, int n_acc, int64_t rows, int64_t cols, int64_t ro
   }
   if (g_wgs_per_cu_override.load() > 0 || g_grid_override.load() > 0) return bound;
   Plan p;
-  if (make_plan(kind, kBwd, rows, cols, rows_per_batch, &p) != TT_OK) return bound;
+  if (backward_plan(kind, rows, cols, rows_per_batch, &p) != TT_OK) return bound;
   size_t need = partial_bytes(p, n_acc, cols);
   if (kind != kGateKind && rows_per_batch == rows) {
     Plan ps;
@@ -458,12 +485,12 @@ int backward_partials(int kind, void* dx, const void* dy, const void* x, const v
     if (rrc != TT_OK) return rrc;
   }
   Plan p;
-  int rc = make_plan(kind, kBwd, rows, cols, rows_per_batch, &p, rope != nullptr, 0, rope ? rope->heads : 0);
+  int rc = backward_plan(kind, rows, cols, rows_per_batch, &p, rope != nullptr, rope ? rope->heads : 0);
   if (rc != TT_OK) return rc;
   const int n_acc = kind == kAdaLN ? 2 : 1;
   if (!rope && workspace_bytes < partial_bytes(p, n_acc, cols)) {
-    // The kernels of ragged rows keep more workgroups resident, hence more partial sums, than those of
-    // whole-line rows.  A workspace (the scratch array above all) that would do for the latter gets their grid.
+    // Ragged rows: a workspace smaller than asked for, but large enough for the kernels of whole-line rows
+    // (which have fewer workgroups resident), gets the grid of those.
     Plan pm;
     if (make_plan(kind, kBwd, rows, cols, rows_per_batch, &pm, false, 0, 0, kMasked) == TT_OK &&
         pm.grid_x < p.grid_x && workspace_bytes >= partial_bytes(pm, n_acc, cols))
@@ -615,8 +642,14 @@ int tt_adaln_backward_static(void* dx, float* dscale, float* dshift, const void*
   int rc = static_scratch(&ws);   // per-device set-up on the first call; a rows == 0 call does only this
   if (rc != TT_OK) return rc;
   if (rows == 0) return TT_OK;
-  rc = tt_adaln_backward(dx, dscale, dshift, dy, x, scale, ws, TT_STATIC_WORKSPACE_BYTES,
-                         rows, cols, rows_per_batch, eps, stream);
+  // More is refused than the array could hold: see kScratchBytes.  (Invalid arguments are for tt_adaln_backward to name.)
+  if (rows > 0 && cols > 0 && rows_per_batch > 0 && rows % rows_per_batch == 0 && cols <= TT_MAX_COLS &&
+      rows / rows_per_batch <= 65535 && dx && dy && x && scale && dscale && dshift) {
+    if (vector_path(cols, {dx, dy, x, scale}) ? !static_takes(rows, cols, rows_per_batch)
+                                              : (size_t)rows * 2 * sizeof(float) > TT_STATIC_WORKSPACE_BYTES)
+      return TT_ERR_STATIC_LIMIT;
+  }
+  rc = tt_adaln_backward(dx, dscale, dshift, dy, x, scale, ws, kScratchBytes, rows, cols, rows_per_batch, eps, stream);
   return rc == TT_ERR_WORKSPACE ? TT_ERR_STATIC_LIMIT : rc;
 }
 

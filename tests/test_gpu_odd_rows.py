@@ -70,3 +70,27 @@ def test_odd_widths_run_on_the_faster_kernels(lib, cols):
         torch.cuda.synchronize()
         assert (ws[:rows * 2] != 1e30).all() and (ws[rows * 2:need // 4] != 1e30).any() == vector
         assert (ws[need // 4:] == 1e30).all()
+
+
+# partial sums of all batches, or of one, that exceed the scratch array of tt_adaln_backward_static: ragged and odd
+# rows, misaligned ones (shift), and a modulation vector for every few rows
+@pytest.mark.parametrize("nb,rpb,cols,shift", [(2, 1000, 5128, 0), (1, 3000, 5128, 0), (1, 3000, 8184, 0), (3, 500, 6136, 0),
+                                               (1, 3000, 5127, 0), (2, 700, 8191, 0), (1, 900, 16383, 0), (1, 300, 32767, 0),
+                                               (5, 60, 32767, 0), (300, 10, 8191, 0), (3000, 2, 1001, 0),
+                                               (1, 3000, 5120, 3), (2, 900, 8192, 1), (1, 500, 16384, 4)])
+def test_static_backward_equals_the_workspace_backward(lib, nb, rpb, cols, shift):
+    rows = nb * rpb
+    x, dy = (shifted(rand_bf16(rows, cols, seed=i), shift) for i in range(2))
+    w = rand_bf16(nb, cols, seed=2, scale=0.2).to(DEV)
+    need = max(lib.tt_adaln_backward_workspace_bytes(rows, cols, rpb), rows * 8)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    st = torch.cuda.current_stream().cuda_stream
+    out = [[torch.full_like(x, float("nan")), torch.full((2, nb, cols), float("nan"), device=DEV)] for _ in range(2)]
+    (a, ga), (b, gb) = out
+    assert lib.tt_adaln_backward(a.data_ptr(), ga[0].data_ptr(), ga[1].data_ptr(), dy.data_ptr(), x.data_ptr(), w.data_ptr(),
+                                 ws.data_ptr(), need, rows, cols, rpb, 1e-6, st) == 0
+    for _ in range(2):                          # the array is left as the first call filled it
+        assert lib.tt_adaln_backward_static(b.data_ptr(), gb[0].data_ptr(), gb[1].data_ptr(), dy.data_ptr(), x.data_ptr(),
+                                            w.data_ptr(), rows, cols, rpb, 1e-6, st) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(a, b) and torch.equal(ga, gb)

@@ -116,9 +116,9 @@ def test_backward_at_any_address_and_workspace(lib, cols, shift):
 
 @pytest.mark.parametrize("cols,batches", [(5128, 2), (6136, 2), (2200, 1), (1000, 1)])
 def test_static_scratch_takes_ragged_tensors(lib, cols, batches):
-    """The kernels of ragged rows may keep twice the workgroups of the masked ones resident; with a
-    workspace that is too small for that (the scratch array at 5128 and 6136 columns) the grid shrinks, and the
-    gradients are the same up to the order of the sums: fp32 sums of 1000 O(1) terms."""
+    """The kernels of ragged rows may keep twice the workgroups of the masked ones resident; where the partial
+    sums of all batches are too large for the scratch array (5128 and 6136 columns) they go through it batch by
+    batch, with the same bits."""
     from teletron_amd import cabi, ops
     rows = 1000 * batches
     need = lib.tt_adaln_backward_workspace_bytes(rows, cols, 1000)
@@ -131,5 +131,4 @@ def test_static_scratch_takes_ragged_tensors(lib, cols, batches):
                                         w.data_ptr(), rows, cols, 1000, 1e-6, torch.cuda.current_stream().cuda_stream) == 0
     torch.cuda.synchronize()
     assert torch.equal(dx, dx2)
-    for a, b in ((g[0], ds), (g[1], dh)):
-        assert float((a - b).norm() / b.norm()) < 1e-5
+    assert torch.equal(g[0], ds) and torch.equal(g[1], dh)
