@@ -73,20 +73,28 @@ __device__ __forceinline__ u32x4 load_row(const void* base, size_t elem_off) {
   if constexpr (ROWS == kRagged && SHORT) return load_cached(base, elem_off);
   else return load_stream(base, elem_off);
 }
-// Stores the pack of slot `seg + lane` (seg: first slot of the wave's segment, a multiple of 64) of a row.
+// Element offset of a lane's pack, from the column that its loads use (no further register) or from its slot.
+// The kernels of 16 waves a row have 128 registers a lane and spill: with every slot in use they are
+// the faster with the latter (32768 columns, AdaLN forward 133 -> 116, gate backward 338 -> 245 us; 16384,
+// AdaLN backward 648 -> 571), where the others lose up to 16 % (ungated residual + norm backward,
+// 8192 x 1536 24.5 -> 29.3: fewer registers let a second workgroup onto the CU, whose partial sums cost more
+// than it gives).
+template <int ROWS, int W>
+__device__ __forceinline__ size_t pack_offset(int64_t row, int C, int col, int packs, int slot) {
+  if constexpr (ROWS == kFull && W >= 16) return (size_t)(row * packs + slot) * kPack;
+  else return (size_t)(row * C + col);
+}
+// Stores a lane's pack (act: the row has it); `left`: packs of the row from the wave's segment of 64 on.
 template <int ROWS, bool SHORT>
-__device__ __forceinline__ void store_row(void* base, int64_t row, int packs, int seg, int lane, u32x4 v) {
-  const int64_t pack = row * packs + seg + lane;
-  u32x4* p = reinterpret_cast<u32x4*>(base) + pack;
-  if constexpr (ROWS != kFull) {
-    if (seg + lane >= packs) return;
-  }
+__device__ __forceinline__ void store_row(void* base, size_t elem_off, bool act, int left, int lane, u32x4 v) {
+  if (!act) return;
   if constexpr (ROWS == kRagged) {
+    u32x4* p = reinterpret_cast<u32x4*>(static_cast<uint16_t*>(base) + elem_off);
     bool shared = true;
     if constexpr (!SHORT) {
       // position of the pack inside its 128-byte line, and whether the segment holds that whole line
       const int at = (static_cast<int>(reinterpret_cast<uintptr_t>(p) >> 4)) & 7;
-      const int last = packs - seg < 64 ? packs - seg - 1 : 63;
+      const int last = left < 64 ? left - 1 : 63;
       shared = lane < at || lane + 7 - at > last;
     }
     if (shared) {
@@ -95,7 +103,7 @@ __device__ __forceinline__ void store_row(void* base, int64_t row, int packs, in
       return;
     }
   }
-  store_stream(p, 0, v);
+  store_stream(base, elem_off, v);
 }
 
 // ---- kOdd rows: packs at any 2-byte address (this target's vector memory instructions take them)

@@ -102,7 +102,7 @@ __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
             acc0[p][j] = fmaf(af[r][p][j], bf[r][p][j], acc0[p][j]);
           }
         }
-        if (row0 + r < S) store_row<ROWS, SHORT>(a.out, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
+        if (row0 + r < S) store_row<ROWS, SHORT>(a.out, pack_offset<ROWS, W>(row, C, col[p], a.packs, (p * W + w) * 64 + lane), act[p], a.packs - (p * W + w) * 64, lane, pack8(o));
       }
     }
   }

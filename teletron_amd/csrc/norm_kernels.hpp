@@ -328,7 +328,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
               store_any(a.y, (size_t)(row * C + col[p]), pack8(o), n[p]);
               if constexpr (XN) store_any(a.x_norm, (size_t)(row * C + col[p]), pack8(xn), n[p]);
             } else if constexpr (XN) store_stream2(a.y, a.x_norm, (size_t)(row * C + col[p]), pack8(o), pack8(xn));
-            else              store_row<ROWS, SHORT>(a.y, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
+            else              store_row<ROWS, SHORT>(a.y, pack_offset<ROWS, W>(row, C, col[p], a.packs, (p * W + w) * 64 + lane), act[p], a.packs - (p * W + w) * 64, lane, pack8(o));
           }
         }
         if (w == 0 && lane == 0) {
@@ -577,7 +577,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
         }
         if constexpr (ODD) {
           if (rv[r]) store_any(a.dx, (size_t)(row * C + col[p]), pack8(o), n[p]);
-        } else if (rv[r]) store_row<ROWS, SHORT>(a.dx, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
+        } else if (rv[r]) store_row<ROWS, SHORT>(a.dx, pack_offset<ROWS, W>(row, C, col[p], a.packs, (p * W + w) * 64 + lane), act[p], a.packs - (p * W + w) * 64, lane, pack8(o));
       }
     }
   }

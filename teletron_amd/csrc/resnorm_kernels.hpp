@@ -185,7 +185,7 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs 
         for (int j = 0; j < 8; ++j) xf[r][p][j] = GATED ? fmaf(gt[p][j], rf[j], xf[r][p][j]) : xf[r][p][j] + rf[j];
         // the residual stream is stored as bf16, and it is that rounded value which is normalised
         const u32x4 sp = pack8(xf[r][p]);
-        if (rv[r]) store_row<ROWS, SHORT>(a.s, row, a.packs, p * 64 * W + w * 64, lane, sp);
+        if (rv[r]) store_row<ROWS, SHORT>(a.s, (size_t)(row * C + col[p]), act[p], a.packs - (p * W + w) * 64, lane, sp);
         unpack8(sp, xf[r][p]);
       }
     }
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs 
             float o[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) o[j] = fmaf(xf[r][p][j] * rstd, g[p][j], sh[p][j]);
-            store_row<ROWS, SHORT>(a.y, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
+            store_row<ROWS, SHORT>(a.y, (size_t)(row * C + col[p]), act[p], a.packs - (p * W + w) * 64, lane, pack8(o));
           }
         }
         if (w == 0 && lane == 0) {
@@ -400,8 +400,8 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_bwd_wide(const ResBwdArgs 
           }
         }
         if (rv[r]) {
-          store_row<ROWS, SHORT>(a.dx, row, a.packs, p * 64 * W + w * 64, lane, pack8(o));
-          if constexpr (GATED) store_row<ROWS, SHORT>(a.dr, row, a.packs, p * 64 * W + w * 64, lane, pack8(o2));
+          store_row<ROWS, SHORT>(a.dx, (size_t)(row * C + col[p]), act[p], a.packs - (p * W + w) * 64, lane, pack8(o));
+          if constexpr (GATED) store_row<ROWS, SHORT>(a.dr, (size_t)(row * C + col[p]), act[p], a.packs - (p * W + w) * 64, lane, pack8(o2));
         }
       }
     }
