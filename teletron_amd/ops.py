@@ -10,6 +10,8 @@ consecutive groups, group ``b`` using modulation vector ``b``.
 from __future__ import annotations
 
 import ctypes
+import importlib
+import importlib.util
 import threading
 from typing import Optional, Tuple
 
@@ -20,7 +22,15 @@ from . import cabi
 BF16 = torch.bfloat16
 
 
-_native = None
+_native = None    # the module, or False where it is not built
+
+
+def _load_native():
+    """native_ops, or False where the package is built without the torch modules (the C ABI alone).  One that is
+    there and does not load (built for another torch) raises."""
+    if importlib.util.find_spec(__package__ + ".native_ops") is None:
+        return False
+    return importlib.import_module(__package__ + ".native_ops")
 
 
 def native(x: torch.Tensor):
@@ -31,9 +41,8 @@ def native(x: torch.Tensor):
     if type(x) not in (torch.Tensor, torch.nn.Parameter) or not x.is_cuda:
         return None
     if _native is None:
-        from . import native_ops      # built by `python -m teletron_amd.build`
-        _native = native_ops
-    return _native
+        _native = _load_native()
+    return _native or None
 
 
 def _require(cond: bool, exc, msg: str):
@@ -196,7 +205,7 @@ def clear_workspaces() -> None:
     until they finish (the caching allocator frees in stream order)."""
     with _WORKSPACES_LOCK:
         _WORKSPACES.clear()
-    if _native is not None:
+    if _native:
         _native.clear_workspaces()
 
 

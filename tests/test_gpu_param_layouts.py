@@ -115,3 +115,22 @@ def test_native_calls_equal_the_python_ones(cols, monkeypatch):
     for (call, inputs), got in zip(calls, native):
         for a, b in zip(got, grads(call(), inputs, 3)):
             assert torch.equal(a, b)
+
+
+def test_operators_run_without_the_native_module(monkeypatch):
+    """As after a build of the C ABI alone: the same bits through ops.py."""
+    import importlib.util
+    from teletron_amd import functional as T, ops
+    x = rand_bf16(2, 29, 1536, seed=1).to(DEV).requires_grad_(True)
+    w = rand_bf16(1536, seed=2).to(DEV).requires_grad_(True)
+    want = grads(T.rms_norm(x, w), [x, w], 3) + grads(T.adaln_modulate(x, w, w), [x, w], 3)
+    find = importlib.util.find_spec
+    monkeypatch.setattr(importlib.util, "find_spec", lambda name, *a: None if name.endswith("native_ops") else find(name, *a))
+    monkeypatch.setitem(__import__("sys").modules, "teletron_amd.native_ops", None)      # and importing it would raise
+    monkeypatch.delattr("teletron_amd.native_ops")
+    monkeypatch.setattr(ops, "_native", None)
+    got = grads(T.rms_norm(x, w), [x, w], 3) + grads(T.adaln_modulate(x, w, w), [x, w], 3)
+    assert ops.native(x) is None
+    ops.clear_workspaces()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

@@ -240,3 +240,21 @@ def test_installed_form_exports_the_reference_module_names(tmp_path):
     r = subprocess.run([sys.executable, "-c", code], cwd=str(tmp_path), env=env, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
     assert str(site) in r.stdout
+
+
+def test_operators_do_without_the_native_module(monkeypatch):
+    """Built with --no-torch-ext there is no native_ops: ops.py then takes every call.  A module that is there
+    and does not load is an error."""
+    import importlib.util
+    from teletron_amd import ops
+    assert ops._load_native().__name__ == "teletron_amd.native_ops"
+    find = importlib.util.find_spec
+    monkeypatch.setattr(importlib.util, "find_spec", lambda name, *a: None if name.endswith("native_ops") else find(name, *a))
+    assert ops._load_native() is False
+    monkeypatch.undo()
+
+    def broken(name):
+        raise ImportError("undefined symbol")
+    monkeypatch.setattr(importlib, "import_module", broken)
+    with pytest.raises(ImportError):
+        ops._load_native()
