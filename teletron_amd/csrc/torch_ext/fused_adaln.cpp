@@ -36,13 +36,13 @@ void torch_launch_adaln_backward(torch::Tensor& dinp, torch::Tensor& dscale, tor
   check_param(dshift, "dshift", cols, dout);
   check_rowstat(inv_variance, "inv_variance", rows, dout);
   c10::hip::HIPGuard guard(dout.device().index());
-  const size_t ws_bytes = tt_adaln_backward_workspace_bytes(rows, cols, rows);
-  torch::Tensor ws = workspace(ws_bytes, dout);
-  check_status(tt_launch_adaln_backward(dinp.data_ptr(), dscale.data_ptr(), dshift.data_ptr(), dout.data_ptr(),
-                                        x_norm.data_ptr(), scale.data_ptr(),
-                                        static_cast<const float*>(inv_variance.data_ptr()), rows, cols,
-                                        ws.data_ptr(), ws_bytes, current_stream(dout)),
-               "torch_launch_adaln_backward");
+  const int rc = with_workspace(tt_adaln_backward_workspace_bytes(rows, cols, rows), dout, [&](void* ws, size_t ws_bytes) {
+    return tt_launch_adaln_backward(dinp.data_ptr(), dscale.data_ptr(), dshift.data_ptr(), dout.data_ptr(),
+                                    x_norm.data_ptr(), scale.data_ptr(),
+                                    static_cast<const float*>(inv_variance.data_ptr()), rows, cols,
+                                    ws, ws_bytes, current_stream(dout));
+  });
+  check_status(rc, "torch_launch_adaln_backward");
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {

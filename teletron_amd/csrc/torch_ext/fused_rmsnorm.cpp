@@ -29,12 +29,12 @@ void torch_launch_rms_backward(torch::Tensor& dinp, torch::Tensor& dweight, cons
   check_param(dweight, "dweight", cols, dout);
   check_rowstat(inv_variance, "inv_variance", rows, dout);
   c10::hip::HIPGuard guard(dout.device().index());
-  const size_t ws_bytes = tt_rmsnorm_backward_workspace_bytes(rows, cols);
-  torch::Tensor ws = workspace(ws_bytes, dout);
-  check_status(tt_launch_rms_backward(dinp.data_ptr(), dweight.data_ptr(), dout.data_ptr(), x_norm.data_ptr(),
-                                      weight.data_ptr(), static_cast<const float*>(inv_variance.data_ptr()),
-                                      rows, cols, ws.data_ptr(), ws_bytes, current_stream(dout)),
-               "torch_launch_rms_backward");
+  const int rc = with_workspace(tt_rmsnorm_backward_workspace_bytes(rows, cols), dout, [&](void* ws, size_t ws_bytes) {
+    return tt_launch_rms_backward(dinp.data_ptr(), dweight.data_ptr(), dout.data_ptr(), x_norm.data_ptr(),
+                                  weight.data_ptr(), static_cast<const float*>(inv_variance.data_ptr()),
+                                  rows, cols, ws, ws_bytes, current_stream(dout));
+  });
+  check_status(rc, "torch_launch_rms_backward");
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {

@@ -7,7 +7,9 @@
 #include <hip/hip_runtime_api.h>
 
 #include <map>
+#include <memory>
 #include <mutex>
+#include <optional>
 #include <utility>
 
 #include "teletron_op.h"
@@ -40,22 +42,50 @@ inline void* current_stream(const torch::Tensor& t) {
 // Backward workspace (per-workgroup partial sums): one tensor per (device, stream), grown on demand
 // and reused from call to call, so a backward call does not go to the allocator (the reference
 // allocates its fp32 [32, C] scratch on every call, teletron_op/fused_rmsnorm/weight_backward.cu:229).
-// Launches on one stream run in order, so consecutive calls never overlap in it.  A stream under
-// graph capture gets memory of its own from the capture's pool: the graph keeps the pointer.
-// The cache is never destroyed (the HIP runtime may be gone by the time static destructors run).
-inline torch::Tensor workspace(size_t bytes, const torch::Tensor& ref) {
+struct Workspace {
+  std::mutex mu;          // held from the look at `memory` until everything that uses it is queued
+  torch::Tensor memory;
+};
+struct Workspaces {
+  std::mutex mu;
+  std::map<std::pair<int, hipStream_t>, std::shared_ptr<Workspace>> kept;
+};
+// Never destroyed: the HIP runtime may be gone by the time static destructors run.
+inline Workspaces& workspaces() {
+  static auto* w = new Workspaces();
+  return *w;
+}
+constexpr int64_t kKeepBytes = 64 << 20;   // more than this is not kept between calls
+
+// Calls launch(memory, bytes), which queues a backward call's two kernels on the current stream of ref's
+// device, and returns its result; `bytes` is what was asked for, however large the kept memory is.  Launches on one stream run in order, so consecutive calls never overlap in
+// the workspace; the lock keeps two host threads from queueing kernel, kernel, reduction, reduction.  The GIL
+// is released first (the launch may wait for room in the queue, and the lock for another Python thread).
+// A stream under graph capture gets memory of its own from the capture's pool: the graph keeps the pointer.
+template <typename F>
+auto with_workspace(size_t bytes, const torch::Tensor& ref, F launch) {
+  std::optional<pybind11::gil_scoped_release> unlocked;
+  if (PyGILState_Check()) unlocked.emplace();   // a call through torch.ops comes without it
   const auto opts = at::TensorOptions().dtype(at::kByte).device(ref.device());
   const int64_t need = static_cast<int64_t>(bytes < 16 ? 16 : bytes);
-  hipStream_t stream = c10::hip::getCurrentHIPStream(ref.device().index()).stream();
+  const int device = static_cast<int>(ref.device().index());
+  hipStream_t stream = c10::hip::getCurrentHIPStream(device).stream();
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) (void)hipGetLastError();
-  if (capturing != hipStreamCaptureStatusNone) return at::empty({need}, opts);
-  static std::mutex mu;
-  static auto* cache = new std::map<std::pair<int, hipStream_t>, torch::Tensor>();
-  std::lock_guard<std::mutex> lock(mu);
-  torch::Tensor& ws = (*cache)[{static_cast<int>(ref.device().index()), stream}];
-  if (!ws.defined() || ws.numel() < need) ws = at::empty({need}, opts);
-  return ws;
+  if (capturing != hipStreamCaptureStatusNone || need > kKeepBytes) {
+    const torch::Tensor own = at::empty({need}, opts);
+    return launch(own.data_ptr(), static_cast<size_t>(need));
+  }
+  std::shared_ptr<Workspace> ws;
+  {
+    std::lock_guard<std::mutex> lock(workspaces().mu);
+    auto& entry = workspaces().kept[{device, stream}];
+    if (!entry) entry = std::make_shared<Workspace>();
+    ws = entry;
+  }
+  std::lock_guard<std::mutex> lock(ws->mu);
+  if (!ws->memory.defined() || ws->memory.numel() < need) ws->memory = at::empty({need}, opts);
+  return launch(ws->memory.data_ptr(), static_cast<size_t>(need));
 }
 inline void check_status(int rc, const char* what) {
   TORCH_CHECK(rc == TT_OK, what, " failed: ", tt_error_string(rc),

@@ -14,33 +14,10 @@ using std::optional;
 
 namespace {
 
-constexpr int64_t kKeepBytes = 64 << 20;
-
-struct Workspaces {
-  std::mutex mu;
-  std::map<std::pair<int, hipStream_t>, Tensor> kept;
-};
-Workspaces& workspaces() {
-  static auto* w = new Workspaces();   // never destroyed: the HIP runtime may be gone before static destructors run
-  return *w;
-}
-
-// One tensor per (device, stream), reused from call to call: launches on one stream run in order.
-// A stream under graph capture gets memory from the capture's pool, and what is over kKeepBytes is not kept.
-Tensor workspace(size_t bytes, const Tensor& ref, hipStream_t stream) {
-  const auto opts = at::TensorOptions().dtype(at::kByte).device(ref.device());
-  const int64_t need = static_cast<int64_t>(bytes < 16 ? 16 : bytes);
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) (void)hipGetLastError();
-  if (capturing != hipStreamCaptureStatusNone || need > kKeepBytes) return at::empty({need}, opts);
-  std::lock_guard<std::mutex> lock(workspaces().mu);
-  Tensor& ws = workspaces().kept[{static_cast<int>(ref.device().index()), stream}];
-  if (!ws.defined() || ws.numel() < need) ws = at::empty({need}, opts);
-  return ws;
-}
 void clear_workspaces() {
-  std::lock_guard<std::mutex> lock(workspaces().mu);
-  workspaces().kept.clear();
+  auto& w = tt_glue::workspaces();
+  std::lock_guard<std::mutex> lock(w.mu);
+  w.kept.clear();
 }
 
 bool plain(const Tensor& t) { return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !at::isTensorSubclassLike(t); }
@@ -95,6 +72,11 @@ bool launched(F f) {
   py::gil_scoped_release unlocked;
   return f() == TT_OK;
 }
+// The same with the backward workspace: f(memory, bytes).
+template <typename F>
+bool launched(size_t bytes, const Tensor& ref, F f) {
+  return tt_glue::with_workspace(bytes, ref, f) == TT_OK;
+}
 // Errors of the allocator and of tensors without memory are raised by ops.py, as its own types.
 template <typename... A>
 auto guarded(py::object (*f)(A...)) {
@@ -131,10 +113,9 @@ py::object adaln_backward(const Tensor& dy, const Tensor& x, const Tensor& scale
   const auto opts = x.options().dtype(bf16 ? at::kBFloat16 : at::kFloat);
   Tensor dx = at::empty_like(x), dscale = at::empty(scale_shape, opts), dshift = at::empty(shift_shape, opts);
   if (dscale.numel() != a.n * cols || dshift.numel() != a.n * cols) return py::none();
-  const size_t bytes = tt_adaln_backward_workspace_bytes(rows, cols, rows / a.n);
-  Tensor ws = workspace(bytes, x, on.stream);
-  if (!launched([&] { return tt_adaln_backward_typed(dx.data_ptr(), dscale.data_ptr(), dshift.data_ptr(), bf16, dy.data_ptr(), x.data_ptr(),
-                              scale.data_ptr(), ws.data_ptr(), ws.numel(), rows, cols, rows / a.n, (float)eps,
+  if (!launched(tt_adaln_backward_workspace_bytes(rows, cols, rows / a.n), x,
+                [&](void* ws, size_t ws_bytes) { return tt_adaln_backward_typed(dx.data_ptr(), dscale.data_ptr(), dshift.data_ptr(), bf16, dy.data_ptr(), x.data_ptr(),
+                              scale.data_ptr(), ws, ws_bytes, rows, cols, rows / a.n, (float)eps,
                               on.stream); }))
     return py::none();
   return py::make_tuple(dx, dscale, dshift);
@@ -198,10 +179,10 @@ py::object rmsnorm_backward(const Tensor& dy, const Tensor& x, const Tensor& wei
   Launch on(x);
   Tensor dx = at::empty_like(x), dweight = at::empty(weight_shape, x.options().dtype(bf16 ? at::kBFloat16 : at::kFloat));
   if (dweight.numel() != cols) return py::none();
-  Tensor ws = workspace(tt_rmsnorm_backward_workspace_bytes(rows, cols), x, on.stream);
-  if (!launched([&] { return tt_rmsnorm_backward_typed(dx.data_ptr(), dweight.data_ptr(), bf16, dy.data_ptr(), x.data_ptr(), weight.data_ptr(),
+  if (!launched(tt_rmsnorm_backward_workspace_bytes(rows, cols), x,
+                [&](void* ws, size_t ws_bytes) { return tt_rmsnorm_backward_typed(dx.data_ptr(), dweight.data_ptr(), bf16, dy.data_ptr(), x.data_ptr(), weight.data_ptr(),
                                 freqs ? static_cast<const float*>(freqs->data_ptr()) : nullptr, head_dim, heads, seq,
-                                ws.data_ptr(), ws.numel(), rows, cols, (float)eps, on.stream); }))
+                                ws, ws_bytes, rows, cols, (float)eps, on.stream); }))
     return py::none();
   return py::make_tuple(dx, dweight);
 }
@@ -228,9 +209,9 @@ py::object gate_backward(const Tensor& dout, const Tensor& gate, const Tensor& r
   Launch on(dout);
   Tensor dres = at::empty_like(dout), dgate = at::empty(gate_shape, dout.options().dtype(bf16 ? at::kBFloat16 : at::kFloat));
   if (dgate.numel() != g.n * cols) return py::none();
-  Tensor ws = workspace(tt_gate_residual_backward_workspace_bytes(rows, cols, rows / g.n), dout, on.stream);
-  if (!launched([&] { return tt_gate_residual_backward_typed(dres.data_ptr(), dgate.data_ptr(), bf16, dout.data_ptr(), gate.data_ptr(),
-                                      residual.data_ptr(), ws.data_ptr(), ws.numel(), rows, cols, rows / g.n,
+  if (!launched(tt_gate_residual_backward_workspace_bytes(rows, cols, rows / g.n), dout,
+                [&](void* ws, size_t ws_bytes) { return tt_gate_residual_backward_typed(dres.data_ptr(), dgate.data_ptr(), bf16, dout.data_ptr(), gate.data_ptr(),
+                                      residual.data_ptr(), ws, ws_bytes, rows, cols, rows / g.n,
                                       on.stream); }))
     return py::none();
   return py::make_tuple(dres, dgate);
@@ -272,11 +253,11 @@ py::object residual_norm_backward(const Tensor& dy, const optional<Tensor>& ds_i
   Tensor dx = at::empty_like(s), dr = gate ? at::empty_like(s) : dx, dscale = at::empty({nb, cols}, opts),
          dshift = at::empty({nb, cols}, opts), dgate;
   if (gate) dgate = at::empty({nb, cols}, opts);
-  Tensor ws = workspace(tt_residual_norm_backward_workspace_bytes(rows, cols, rows / nb, gate ? 1 : 0), s, on.stream);
-  if (!launched([&] { return tt_residual_norm_backward_typed(dx.data_ptr(), gate ? dr.data_ptr() : nullptr, dscale.data_ptr(), dshift.data_ptr(),
+  if (!launched(tt_residual_norm_backward_workspace_bytes(rows, cols, rows / nb, gate ? 1 : 0), s,
+                [&](void* ws, size_t ws_bytes) { return tt_residual_norm_backward_typed(dx.data_ptr(), gate ? dr.data_ptr() : nullptr, dscale.data_ptr(), dshift.data_ptr(),
                                       gate ? dgate.data_ptr() : nullptr, bf16, dy.data_ptr(), ds_in ? ds_in->data_ptr() : nullptr,
                                       s.data_ptr(), gate ? r->data_ptr() : nullptr, gate ? gate->data_ptr() : nullptr, g.n,
-                                      scale.data_ptr(), a.n, affine, ws.data_ptr(), ws.numel(), rows, cols, rows / nb, (float)eps,
+                                      scale.data_ptr(), a.n, affine, ws, ws_bytes, rows, cols, rows / nb, (float)eps,
                                       on.stream); }))
     return py::none();
   return py::make_tuple(dx, dr, dscale, dshift, gate ? py::cast(dgate) : py::object(py::none()));

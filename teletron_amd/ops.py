@@ -9,6 +9,7 @@ consecutive groups, group ``b`` using modulation vector ``b``.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import importlib
 import importlib.util
@@ -193,7 +194,14 @@ def rmsnorm_forward_saving(x: torch.Tensor, weight: torch.Tensor, eps: float, sa
     return (y if view is None else y.permute(_inverse(perm))), kept
 
 
-_WORKSPACES = {}   # (device index, stream handle) -> uint8 tensor, grown on demand
+class _Workspace:
+    """The kept backward workspace of one stream (uint8, grown on demand), and the lock under which it is used."""
+
+    def __init__(self):
+        self.lock, self.memory = threading.RLock(), None
+
+
+_WORKSPACES = {}   # (device index, stream handle) -> _Workspace
 _WORKSPACES_LOCK = threading.Lock()   # backward runs on autograd's threads, one per device
 # the element-wise path's row statistics (rows * 8 bytes) are only kept between calls up to this size
 _WORKSPACE_KEEP_BYTES = 64 << 20
@@ -209,27 +217,31 @@ def clear_workspaces() -> None:
         _native.clear_workspaces()
 
 
-def _workspace(lib_bytes: int, rows: int, *tensors: torch.Tensor) -> torch.Tensor:
-    """Backward workspace (partial column sums), kept per device and stream and reused from call to
-    call: launches on one stream run in order, so consecutive backward calls never overlap in it.
-    Tensors that are not 16-byte aligned need at least two floats per row there."""
+@contextlib.contextmanager
+def _workspace(lib_bytes: int, rows: int, *tensors: torch.Tensor):
+    """Backward workspace (partial column sums) as ``(address, bytes)``, kept per device and stream and reused
+    from call to call: launches on one stream run in order, so consecutive backward calls never overlap in it.
+    It is locked until the caller has queued both of its kernels, or two host threads on one stream could
+    queue kernel, kernel, reduction, reduction.  Tensors that are not 16-byte aligned need at least two floats
+    per row there."""
     need = lib_bytes
     if any(t.data_ptr() % 16 for t in tensors):
         need = max(need, rows * 8)
     need = max(need, 16)
     dev = tensors[0].device
-    if torch.cuda.is_current_stream_capturing():
+    if torch.cuda.is_current_stream_capturing() or need > _WORKSPACE_KEEP_BYTES:
         # a captured graph keeps the pointers it recorded: give it memory of its own (from the
         # capture's private pool), never the shared buffer
-        return torch.empty(need, dtype=torch.uint8, device=dev)
+        own = torch.empty(need, dtype=torch.uint8, device=dev)
+        yield own.data_ptr(), need
+        return
     key = (dev.index, _stream(tensors[0]))
     with _WORKSPACES_LOCK:
-        ws = _WORKSPACES.get(key)
-        if ws is None or ws.numel() < need:
-            ws = torch.empty(need, dtype=torch.uint8, device=dev)
-            if need <= _WORKSPACE_KEEP_BYTES:
-                _WORKSPACES[key] = ws
-    return ws
+        ws = _WORKSPACES.setdefault(key, _Workspace())
+    with ws.lock:
+        if ws.memory is None or ws.memory.numel() < need:
+            ws.memory = torch.empty(need, dtype=torch.uint8, device=dev)
+        yield ws.memory.data_ptr(), need
 
 
 def _stream(t: torch.Tensor) -> int:
@@ -275,10 +287,10 @@ def adaln_backward_packed(dy: torch.Tensor, x: torch.Tensor, scale: torch.Tensor
     if rows == 0:
         return dx, torch.zeros(2, nb, cols, dtype=dtype, device=x.device)
     grads = torch.empty(2, nb, cols, dtype=dtype, device=x.device)
-    with torch.cuda.device(x.device):
-        ws = _workspace(cabi.load().tt_adaln_backward_workspace_bytes(rows, cols, rpb), rows, x, dy, dx, scale)
+    with torch.cuda.device(x.device), \
+            _workspace(cabi.load().tt_adaln_backward_workspace_bytes(rows, cols, rpb), rows, x, dy, dx, scale) as (ws, ws_bytes):
         cabi.call("tt_adaln_backward_typed", dx.data_ptr(), grads[0].data_ptr(), grads[1].data_ptr(), int(dtype == BF16),
-                  dy.data_ptr(), x.data_ptr(), scale.data_ptr(), ws.data_ptr(), ws.numel(),
+                  dy.data_ptr(), x.data_ptr(), scale.data_ptr(), ws, ws_bytes,
                   rows, cols, rpb, float(eps), _stream(x))
     return dx, grads
 
@@ -331,10 +343,10 @@ def rmsnorm_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, ep
     if rows == 0:
         return dx, torch.zeros(cols, dtype=dtype, device=x.device)
     dweight = torch.empty(cols, dtype=dtype, device=x.device)
-    with torch.cuda.device(x.device):
-        ws = _workspace(cabi.load().tt_rmsnorm_backward_workspace_bytes(rows, cols), rows, x, dy, dx, weight)
+    with torch.cuda.device(x.device), \
+            _workspace(cabi.load().tt_rmsnorm_backward_workspace_bytes(rows, cols), rows, x, dy, dx, weight) as (ws, ws_bytes):
         cabi.call("tt_rmsnorm_backward_typed", dx.data_ptr(), dweight.data_ptr(), int(dtype == BF16), dy.data_ptr(),
-                  x.data_ptr(), weight.data_ptr(), None, 0, 0, 0, ws.data_ptr(), ws.numel(), rows, cols, float(eps), _stream(x))
+                  x.data_ptr(), weight.data_ptr(), None, 0, 0, 0, ws, ws_bytes, rows, cols, float(eps), _stream(x))
     return dx, dweight
 
 
@@ -395,10 +407,10 @@ def gate_residual_backward(dout: torch.Tensor, gate: torch.Tensor, residual: tor
     if rows == 0:
         return dres, torch.zeros(nb, cols, dtype=dtype, device=dout.device)
     dgate = torch.empty(nb, cols, dtype=dtype, device=dout.device)
-    with torch.cuda.device(dout.device):
-        ws = _workspace(cabi.load().tt_gate_residual_backward_workspace_bytes(rows, cols, rpb), 0, dout)
+    with torch.cuda.device(dout.device), \
+            _workspace(cabi.load().tt_gate_residual_backward_workspace_bytes(rows, cols, rpb), 0, dout) as (ws, ws_bytes):
         cabi.call("tt_gate_residual_backward_typed", dres.data_ptr(), dgate.data_ptr(), int(dtype == BF16), dout.data_ptr(), gate.data_ptr(),
-                  residual.data_ptr(), ws.data_ptr(), ws.numel(), rows, cols, rpb, _stream(dout))
+                  residual.data_ptr(), ws, ws_bytes, rows, cols, rpb, _stream(dout))
     return dres, dgate
 
 
@@ -445,10 +457,10 @@ def rmsnorm_rope_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tenso
     if rows == 0:
         return dx, torch.zeros(cols, dtype=dtype, device=x.device)
     dweight = torch.empty(cols, dtype=dtype, device=x.device)
-    with torch.cuda.device(x.device):
-        ws = _workspace(cabi.load().tt_rmsnorm_backward_workspace_bytes(rows, cols), 0, x)
+    with torch.cuda.device(x.device), \
+            _workspace(cabi.load().tt_rmsnorm_backward_workspace_bytes(rows, cols), 0, x) as (ws, ws_bytes):
         cabi.call("tt_rmsnorm_backward_typed", dx.data_ptr(), dweight.data_ptr(), int(dtype == BF16), dy.data_ptr(),
-                  x.data_ptr(), weight.data_ptr(), freqs.data_ptr(), head_dim, 0, seq, ws.data_ptr(), ws.numel(),
+                  x.data_ptr(), weight.data_ptr(), freqs.data_ptr(), head_dim, 0, seq, ws, ws_bytes,
                   rows, cols, float(eps), _stream(x))
     return dx, dweight
 
@@ -507,10 +519,10 @@ def rmsnorm_rope_heads_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch
     if rows == 0:
         return (dx if perm is None else dx.permute(_inverse(perm))), torch.zeros(d, dtype=dtype, device=xm.device)
     dweight = torch.empty(d, dtype=dtype, device=xm.device)
-    with torch.cuda.device(xm.device):
-        ws = _workspace(cabi.load().tt_rmsnorm_backward_workspace_bytes(rows, d), 0, xm)
+    with torch.cuda.device(xm.device), \
+            _workspace(cabi.load().tt_rmsnorm_backward_workspace_bytes(rows, d), 0, xm) as (ws, ws_bytes):
         cabi.call("tt_rmsnorm_backward_typed", dx.data_ptr(), dweight.data_ptr(), int(dtype == BF16), dym.data_ptr(),
-                  xm.data_ptr(), weight.data_ptr(), freqs.data_ptr(), d, heads, seq, ws.data_ptr(), ws.numel(),
+                  xm.data_ptr(), weight.data_ptr(), freqs.data_ptr(), d, heads, seq, ws, ws_bytes,
                   rows, d, float(eps), _stream(xm))
     return (dx if perm is None else dx.permute(_inverse(perm))), dweight
 
@@ -628,10 +640,10 @@ def residual_norm_backward(dy: torch.Tensor, ds_in: Optional[torch.Tensor], s: t
             (torch.zeros(nb, cols, **like) if gate is not None else None)
     dscale, dshift = torch.empty(nb, cols, **like), torch.empty(nb, cols, **like)
     dgate = torch.empty(nb, cols, **like) if gate is not None else None
-    with torch.cuda.device(s.device):
-        ws = _workspace(cabi.load().tt_residual_norm_backward_workspace_bytes(rows, cols, rpb, int(gate is not None)), 0, s)
+    with torch.cuda.device(s.device), \
+            _workspace(cabi.load().tt_residual_norm_backward_workspace_bytes(rows, cols, rpb, int(gate is not None)), 0, s) as (ws, ws_bytes):
         cabi.call("tt_residual_norm_backward_typed", dx.data_ptr(), _ptr(dr if gate is not None else None),
                   dscale.data_ptr(), dshift.data_ptr(), _ptr(dgate), int(dtype == BF16), dy.data_ptr(), _ptr(ds_in), s.data_ptr(),
                   _ptr(residual if gate is not None else None), _ptr(gate), n_gate, scale.data_ptr(), n_param,
-                  int(bool(affine)), ws.data_ptr(), ws.numel(), rows, cols, rpb, float(eps), _stream(s))
+                  int(bool(affine)), ws, ws_bytes, rows, cols, rpb, float(eps), _stream(s))
     return dx, dr, dscale, dshift, dgate
