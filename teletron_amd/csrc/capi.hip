@@ -149,10 +149,22 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
     k = res == 2 ? resnorm_gated_kernel(dir == kBwd, idx, mode) : resnorm_plain_kernel(dir == kBwd, idx, mode);
   } else if (rope) {
     if (kind != kRMS || dir == kBwdSaved || dir == kFwdXn) return TT_ERR_UNSUPPORTED;
-    // Token mode has larger tiles: where the tensor is too small to give every CU several, the forward is
-    // faster row by row (2000 x 24 x 64: 7.6 against 10.6 us).
-    if (narrow && dir == kFwd && cache_resident && !(rope_heads == kRopeTokenHeads && kNarrowL[idx] == kRopeTokenMaxL))
-      rope_heads = 0;
+    // Token mode saves table look-ups, but its tiles are three times those of the look-up per row: on tensors
+    // that the caches hold, its forward waits for one tile a CU, and with four loads a wave it is slower
+    // throughout; its backward has fewer waves resident (237 registers against 138).  Kernel us per token | per row:
+    //   forward  24 heads of 128,   1 MB 4.7 | 3.8    4: 4.8 | 4.0    12: 5.5 | 6.2    32: 12.3 | 13.8    63: 23.7 | 24.6
+    //            12 of 128 (R = 3), 1: 4.0 | 3.6      4: 3.9 | 4.0    12: 6.1 | 6.2    32: 13.4 | 14.1    63: 25.4 | 25.2
+    //            16 of 128 (R = 4), 1: 4.1 | 3.5      4: 4.2 | 4.1    12: 5.9 | 6.0    32: 14.2 | 13.9    63: 27.9 | 24.6
+    //   backward 24 heads of 128,   1: 5.4 | 4.8      4: 5.7 | 5.4    12: 7.7 | 8.3    32: 19.4 | 17.5    63: 36.5 | 35.3
+    //            16 of 128,         1: 5.5 | 4.7      4: 5.6 | 5.2    12: 9.7 | 8.3    32: 19.7 | 17.5    63: 35.7 | 35.6
+    // (48 heads of 128 as 24; 64 columns as 128 with half the heads.  Beyond the caches: see rope_token_R.)
+    if (narrow && rope_heads > 0 && cache_resident) {
+      int cus = 0;
+      const int rc = current_device_cus(&cus);
+      if (rc != TT_OK) return rc;
+      const int r = rope_token_R(kNarrowL[idx], rope_heads);
+      if (dir == kBwd || r == 4 || rows < (int64_t)cus * rope_token_NW(r) * r * (kWave / kNarrowL[idx])) rope_heads = 0;
+    }
     k = rms_rope_kernel(narrow, dir == kBwd, idx, full, rope_heads);
   } else if (dir == kFwdXn) {
     if (kind != kAdaLN) return TT_ERR_UNSUPPORTED;

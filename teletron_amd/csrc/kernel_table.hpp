@@ -235,15 +235,15 @@ KernelInfo info_bwd_rope_narrow() {
 // token, so the (cos, sin) entries are loaded once per tile and lane).  R loads of 64 / L rows each have to
 // divide a token's heads: instantiated for rows of 8 and 16 lanes (head_dim 40 ... 128), the largest of
 // R = 6, 4, 3 that divides (24 heads of 128: 6, 16: 4, 12: 3; 24 heads of 64: 3).  Other head counts
-// look every row up (ROPE = 1, two loads).  us forward / backward + reduction, per row -> per token:
-// 2 x 60000 x 12 x 128 137 / 190 -> 127 / 184, 60000 x 16 x 128 92 / 128 -> 89 / 127, 2 x 60000 x 24 x 64
+// look every row up (ROPE = 1, two loads), and so do most tensors that fit the caches (make_plan).
+// us forward / backward + reduction, per row -> per token: 2 x 60000 x 12 x 128 137 / 190 -> 127 / 184, 60000 x 16 x 128 92 / 128 -> 89 / 127, 2 x 60000 x 24 x 64
 // 133 / 189 -> 127 / 183.  R = 5 is slower (60000 x 40 x 128 221 / 318 -> 227 / 321).
 // One workgroup per CU with about 24 loads per lane column and tensor in flight measured best (24
 // heads of 128, four waves of six: forward 245 us, backward + reduction 356 us at 118800 tokens; 5 / 6 / 8
 // waves: 277 / 265 / 267 us forward, 378 / 368 / 380 us backward; 2 and 3 waves need 2-3 workgroups per
 // CU and reach 259-265 us).
-constexpr int kRopeTokenMinL = 8, kRopeTokenMaxL = 16, kRopeTokenHeads = 24;   // 24 x 128: HunyuanVideo, at every size
-constexpr int rope_token_NW(int R) { return (24 + R / 2) / R; }
+constexpr int kRopeTokenMinL = 8, kRopeTokenMaxL = 16;
+constexpr int rope_token_NW(int R) { return R > 0 ? (24 + R / 2) / R : 0; }
 template <int L, int R, bool FULL>
 KernelInfo info_rope_token(bool backward) {
   constexpr int NW = rope_token_NW(R);
