@@ -1,9 +1,10 @@
 // Element-wise (16-bit load/store) kernels for what the vector kernels do not take: rows of at most
 // 256 values whose width is not a multiple of 8 or whose tensors are not 16-byte aligned, and the
 // backward of such rows where they are longer than 16384 values or the partial column sums would be
-// too large or do not fit the workspace (odd_plan in capi.hip).  Correctness path, not a bandwidth path: one 256-thread
-// workgroup per row, the row is re-read from cache for each pass, parameter gradients come from a
-// second kernel that walks the rows column by column with the row statistics saved by the first.
+// too large or do not fit the workspace (odd_plan in capi.hip).  Correctness path, not a bandwidth
+// path: one 256-thread workgroup per row, the row is re-read from cache for each pass, parameter
+// gradients come from a second kernel that walks the rows column by column with the row statistics
+// saved by the first.
 #pragma once
 #include "common.hpp"
 #include "norm_kernels.hpp"

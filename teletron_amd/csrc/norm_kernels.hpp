@@ -39,7 +39,7 @@ struct FwdArgs {
   int64_t rows_per_batch;
   int64_t n_tiles;  // tiles per batch
   int cols;
-  int packs;        // cols / 8
+  int packs;        // cols / 8, rounded up
   float eps;
   float inv_cols;
   // rotary embedding fused behind RMSNorm (ROPE kernels only): (cos, sin) per position and

@@ -3,7 +3,8 @@ every bit of the result depend on its arguments alone.  Tolerances as in test_gp
 import pytest
 import torch
 
-from test_gpu_parity import DEV, rand_bf16
+from test_gpu_configs import whole_tensor_check
+from test_gpu_parity import DEV, assert_grad_close, rand_bf16
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +95,56 @@ def test_static_backward_equals_the_workspace_backward(lib, nb, rpb, cols, shift
                                             w.data_ptr(), rows, cols, rpb, 1e-6, st) == 0
         torch.cuda.synchronize()
         assert torch.equal(a, b) and torch.equal(ga, gb)
+
+
+@pytest.mark.parametrize("rows,cols,shift", [(30000, 257, 0), (9000, 1001, 0), (7001, 4095, 0), (1300, 16383, 0), (9000, 1536, 3),
+                                             (140000, 257, 0), (36000, 1001, 0), (24000, 1536, 5), (2100, 16383, 0), (1100, 32767, 0)])
+def test_many_odd_rows(lib, rows, cols, shift):
+    """Several tiles a workgroup, in the caches and (from the sixth case) past the 64 MiB where the plans change:
+    every element against torch fp32 on the GPU, the parameter gradients against fp64 sums."""
+    from teletron_amd import ops
+    nb, eps = 2 if rows % 2 == 0 else 1, 1e-6
+    g = torch.Generator(device=DEV).manual_seed(cols)
+    x, dy = (shifted(torch.randn(rows, cols, generator=g, device=DEV).to(torch.bfloat16), shift) for _ in range(2))
+    p = (0.2 * torch.randn(2, nb, cols, generator=g, device=DEV)).to(torch.bfloat16)
+    w = (1 + p[0, 0].float()).to(torch.bfloat16)
+    group = torch.arange(rows, device=DEV) // (rows // nb)
+
+    y, mean, rstd = ops.adaln_forward(x, p[0], p[1], eps, return_stats=True)
+    yr = ops.rmsnorm_forward(x, w, eps)
+    y2, xn, inv = torch.empty_like(x), torch.empty_like(x), torch.empty(rows, device=DEV)
+    st = torch.cuda.current_stream().cuda_stream
+    assert lib.tt_launch_adaln_forward(y2.data_ptr(), xn.data_ptr(), x.data_ptr(), p[0, 0].data_ptr(), p[1, 0].data_ptr(),
+                                       rows, cols, eps, inv.data_ptr(), st) == 0
+    dx, ds, dh = ops.adaln_backward(dy, x, p[0], eps)
+    dxr, dw = ops.rmsnorm_backward(dy, x, w, eps)
+
+    def parts(r0, r1):
+        xs = x[r0:r1].float()
+        d = xs - xs.mean(-1, keepdim=True)
+        return d * torch.rsqrt(d.pow(2).mean(-1, keepdim=True) + eps), torch.rsqrt(d.pow(2).mean(-1, keepdim=True) + eps), \
+            xs * torch.rsqrt(xs.pow(2).mean(-1, keepdim=True) + eps), torch.rsqrt(xs.pow(2).mean(-1, keepdim=True) + eps)
+
+    def grad(r0, r1, k, gg):
+        xh, rs = parts(r0, r1)[k:k + 2]
+        return rs * (gg - (gg.mean(-1, keepdim=True) if k == 0 else 0) - xh * (gg * xh).mean(-1, keepdim=True))
+
+    scale, shift_ = 1 + p[0].float(), p[1].float()
+    whole_tensor_check(y, lambda a, b: parts(a, b)[0] * scale[group[a:b]] + shift_[group[a:b]])
+    whole_tensor_check(yr, lambda a, b: parts(a, b)[2] * w.float())
+    whole_tensor_check(xn, lambda a, b: parts(a, b)[0])
+    whole_tensor_check(y2, lambda a, b: parts(a, b)[0] * scale[0] + shift_[0])
+    whole_tensor_check(dx, lambda a, b: grad(a, b, 0, dy[a:b].float() * scale[group[a:b]]))
+    whole_tensor_check(dxr, lambda a, b: grad(a, b, 2, dy[a:b].float() * w.float()))
+    sums = torch.zeros(3, nb, cols, dtype=torch.float64, device=DEV)
+    for a in range(0, rows, 8192):
+        b = min(a + 8192, rows)
+        xh, rs, xr, _ = parts(a, b)
+        d = dy[a:b].double()
+        for i, t in enumerate((d * xh.double(), d, d * xr.double())):
+            sums[i].index_add_(0, group[a:b], t)
+        torch.testing.assert_close(rstd[a:b], rs[:, 0], rtol=1e-5, atol=0)
+    assert torch.equal(rstd, inv)
+    assert_grad_close(ds, sums[0].cpu(), rows, "dscale")
+    assert_grad_close(dh, sums[1].cpu(), rows, "dshift")
+    assert_grad_close(dw, sums[2].sum(0).cpu(), rows, "dweight")

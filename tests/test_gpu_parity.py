@@ -181,7 +181,7 @@ def test_eps_zero_with_ragged_row_tail(cols):
                       dy.reshape(-1, cols), 0.0, f"rmsnorm eps=0 [{nb * rpb},{cols}]")
 
 
-# ------------------------------------------------------------------ element-wise path: odd widths, misaligned tensors
+# ------------------------------------------------------------------ odd widths, misaligned tensors
 @pytest.mark.parametrize("cols", [1, 3, 7, 12, 100, 257, 1001, 5121])
 def test_widths_not_multiple_of_8(cols):
     x = rand_bf16(2, 37, cols, seed=cols, offset=0.25)
@@ -193,7 +193,7 @@ def test_widths_not_multiple_of_8(cols):
                   rand_bf16(53, cols, seed=cols + 6), 1e-6, f"rmsnorm odd width {cols}")
 
 
-def test_misaligned_tensors_take_the_elementwise_path():
+def test_misaligned_tensors_agree_with_aligned_ones():
     from teletron_amd import ops
     rows, cols = 129, 1024
     base = rand_bf16(rows * cols + 8, seed=50).to(DEV)
@@ -211,7 +211,7 @@ def test_misaligned_tensors_take_the_elementwise_path():
     assert_bf16_close(y, yo, "misaligned y")
     assert_bf16_close(dx, dxo, "misaligned dx")
     assert_grad_close(dw, dwo, rows, "misaligned dweight")
-    # both paths round the same fp32 formula: they agree to within one bf16 ulp
+    # both kernels round the same fp32 formula: they agree to within one bf16 ulp
     torch.testing.assert_close(y.float(), y2.float(), rtol=8e-3, atol=1e-3)
     torch.testing.assert_close(dx.float(), dx2.float(), rtol=8e-3, atol=2e-3)
     torch.testing.assert_close(dw, dw2, rtol=1e-3, atol=1e-3)

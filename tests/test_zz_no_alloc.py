@@ -99,12 +99,12 @@ def test_static_backward_matches_workspace_backward_twice():
     print("case: tt_adaln_backward_static rows=6000 cols=5120 batches=2, then rows=1201 cols=1536 batches=1", flush=True)
     _run(6000, 5120, 2, seed=11)
     _run(1201, 1536, 1, seed=12)     # smaller input, same device array
-    _run(77, 1000, 1, seed=13)       # ragged width (masked kernel variant)
+    _run(77, 1000, 1, seed=13)       # ragged width
 
 
 def test_static_backward_on_the_element_wise_path():
-    """Widths that are not a multiple of 8 take the element-wise kernels, which keep two floats per
-    row in the scratch array: bit-equal where rows * 8 bytes fit, TT_ERR_STATIC_LIMIT where not."""
+    """Widths that are not a multiple of 8: 1001 runs on vector kernels, 77 and 9 on element-wise ones, which keep two
+    floats per row in the scratch array.  Bit-equal where rows * 8 bytes fit, TT_ERR_STATIC_LIMIT where not."""
     print("case: tt_adaln_backward_static rows=4000 cols=1001 batches=2, then rows=2200000 cols=9", flush=True)
     _run(4000, 1001, 2, seed=14)
     _run(513, 77, 1, seed=15)
