@@ -575,7 +575,7 @@ const char* tt_error_string(int code) {
     case TT_ERR_UNSUPPORTED: return "unsupported shape or alignment";
     case TT_ERR_WORKSPACE: return "workspace missing, misaligned or too small";
     case TT_ERR_HIP: return "HIP runtime error (see tt_last_hip_error)";
-    case TT_ERR_STATIC_LIMIT: return "shape needs more than TT_STATIC_WORKSPACE_BYTES of scratch (partial sums, or rows * 8 bytes on the element-wise path): use the entry point that takes a workspace";
+    case TT_ERR_STATIC_LIMIT: return "shape needs more than TT_STATIC_WORKSPACE_BYTES of scratch (partial sums, or rows * 8 bytes where cols % 8 != 0 or a tensor is misaligned): use the entry point that takes a workspace";
     default: return "unknown error code";
   }
 }

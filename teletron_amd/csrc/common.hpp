@@ -46,7 +46,7 @@ __device__ __forceinline__ u32x4 load_cached(const void* base, size_t elem_off) 
 
 // How the rows of a wide kernel lie on its lane slots and in memory.
 enum Rows : int {
-  kMasked = 0,   // fewer packs than lane slots; a row is a whole number of 128-byte lines
+  kMasked = 0,   // fewer packs than lane slots; a row is a whole number of 128-byte lines (x_norm forward: any)
   kFull = 1,     // every lane slot holds a pack
   kRagged = 2,   // as kMasked, but rows start anywhere inside a line (cols % 64 != 0)
   kOdd = 3,      // any row length and 2-byte aligned tensors; the last pack may be short

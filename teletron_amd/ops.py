@@ -203,7 +203,7 @@ class _Workspace:
 
 _WORKSPACES = {}   # (device index, stream handle) -> _Workspace
 _WORKSPACES_LOCK = threading.Lock()   # backward runs on autograd's threads, one per device
-# the element-wise path's row statistics (rows * 8 bytes) are only kept between calls up to this size
+# larger ones (the partial sums of thousands of modulation vectors, the row statistics of very short rows) are not kept
 _WORKSPACE_KEEP_BYTES = 64 << 20
 
 
