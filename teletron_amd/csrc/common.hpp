@@ -40,6 +40,11 @@ __device__ __forceinline__ void store_stream2(void* base0, void* base1, size_t e
   asm volatile("s_nop 3\n\tglobal_store_dwordx4 %0, %2, off sc0 sc1 nt\n\t"
                "global_store_dwordx4 %1, %3, off sc0 sc1 nt\n\ts_nop 3" ::"v"(p0), "v"(p1), "v"(v0), "v"(v1) : "memory");
 }
+// Values that the next kernel reads, perhaps on another XCD: written through to where all XCDs see them
+// (device scope), but cached there.
+__device__ __forceinline__ void store_agent(float* p, f32x4 v) {
+  asm volatile("s_nop 3\n\tglobal_store_dwordx4 %0, %1, off sc1\n\ts_nop 3" ::"v"(p), "v"(v) : "memory");
+}
 __device__ __forceinline__ u32x4 load_cached(const void* base, size_t elem_off) {
   return *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(base) + elem_off);
 }

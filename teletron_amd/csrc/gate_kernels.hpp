@@ -37,7 +37,7 @@ __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
 
   int col[P];
   bool act[P];
-  float g[P][8], acc0[P][8], acc1[P][8];
+  float g[P][8], acc[1][P][8];
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     const int pk = p * 64 * W + w * 64 + lane;
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
     }
     unpack8(r0, g[p]);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) { acc0[p][j] = 0.f; acc1[p][j] = 0.f; }
+    for (int j = 0; j < 8; ++j) acc[0][p][j] = 0.f;
   }
 
   u32x4 rawa[R][P], rawb[R][P];
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
             o[j] = fmaf(g[p][j], bf[r][p][j], af[r][p][j]);
           } else {
             o[j] = af[r][p][j] * g[p][j];
-            acc0[p][j] = fmaf(af[r][p][j], bf[r][p][j], acc0[p][j]);
+            acc[0][p][j] = fmaf(af[r][p][j], bf[r][p][j], acc[0][p][j]);
           }
         }
         if (row0 + r < S) store_row<ROWS, SHORT>(a.out, pack_offset<ROWS, W>(row, C, col[p], a.packs, (p * W + w) * 64 + lane), act[p], a.packs - (p * W + w) * 64, lane, pack8(o));
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
     }
   }
   if constexpr (MODE == kGateBwd)
-    wide_write_partials<false, W, P, Q>(acc0, acc1, act, col, a.partials, b, C, q, w, lane);
+    wide_write_partials<1, W, P, Q>(acc, a.partials, b, C, q, w, lane);
 }
 
 template <int MODE, int L, int R, int NW, bool FULL>

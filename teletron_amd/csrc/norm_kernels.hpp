@@ -340,59 +340,45 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
   }
 }
 
-// Epilogue of the wide backward kernels: fold the Q row groups of the workgroup into
-// group 0 (in group order, through LDS) and write the workgroup's partial column sums.
-template <bool ADALN, int W, int P, int Q, bool ODD = false>
-__device__ __forceinline__ void wide_write_partials(float (&acc0)[P][8], float (&acc1)[P][8], const bool (&act)[P],
-                                                    const int (&col)[P], float* partials, int64_t b, int C,
+// Epilogue of the wide backward kernels: the workgroup's partial column sums, the Q row groups added in
+// group order.  All groups lay their sums out in LDS as they lie in the row, so that every wave then adds
+// and stores whole cache lines, 16 bytes a lane.
+// What bounds it: 256 workgroups write 5 to 15 MB at once while nothing else is left to do, and dirty lines
+// in the L2 hold up the end of the kernel.  Hence written through to device scope, but not past the caches, from
+// which reduce_partials reads it next.  Backward + reduction, us, one group storing 32 bytes a lane with plain stores ->
+// this: AdaLN 512 x 5120 11.4 + 4.6 -> 9.2 + 4.4, 1500 x 5120 15.9 + 4.2 -> 14.1 + 4.0, RMSNorm 512 x 5120 7.2 + 3.6 ->
+// 6.2 + 3.6, residual + norm 1300 x 3072 16.6 + 6.2 -> 14.3 + 5.4.  Laid out like this but with plain stores 10.4 + 3.8,
+// with non-temporal ones ("sc1 nt") 9.2 + 5.7 in the first of these.
+template <int NACC, int W, int P, int Q, bool ODD = false>
+__device__ __forceinline__ void wide_write_partials(const float (&acc)[NACC][P][8], float* partials, int64_t b, int C,
                                                     int q, int w, int lane) {
-  constexpr int NACC = ADALN ? 2 : 1;
-  __shared__ __attribute__((aligned(16))) float comb[Q > 1 ? 64 * W * P * 8 : 4];
-  if constexpr (Q > 1) {
+  constexpr int SLOTS = 64 * W * P;   // of a row group: slot = pack of the row
+  __shared__ __attribute__((aligned(16))) float comb[Q][SLOTS * kPack];
+  float* base = partials + ((size_t)(b * gridDim.x + blockIdx.x) * NACC) * C;
 #pragma unroll
-    for (int acc = 0; acc < NACC; ++acc) {
-      for (int qq = 1; qq < Q; ++qq) {
-        __syncthreads();
-        if (q == qq) {
-#pragma unroll
-          for (int p = 0; p < P; ++p)
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-              comb[((p * W + w) * 64 + lane) * 8 + j] = acc == 0 ? acc0[p][j] : acc1[p][j];
-        }
-        __syncthreads();
-        if (q == 0) {
-#pragma unroll
-          for (int p = 0; p < P; ++p)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              const float t = comb[((p * W + w) * 64 + lane) * 8 + j];
-              if (acc == 0) acc0[p][j] += t; else acc1[p][j] += t;
-            }
-        }
-      }
-    }
-  }
-  if (q == 0) {
-    float* base = partials + ((size_t)(b * gridDim.x + blockIdx.x) * NACC) * C;
+  for (int n = 0; n < NACC; ++n) {
+    if (n > 0) __syncthreads();
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      if constexpr (ODD) {
+      f32x4* d = reinterpret_cast<f32x4*>(&comb[q][((p * W + w) * 64 + lane) * kPack]);
+      d[0] = f32x4{acc[n][p][0], acc[n][p][1], acc[n][p][2], acc[n][p][3]};
+      d[1] = f32x4{acc[n][p][4], acc[n][p][5], acc[n][p][6], acc[n][p][7]};
+    }
+    __syncthreads();
+    float* out = base + (size_t)n * C;
+    if constexpr (ODD) {
+      for (int c = threadIdx.x; c < C; c += 64 * W * Q) {
+        float t = comb[0][c];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (col[p] + j < C) {
-            base[col[p] + j] = acc0[p][j];
-            if constexpr (ADALN) base[C + col[p] + j] = acc1[p][j];
-          }
-      } else if (act[p]) {
-        f32x4* d0 = reinterpret_cast<f32x4*>(base + col[p]);
-        d0[0] = f32x4{acc0[p][0], acc0[p][1], acc0[p][2], acc0[p][3]};
-        d0[1] = f32x4{acc0[p][4], acc0[p][5], acc0[p][6], acc0[p][7]};
-        if constexpr (ADALN) {
-          f32x4* d1 = reinterpret_cast<f32x4*>(base + C + col[p]);
-          d1[0] = f32x4{acc1[p][0], acc1[p][1], acc1[p][2], acc1[p][3]};
-          d1[1] = f32x4{acc1[p][4], acc1[p][5], acc1[p][6], acc1[p][7]};
-        }
+        for (int qq = 1; qq < Q; ++qq) t += comb[qq][c];
+        out[c] = t;
+      }
+    } else {
+      for (int c = threadIdx.x * 4; c < C; c += 256 * W * Q) {
+        f32x4 t = *reinterpret_cast<const f32x4*>(&comb[0][c]);
+#pragma unroll
+        for (int qq = 1; qq < Q; ++qq) t += *reinterpret_cast<const f32x4*>(&comb[qq][c]);
+        store_agent(out + c, t);
       }
     }
   }
@@ -420,8 +406,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
   bool act[P];
   const int drop = ODD ? a.packs * kPack - C : 0;   // as in the forward kernel
   float g[P][8];
-  float acc0[P][8];  // dscale / dgamma
-  float acc1[P][8];  // dshift (AdaLN only)
+  float acc[NACC][P][8];   // dscale / dgamma, dshift (AdaLN only)
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     const int pk = p * 64 * W + w * 64 + lane;
@@ -434,8 +419,8 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       if constexpr (ADALN) g[p][j] += 1.0f;
-      acc0[p][j] = 0.f;
-      acc1[p][j] = 0.f;
+#pragma unroll
+      for (int k = 0; k < NACC; ++k) acc[k][p][j] = 0.f;
     }
   }
 
@@ -571,8 +556,8 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
         for (int j = 0; j < 8; ++j) {
           const float xh = xf[r][p][j] * rstd;
           const float dyv = df[r][p][j];
-          acc0[p][j] = fmaf(dyv, xh, acc0[p][j]);
-          if constexpr (ADALN) acc1[p][j] += dyv;
+          acc[0][p][j] = fmaf(dyv, xh, acc[0][p][j]);
+          if constexpr (ADALN) acc[NACC - 1][p][j] += dyv;
           o[j] = fmaf(xh, k2, fmaf(dyv * g[p][j], rstd, k1));
         }
         if constexpr (ODD) {
@@ -582,7 +567,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
     }
   }
 
-  wide_write_partials<ADALN, W, P, Q, ODD>(acc0, acc1, act, col, a.partials, b, C, q, w, lane);
+  wide_write_partials<NACC, W, P, Q, ODD>(acc, a.partials, b, C, q, w, lane);
 }
 
 // Position of a row for the narrow ROPE kernels: one row is one head, `rows_per_pos` consecutive
@@ -920,6 +905,7 @@ struct BwdSavedArgs {
 template <int KIND, int W, int P, int R, int Q, bool FULL>
 __global__ __launch_bounds__(64 * W * Q) void norm_bwd_saved_wide(const BwdSavedArgs a) {
   constexpr bool ADALN = (KIND == kAdaLN);
+  constexpr int NACC = ADALN ? 2 : 1;
   constexpr int NV = ADALN ? 2 : 1;
   __shared__ float red[2][Q][W * R * NV];
 
@@ -935,7 +921,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_saved_wide(const BwdSaved
   bool act[P];
   float g[P][8];    // 1 + scale, or weight
   float gi[P][8];   // RMSNorm: 1 / weight (x_hat = y / weight); 0 on masked lanes
-  float acc0[P][8], acc1[P][8];
+  float acc[NACC][P][8];
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     const int pk = p * 64 * W + w * 64 + lane;
@@ -948,8 +934,8 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_saved_wide(const BwdSaved
     for (int j = 0; j < 8; ++j) {
       if constexpr (ADALN) g[p][j] += 1.0f;
       gi[p][j] = (!ADALN && act[p]) ? 1.0f / g[p][j] : 0.f;
-      acc0[p][j] = 0.f;
-      acc1[p][j] = 0.f;
+#pragma unroll
+      for (int k = 0; k < NACC; ++k) acc[k][p][j] = 0.f;
     }
   }
 
@@ -1025,15 +1011,15 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_saved_wide(const BwdSaved
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const float dyv = df[r][p][j];
-          acc0[p][j] = fmaf(dyv, xh[r][p][j], acc0[p][j]);
-          if constexpr (ADALN) acc1[p][j] += dyv;
+          acc[0][p][j] = fmaf(dyv, xh[r][p][j], acc[0][p][j]);
+          if constexpr (ADALN) acc[NACC - 1][p][j] += dyv;
           o[j] = fmaf(xh[r][p][j], k2, fmaf(dyv * g[p][j], rstd[r], k1));
         }
         if (rv[r] && act[p]) store_stream(a.dx, (size_t)(row * C + col[p]), pack8(o));
       }
     }
   }
-  wide_write_partials<ADALN, W, P, Q>(acc0, acc1, act, col, a.partials, b, C, q, w, lane);
+  wide_write_partials<NACC, W, P, Q>(acc, a.partials, b, C, q, w, lane);
 }
 
 template <int KIND, int L, int R, int NW, bool FULL>

@@ -66,48 +66,6 @@ struct ResBwdArgs {
   float one;
 };
 
-// Epilogue: fold the Q row groups of the workgroup into group 0 (group order, through LDS) and
-// write the workgroup's NACC partial column sums.
-template <int NACC, int W, int P, int Q>
-__device__ __forceinline__ void wide_write_partials_n(float (&acc)[NACC][P][8], const bool (&act)[P], const int (&col)[P],
-                                                      float* partials, int64_t b, int C, int q, int w, int lane) {
-  __shared__ __attribute__((aligned(16))) float comb[Q > 1 ? 64 * W * P * 8 : 4];
-  if constexpr (Q > 1) {
-#pragma unroll
-    for (int n = 0; n < NACC; ++n) {
-      for (int qq = 1; qq < Q; ++qq) {
-        __syncthreads();
-        if (q == qq) {
-#pragma unroll
-          for (int p = 0; p < P; ++p)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) comb[((p * W + w) * 64 + lane) * 8 + j] = acc[n][p][j];
-        }
-        __syncthreads();
-        if (q == 0) {
-#pragma unroll
-          for (int p = 0; p < P; ++p)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc[n][p][j] += comb[((p * W + w) * 64 + lane) * 8 + j];
-        }
-      }
-    }
-  }
-  if (q == 0) {
-    float* base = partials + ((size_t)(b * gridDim.x + blockIdx.x) * NACC) * C;
-#pragma unroll
-    for (int n = 0; n < NACC; ++n)
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-        if (act[p]) {
-          f32x4* d = reinterpret_cast<f32x4*>(base + (size_t)n * C + col[p]);
-          d[0] = f32x4{acc[n][p][0], acc[n][p][1], acc[n][p][2], acc[n][p][3]};
-          d[1] = f32x4{acc[n][p][4], acc[n][p][5], acc[n][p][6], acc[n][p][7]};
-        }
-      }
-  }
-}
-
 // ============================================================================ forward
 template <int W, int P, int R, int Q, int ROWS, bool GATED>
 __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs a) {
@@ -407,7 +365,7 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_bwd_wide(const ResBwdArgs 
     }
   }
 
-  wide_write_partials_n<NACC, W, P, Q>(acc, act, col, a.partials, b, C, q, w, lane);
+  wide_write_partials<NACC, W, P, Q>(acc, a.partials, b, C, q, w, lane);
 }
 
 }  // namespace tt
