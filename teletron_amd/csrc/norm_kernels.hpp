@@ -1113,17 +1113,23 @@ __global__ __launch_bounds__(64 * NW) void norm_bwd_saved_narrow(const BwdSavedA
 }
 
 // ============================================================================ second pass
-// out[acc][b][c] = sum_j partials[b][j][acc][c], j in a fixed order: 16 waves take
-// the partials j = wave, wave+16, ... and are then folded in wave order through LDS.
-// The output is fp32, or bf16 (rounded once) when out_bf16 is set.
-template <int NACC>
+// out[acc][b][c] = sum_j partials[b][j][acc][c], j in a fixed order.  A workgroup takes LC columns; each LC lanes
+// of it take the partials j = slot, slot + SLOTS, ..., and the slots are folded inside the wave and then in wave
+// order through LDS.  The output is fp32, or bf16 (rounded once) when out_bf16 is set.
+// Bound by the latency of its few dependent steps, not by the 0.1 to 15 MB it reads: 32 columns a workgroup instead of 64
+// give twice the workgroups and the loads of 256 partials in one round.  us at 64 -> 32 -> 16 columns: 512 partials
+// of 2 x 3072 sums 5.5 -> 4.3 -> 6.1, 256 of 3 x 5120 5.3 -> 4.7 -> 8.7, 768 of 128 4.8 -> 3.9 -> 4.0; 256 of 1536 to 5120
+// 3.9 either way.  (16 columns are half a cache line, which two workgroups then fetch.)
+template <int NACC, int LC>
 __global__ __launch_bounds__(1024) void reduce_partials(void* __restrict__ out0, void* __restrict__ out1,
                                                         void* __restrict__ out2, const float* __restrict__ partials,
                                                         int n_partials, int cols, int out_bf16) {
-  __shared__ float fold[16][NACC][64];
+  constexpr int SLOTS = 16 * 64 / LC;
+  __shared__ float fold[16][NACC][LC];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + lane;
+  const int cl = lane & (LC - 1);
+  const int c = blockIdx.x * LC + cl;
   const int64_t b = blockIdx.y;
   float s[NACC];
 #pragma unroll
@@ -1132,13 +1138,13 @@ __global__ __launch_bounds__(1024) void reduce_partials(void* __restrict__ out0,
     const float* base = partials + (size_t)b * n_partials * NACC * cols + c;
     // 8 independent loads per accumulator in flight, in the ragged last round too (a missing
     // partial contributes +0.0f, which changes no sum); the sum order stays fixed.
-    for (int j = wave; j < n_partials; j += 8 * 16) {
+    for (int j = wave * (64 / LC) + lane / LC; j < n_partials; j += 8 * SLOTS) {
       float t[8][NACC];
 #pragma unroll
       for (int u = 0; u < 8; ++u)
 #pragma unroll
         for (int acc = 0; acc < NACC; ++acc)
-          t[u][acc] = j + u * 16 < n_partials ? base[((size_t)(j + u * 16) * NACC + acc) * cols] : 0.f;
+          t[u][acc] = j + u * SLOTS < n_partials ? base[((size_t)(j + u * SLOTS) * NACC + acc) * cols] : 0.f;
 #pragma unroll
       for (int u = 0; u < 8; ++u)
 #pragma unroll
@@ -1146,13 +1152,18 @@ __global__ __launch_bounds__(1024) void reduce_partials(void* __restrict__ out0,
     }
   }
 #pragma unroll
-  for (int acc = 0; acc < NACC; ++acc) fold[wave][acc][lane] = s[acc];
-  __syncthreads();
-  if (wave < NACC && c < cols) {
-    float t = fold[0][wave][lane];
+  for (int acc = 0; acc < NACC; ++acc) {
 #pragma unroll
-    for (int ww = 1; ww < 16; ++ww) t += fold[ww][wave][lane];
-    void* out = wave == 0 ? out0 : wave == 1 ? out1 : out2;
+    for (int m = LC; m < 64; m <<= 1) s[acc] += __shfl_xor(s[acc], m, 64);
+    if (lane < LC) fold[wave][acc][cl] = s[acc];
+  }
+  __syncthreads();
+  const int acc = threadIdx.x / LC;
+  if (acc < NACC && c < cols) {
+    float t = fold[0][acc][cl];
+#pragma unroll
+    for (int ww = 1; ww < 16; ++ww) t += fold[ww][acc][cl];
+    void* out = acc == 0 ? out0 : acc == 1 ? out1 : out2;
     const size_t idx = (size_t)b * cols + c;
     if (out_bf16) static_cast<uint16_t*>(out)[idx] = f32_to_bf16(t);
     else          static_cast<float*>(out)[idx] = t;

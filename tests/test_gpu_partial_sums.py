@@ -53,3 +53,20 @@ def test_gate_and_residual_gradients(cols):
     dx = ds.double() + rstd * (g - g.mean(-1, keepdim=True) - xh * (g * xh).mean(-1, keepdim=True))
     for got, ref, name in ((dscale, d * xh, "dscale"), (dshift, d, "dshift"), (dgate, dx * r.double(), "dgate of the update")):
         assert_grad_close(got, ref.sum(0).cpu(), rows, name)
+
+
+# rounds of 8 x 16 and 8 x 32 partials, a last one of a single partial, column counts beside whole workgroups of 32 and 64
+@pytest.mark.parametrize("n_partials", [1, 31, 33, 256, 257, 777])
+@pytest.mark.parametrize("n_batches,cols", [(1, 1), (1, 33), (1, 128), (1, 5128), (2, 8191), (3, 5120), (300, 72), (70, 300)])
+@pytest.mark.parametrize("n_acc", [1, 2])
+def test_reduction(lib, n_partials, n_batches, cols, n_acc):
+    """Any order of n additions is off by at most n 2^-24 sum |x|."""
+    g = torch.Generator(device=DEV).manual_seed(n_partials + cols)
+    ws = torch.randn(n_batches, n_partials, n_acc, cols, generator=g, device=DEV)
+    out = torch.full((n_acc, n_batches, cols), float("nan"), device=DEV)
+    assert lib.tt_reduce_partials(out[0].data_ptr(), out[1].data_ptr() if n_acc == 2 else None, ws.data_ptr(), n_batches,
+                                  n_partials, n_acc, cols, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    d = ws.double()
+    err = (out.double().transpose(0, 1) - d.sum(1)).abs()
+    assert (err <= n_partials * 2.0 ** -24 * d.abs().sum(1)).all()
