@@ -113,8 +113,11 @@ struct Plan {
   KernelInfo k;
   int64_t n_batches = 0;
   int64_t n_tiles = 0;   // per batch
-  int grid_x = 0;        // workgroups per batch == partial sums per batch
+  int grid_x = 0;        // most workgroups per batch: what workspaces are sized for
+  int max_x = 0;         // workgroups per batch that are launched at most, 0: grid_x
   int packs = 0;
+  // workgroups per batch that are launched == partial sums per batch
+  int grid() const { return max_x && max_x < grid_x ? max_x : grid_x; }
 };
 
 enum Dir { kFwd, kBwd, kBwdSaved, kFwdXn };   // kFwdXn: AdaLN forward that also stores x_norm
@@ -203,6 +206,17 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   const int ov = g_wgs_per_cu_override.load(std::memory_order_relaxed);
   if (ov > 0) per_cu = ov;
   if (per_cu > kMaxWgsPerCu) per_cu = kMaxWgsPerCu;
+
+  // The backward kernels of wide rows leave partial sums of 4 to 12 bytes a column and workgroup, which on tensors
+  // that the caches hold cost more than a second workgroup on the CU gives: one a CU.  Kernel us, two -> one, backward +
+  // reduction: saved AdaLN 1692 x 3072 14.3 + 4.4 -> 10.8 + 3.2, 9000 x 3072 32.7 + 4.8 -> 30.4 + 4.7, AdaLN 1200 x 5128
+  // 18.1 + 6.7 -> 15.5 + 4.3, residual + norm 1300 x 3072 14.1 + 4.4 -> 11.0 + 3.9, gate 1222 x 3536 8.9 + 3.8 -> 8.2 + 3.1,
+  // RMSNorm 3000 x 3072 15.3 + 3.8 -> 13.6 + 3.8, with the rotary embedding 5000 x 3072 23.7 + 3.9 -> 21.2 + 3.9.
+  // Not where over a quarter of the lanes are idle: one workgroup then has too little in flight (RMSNorm 19660 x 640
+  // 17.9 -> 19.7 with the reduction), nor for narrow rows, whose partial sums are small (40 heads of 128 x 3000 17 -> 22).
+  // Workspaces stay sized for grid_x, so that sizes asked for once hold.
+  if (ov <= 0 && cache_resident && !narrow && (dir == kBwd || dir == kBwdSaved) && packs * 4 >= slots * 3)
+    plan->max_x = rows / rows_per_batch < cus ? (int)(cus / (rows / rows_per_batch)) : 1;
 
   plan->k = k;
   plan->packs = packs;
@@ -328,7 +342,7 @@ size_t workspace_for(int kind, int n_acc, int64_t rows, int64_t cols, int64_t ro
 template <typename Args>
 int launch(const Plan& p, Args& args, void* stream) {
   void* kargs[] = {&args};
-  hipError_t e = hipLaunchKernel(p.k.fn, dim3(p.grid_x, (unsigned)p.n_batches, 1), dim3(p.k.threads, 1, 1),
+  hipError_t e = hipLaunchKernel(p.k.fn, dim3(p.grid(), (unsigned)p.n_batches, 1), dim3(p.k.threads, 1, 1),
                                  kargs, 0, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e);
   return TT_OK;
@@ -409,7 +423,7 @@ int backward_generic(int kind, void* dx, void* out0, void* out1, const void* dy,
       b.cols = (int)cols; b.packs = p.packs; b.eps = eps; b.inv_cols = 1.0f / (float)cols;
       rc = launch(p, b, stream);
       if (rc != TT_OK) return rc;
-      return reduce(out0, out1, workspace, (int)p.n_batches, p.grid_x, n_acc, cols, out_bf16, stream);
+      return reduce(out0, out1, workspace, (int)p.n_batches, p.grid(), n_acc, cols, out_bf16, stream);
     }
   }
   int grid = 0;
@@ -516,7 +530,7 @@ int backward_partials(int kind, void* dx, const void* dy, const void* x, const v
   a.rows_per_batch = rows_per_batch; a.n_tiles = p.n_tiles;
   a.cols = (int)cols; a.packs = p.packs; a.eps = eps; a.inv_cols = 1.0f / (float)cols;
   rc = launch(p, a, stream);
-  if (rc == TT_OK && n_partials) *n_partials = p.grid_x;
+  if (rc == TT_OK && n_partials) *n_partials = p.grid();
   return rc;
 }
 
@@ -537,7 +551,7 @@ int backward_saved_partials(int kind, void* dx, const void* dy, const void* xs, 
   a.rows_per_batch = rows; a.n_tiles = p.n_tiles;
   a.cols = (int)cols; a.packs = p.packs; a.inv_cols = 1.0f / (float)cols;
   rc = launch(p, a, stream);
-  if (rc == TT_OK) *n_partials = p.grid_x;
+  if (rc == TT_OK) *n_partials = p.grid();
   return rc;
 }
 
@@ -792,7 +806,7 @@ int tt_gate_residual_backward_typed(void* dresidual, void* dgate, int grads_bf16
   a.rows_per_batch = rows_per_batch; a.n_tiles = p.n_tiles; a.cols = (int)cols; a.packs = p.packs;
   rc = launch(p, a, stream);
   if (rc != TT_OK) return rc;
-  return reduce(dgate, nullptr, workspace, (int)(rows / rows_per_batch), p.grid_x, 1, cols, grads_bf16 != 0, stream);
+  return reduce(dgate, nullptr, workspace, (int)(rows / rows_per_batch), p.grid(), 1, cols, grads_bf16 != 0, stream);
 }
 
 int tt_gate_residual_backward(void* dresidual, float* dgate, const void* dout, const void* gate,
@@ -874,7 +888,7 @@ int tt_residual_norm_backward_typed(void* dx, void* dr, void* dscale, void* dshi
   a.cols = (int)cols; a.packs = p.packs; a.eps = eps; a.inv_cols = 1.0f / (float)cols; a.one = affine ? 0.f : 1.f;
   rc = launch(p, a, stream);
   if (rc != TT_OK) return rc;
-  return reduce(dscale, dshift, workspace, (int)p.n_batches, p.grid_x, n_acc, cols, grads_bf16 != 0, stream, dgate);
+  return reduce(dscale, dshift, workspace, (int)p.n_batches, p.grid(), n_acc, cols, grads_bf16 != 0, stream, dgate);
 }
 
 int tt_residual_norm_backward(void* dx, void* dr, float* dscale, float* dshift, float* dgate,
