@@ -3,5 +3,5 @@
 #include "kernel_table.hpp"
 
 namespace tt {
-KernelInfo adaln_bwd_saved_kernel(bool narrow, int idx, bool full) { return lookup_bwd_saved<kAdaLN>(narrow, idx, full); }
+KernelInfo adaln_bwd_saved_kernel(bool narrow, int idx, int rows) { return lookup_bwd_saved<kAdaLN>(narrow, idx, rows); }
 }  // namespace tt

@@ -146,11 +146,8 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   // a row of whole 128-byte lines or not: see enum Rows
   const int mode = odd ? kOdd : full ? kFull : (cols * 2) % 128 == 0 || force == kMasked ? kMasked : kRagged;
   const bool cache_resident = rows * cols * 2 < (int64_t)64 << 20;
-  KernelInfo k;
-  if (res) {
-    if (narrow || kind != kAdaLN || dir == kBwdSaved || dir == kFwdXn) return TT_ERR_UNSUPPORTED;
-    k = res == 2 ? resnorm_gated_kernel(dir == kBwd, idx, mode) : resnorm_plain_kernel(dir == kBwd, idx, mode);
-  } else if (rope) {
+  if (res && (narrow || kind != kAdaLN || dir == kBwdSaved || dir == kFwdXn)) return TT_ERR_UNSUPPORTED;
+  if (rope) {
     if (kind != kRMS || dir == kBwdSaved || dir == kFwdXn) return TT_ERR_UNSUPPORTED;
     // Token mode saves table look-ups, but its tiles are three times those of the look-up per row: on tensors
     // that the caches hold, its forward waits for one tile a CU, and with four loads a wave it is slower
@@ -168,18 +165,22 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
       const int r = rope_token_R(kNarrowL[idx], rope_heads);
       if (dir == kBwd || r == 4 || rows < (int64_t)cus * rope_token_NW(r) * r * (kWave / kNarrowL[idx])) rope_heads = 0;
     }
-    k = rms_rope_kernel(narrow, dir == kBwd, idx, full, rope_heads);
-  } else if (dir == kFwdXn) {
-    if (kind != kAdaLN) return TT_ERR_UNSUPPORTED;
-    k = adaln_fwd_xnorm_kernel(narrow, idx, odd ? kOdd : full ? kFull : kMasked);
-  } else if (kind == kAdaLN)
-    k = dir == kFwd ? adaln_fwd_kernel(narrow, idx, mode)
-      : dir == kBwd ? adaln_bwd_kernel(narrow, idx, mode) : adaln_bwd_saved_kernel(narrow, idx, full);
-  else if (kind == kRMS)
-    k = dir == kFwd ? rms_fwd_kernel(narrow, idx, mode)
-      : dir == kBwd ? rms_bwd_kernel(narrow, idx, mode) : rms_bwd_saved_kernel(narrow, idx, full);
-  else
-    k = dir == kFwd ? gate_fwd_kernel(narrow, idx, mode) : gate_bwd_kernel(narrow, idx, mode);
+  }
+  if (dir == kFwdXn && kind != kAdaLN) return TT_ERR_UNSUPPORTED;
+  const auto pick = [&](int rows_kind) -> KernelInfo {
+    if (res == 2) return resnorm_gated_kernel(dir == kBwd, idx, rows_kind);
+    if (res) return resnorm_plain_kernel(dir == kBwd, idx, rows_kind);
+    if (rope) return rms_rope_kernel(narrow, dir == kBwd, idx, rows_kind, rope_heads);
+    if (dir == kFwdXn) return adaln_fwd_xnorm_kernel(narrow, idx, rows_kind);
+    if (kind == kAdaLN)
+      return dir == kFwd ? adaln_fwd_kernel(narrow, idx, rows_kind)
+           : dir == kBwd ? adaln_bwd_kernel(narrow, idx, rows_kind) : adaln_bwd_saved_kernel(narrow, idx, rows_kind);
+    if (kind == kRMS)
+      return dir == kFwd ? rms_fwd_kernel(narrow, idx, rows_kind)
+           : dir == kBwd ? rms_bwd_kernel(narrow, idx, rows_kind) : rms_bwd_saved_kernel(narrow, idx, rows_kind);
+    return dir == kFwd ? gate_fwd_kernel(narrow, idx, rows_kind) : gate_bwd_kernel(narrow, idx, rows_kind);
+  };
+  const KernelInfo k = pick(mode);
   if (!k.fn) return TT_ERR_UNSUPPORTED;
 
   int cus = 0, per_cu = 0;
@@ -218,7 +219,16 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   if (ov <= 0 && cache_resident && !narrow && (dir == kBwd || dir == kBwdSaved) && packs * 4 >= slots * 3)
     plan->max_x = rows / rows_per_batch < cus ? (int)(cus / (rows / rows_per_batch)) : 1;
 
-  plan->k = k;
+  // Tensors that fit the caches are read with ordinary loads (kKeep; the plan is that of the other kernel).  As fast
+  // as streaming loads on inputs that no cache holds, and the next kernel to read them finds them there (forward, then
+  // backward, three sets of tensors in turn; kernel us, streaming -> kept, forward and backward): AdaLN 1500 x 5120 7.6 / 14.0
+  // -> 6.6 / 11.0, 5000 x 4096 16.1 / 24.5 -> 12.9 / 21.8, RMSNorm 5000 x 1536 7.6 / 11.6 -> 6.2 / 9.4, gate 2500 x 3072 10.4 / 10.4
+  // -> 8.8 / 6.2, 6000 x 4096 25.3 / 24.5 -> 24.5 / 23.5, residual + norm 2000 x 3072 11.9 / 17.0 -> 9.4 / 14.1.  With more tensors
+  // a call the limit is lower: residual + norm 2605 x 5120 21.4 / 24.4 -> 21.8 / 24.4, 6000 x 4096 33.4 / 35.8 -> 34.2 / 37.2, x_norm
+  // forward and its backward 4972 x 3072 18.1 / 21.8 -> 17.0 / 20.9, 9000 x 3072 31.0 / 32.4 -> 30.8 / 33.4; gated, 4000 x 3072
+  // 18.8 / 29.1 -> 18.6 / 29.1.  Beyond the caches streaming is the faster (75600 x 5120 374 -> 410).
+  const int64_t keep_mib = res == 2 ? 0 : res ? 20 : dir == kFwdXn || dir == kBwdSaved ? 40 : 64;
+  plan->k = rows * cols * 2 < keep_mib << 20 ? pick(mode | kKeep) : k;
   plan->packs = packs;
   plan->n_batches = rows / rows_per_batch;
   plan->n_tiles = (rows_per_batch + k.tile_rows - 1) / k.tile_rows;

@@ -20,9 +20,12 @@ constexpr int kPack = 8;    // bf16 elements per 128-bit pack
 // kept in L2), which measured 1-2 % faster than plain "nt" stores under the 2-reads-1-write mix
 // of the backward kernels.  The compiler's builtin only offers "nt", hence the asm for stores;
 // it is an ordinary vector store.  Parameters use ordinary cached loads.
+// KEEP: ordinary loads, see kKeep.
+template <bool KEEP = false>
 __device__ __forceinline__ u32x4 load_stream(const void* base, size_t elem_off) {
   const u32x4* p = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(base) + elem_off);
-  return __builtin_nontemporal_load(p);
+  if constexpr (KEEP) return *p;
+  else return __builtin_nontemporal_load(p);
 }
 __device__ __forceinline__ void store_stream(void* base, size_t elem_off, u32x4 v) {
   u32x4* p = reinterpret_cast<u32x4*>(static_cast<uint16_t*>(base) + elem_off);
@@ -55,7 +58,12 @@ enum Rows : int {
   kFull = 1,     // every lane slot holds a pack
   kRagged = 2,   // as kMasked, but rows start anywhere inside a line (cols % 64 != 0)
   kOdd = 3,      // any row length and 2-byte aligned tensors; the last pack may be short
+  // Added to the others (and to kFull / kMasked of the narrow kernels): the activations are read with ordinary loads,
+  // so that tensors which fit the caches stay there for the next kernel that reads them.
+  kKeep = 4,
 };
+constexpr int row_mode(int rows) { return rows & 3; }
+constexpr bool keeps(int rows) { return (rows & kKeep) != 0; }
 // Where rows are not whole lines, the segments of neighbouring waves and rows share the lines at
 // their ends.  A written-through store sends its part of such a line to memory on its own, and
 // memory turns a part of a 64-byte sector into a read and a write; those lines have to meet in
@@ -72,11 +80,15 @@ enum Rows : int {
 //   gate  1000: 73 / 75 | 66 / 58 | 61 / 64;  3000: 246 / 247 | 188 / 192 | 179 / 182
 //   residual + norm 1544: 179 / 187 | 133 / 137 | 128 / 142;  gated: 179 / 232 | 134 / 207 | 129 / 192
 constexpr bool short_rows(int W, int P) { return W * P <= 6; }
+// The instantiation that stands for `rows`: kKeep goes where the loads are ordinary ones anyway, and above 6144 columns.
+constexpr int kernel_rows(int W, int P, int rows, bool is_short) {
+  return W * P > 12 || (row_mode(rows) == kRagged && is_short) || row_mode(rows) == kOdd ? row_mode(rows) : rows;
+}
 
-template <int ROWS, bool SHORT>
+template <int ROWS, bool SHORT, bool KEEP>
 __device__ __forceinline__ u32x4 load_row(const void* base, size_t elem_off) {
   if constexpr (ROWS == kRagged && SHORT) return load_cached(base, elem_off);
-  else return load_stream(base, elem_off);
+  else return load_stream<KEEP>(base, elem_off);
 }
 // Element offset of a lane's pack, from the column that its loads use (no further register) or from its slot.
 // The kernels of 16 waves a row have 128 registers a lane and spill: with every slot in use they are

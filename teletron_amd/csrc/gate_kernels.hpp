@@ -24,8 +24,10 @@ struct GateArgs {
 
 enum GateMode : int { kGateFwd = 0, kGateBwd = 1 };
 
-template <int MODE, int W, int P, int R, int Q, int ROWS>
+template <int MODE, int W, int P, int R, int Q, int RK>
 __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
+  constexpr int ROWS = row_mode(RK);
+  constexpr bool KEEP = keeps(RK);
   constexpr bool FULL = ROWS == kFull, SHORT = false;   // SHORT: see enum Rows
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -64,8 +66,8 @@ __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
         rawb[r][p] = u32x4{0, 0, 0, 0};
         if (r0 + r < S && act[p]) {
           const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
-          rawa[r][p] = load_row<ROWS, SHORT>(a.a, off);
-          rawb[r][p] = load_row<ROWS, SHORT>(a.b, off);
+          rawa[r][p] = load_row<ROWS, SHORT, KEEP>(a.a, off);
+          rawb[r][p] = load_row<ROWS, SHORT, KEEP>(a.b, off);
         }
       }
   };
@@ -110,8 +112,9 @@ __global__ __launch_bounds__(64 * W * Q) void gate_wide(const GateArgs a) {
     wide_write_partials<1, W, P, Q>(acc, a.partials, b, C, q, w, lane);
 }
 
-template <int MODE, int L, int R, int NW, bool FULL>
+template <int MODE, int L, int R, int NW, int RK>
 __global__ __launch_bounds__(64 * NW) void gate_narrow(const GateArgs a) {
+  constexpr bool FULL = row_mode(RK) == kFull, KEEP = keeps(RK);
   constexpr int RPW = 64 / L;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -145,8 +148,8 @@ __global__ __launch_bounds__(64 * NW) void gate_narrow(const GateArgs a) {
       rawb[r] = u32x4{0, 0, 0, 0};
       if (rr < S && act) {
         const size_t off = (size_t)((b * S + rr) * C + col);
-        rawa[r] = load_stream(a.a, off);
-        rawb[r] = load_stream(a.b, off);
+        rawa[r] = load_stream<KEEP>(a.a, off);
+        rawb[r] = load_stream<KEEP>(a.b, off);
       }
     }
   };

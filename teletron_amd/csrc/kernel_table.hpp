@@ -65,7 +65,7 @@ constexpr int bwd_wide_R(int W, int P) { return 1; }
 // per row) is 2-3 % slower with R = 2 everywhere.  Ragged rows lose with two as well (60000 x 2200:
 // 162 -> 184 us, 1000: 71 -> 77 us).
 constexpr int adaln_bwd_wide_R(int W, int P, int rows) {
-  if (rows == kRagged || rows == kOdd) return bwd_wide_R(W, P);
+  if (row_mode(rows) == kRagged || row_mode(rows) == kOdd) return bwd_wide_R(W, P);
   return ((P == 1 && W >= 2 && W <= 4) || (P == 2 && (W == 3 || W == 6))) ? 2 : bwd_wide_R(W, P);
 }
 constexpr int fwd_wide_Q(int W, int P) {
@@ -98,33 +98,48 @@ inline int select_narrow(int packs) {
 template <int KIND, int W, int P, int ROWS>
 KernelInfo info_fwd_wide() {
   constexpr int R = fwd_wide_R(W, P), Q = fwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_fwd_wide<KIND, W, P, R, Q, ROWS>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_fwd_wide<KIND, W, P, R, Q, kernel_rows(W, P, ROWS, short_rows(W, P))>), 64 * W * Q, Q * R, P * R};
 }
 template <int KIND, int W, int P, int ROWS>
 KernelInfo info_bwd_wide() {
   constexpr int R = KIND == kAdaLN ? adaln_bwd_wide_R(W, P, ROWS) : bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_bwd_wide<KIND, W, P, R, Q, ROWS>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_bwd_wide<KIND, W, P, R, Q, kernel_rows(W, P, ROWS, short_rows(W, P))>), 64 * W * Q, Q * R, P * R};
 }
-template <int KIND, int W, int P, bool FULL>
+template <int KIND, int W, int P, int ROWS>
 KernelInfo info_bwd_saved_wide() {
   constexpr int R = bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_bwd_saved_wide<KIND, W, P, R, Q, FULL>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_bwd_saved_wide<KIND, W, P, R, Q, kernel_rows(W, P, ROWS, false)>), 64 * W * Q, Q * R, P * R};
 }
-template <int KIND, int L, bool FULL>
+template <int KIND, int L, int ROWS>
 KernelInfo info_bwd_saved_narrow() {
   constexpr int R = KIND == kRMS ? kNarrowRmsBwdR : kNarrowR, NW = kNarrowNW;
-  return {reinterpret_cast<const void*>(&norm_bwd_saved_narrow<KIND, L, R, NW, FULL>), 64 * NW, NW * R * (64 / L), R};
+  return {reinterpret_cast<const void*>(&norm_bwd_saved_narrow<KIND, L, R, NW, ROWS>), 64 * NW, NW * R * (64 / L), R};
 }
-template <int KIND, int L, bool FULL>
+template <int KIND, int L, int ROWS>
 KernelInfo info_fwd_narrow() {
-  constexpr int R = (KIND == kRMS && FULL) ? kNarrowRmsFwdFullR : kNarrowR, NW = kNarrowNW;
-  return {reinterpret_cast<const void*>(&norm_fwd_narrow<KIND, L, R, NW, FULL>), 64 * NW, NW * R * (64 / L), R};
+  constexpr int R = (KIND == kRMS && row_mode(ROWS) == kFull) ? kNarrowRmsFwdFullR : kNarrowR, NW = kNarrowNW;
+  return {reinterpret_cast<const void*>(&norm_fwd_narrow<KIND, L, R, NW, ROWS>), 64 * NW, NW * R * (64 / L), R};
 }
-template <int KIND, int L, bool FULL>
+template <int KIND, int L, int ROWS>
 KernelInfo info_bwd_narrow() {
   constexpr int R = KIND == kRMS ? kNarrowRmsBwdR : kNarrowR, NW = kNarrowNW;
-  return {reinterpret_cast<const void*>(&norm_bwd_narrow<KIND, L, R, NW, FULL>), 64 * NW, NW * R * (64 / L), R};
+  return {reinterpret_cast<const void*>(&norm_bwd_narrow<KIND, L, R, NW, ROWS>), 64 * NW, NW * R * (64 / L), R};
 }
+
+// Return the instantiation for `rows` (enum Rows): of kernels for whole-line rows (CALL: the arguments), of all but odd
+// rows, of all.
+#define TT_LINES(INFO, CALL, ...)                                             \
+  return rows == kFull             ? INFO<__VA_ARGS__, kFull> CALL            \
+         : rows == (kFull | kKeep) ? INFO<__VA_ARGS__, kFull | kKeep> CALL    \
+         : keeps(rows)             ? INFO<__VA_ARGS__, kMasked | kKeep> CALL  \
+                                   : INFO<__VA_ARGS__, kMasked> CALL;
+#define TT_ROWS(INFO, ...)                                          \
+  if (rows == kRagged) return INFO<__VA_ARGS__, kRagged>();         \
+  if (rows == (kRagged | kKeep)) return INFO<__VA_ARGS__, kRagged | kKeep>(); \
+  TT_LINES(INFO, (), __VA_ARGS__)
+#define TT_ROWS_ODD(INFO, ...)                                      \
+  if (row_mode(rows) == kOdd) return INFO<__VA_ARGS__, kOdd>();     \
+  TT_ROWS(INFO, __VA_ARGS__)
 
 // AdaLN forward that also stores x_norm (the reference's forward contract): one read and two
 // write streams.  Bare streams of that mix (no arithmetic) reach 5.7-5.9 TB/s on MI355X (370-385 us
@@ -139,27 +154,26 @@ constexpr int fwd_xn_wide_Q(int W, int P) { return 1; }
 template <int W, int P, int ROWS>
 KernelInfo info_fwd_xn_wide() {
   constexpr int R = fwd_wide_R(W, P), Q = fwd_xn_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_fwd_wide<kAdaLN, W, P, R, Q, ROWS, false, true>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_fwd_wide<kAdaLN, W, P, R, Q, kernel_rows(W, P, ROWS, false), false, true>), 64 * W * Q, Q * R, P * R};
 }
-template <int L, bool FULL>
+template <int L, int ROWS>
 KernelInfo info_fwd_xn_narrow() {
   constexpr int R = kNarrowR, NW = kNarrowNW;
-  return {reinterpret_cast<const void*>(&norm_fwd_narrow<kAdaLN, L, R, NW, FULL, 0, true>), 64 * NW, NW * R * (64 / L), R};
+  return {reinterpret_cast<const void*>(&norm_fwd_narrow<kAdaLN, L, R, NW, ROWS, 0, true>), 64 * NW, NW * R * (64 / L), R};
 }
 inline KernelInfo lookup_fwd_xn(bool narrow, int idx, int rows) {
   if (narrow) {
     switch (idx) {
-#define X(i, L) case i: return rows == kFull ? info_fwd_xn_narrow<L, true>() : info_fwd_xn_narrow<L, false>();
+#define X(i, L) case i: TT_LINES(info_fwd_xn_narrow, (), L)
       TT_NARROW_LIST(X)
 #undef X
     }
   } else {
     switch (idx) {
-#define X(i, W, P)                                           \
-  case i:                                                    \
-    return rows == kFull  ? info_fwd_xn_wide<W, P, kFull>()  \
-           : rows == kOdd ? info_fwd_xn_wide<W, P, kOdd>()   \
-                          : info_fwd_xn_wide<W, P, kMasked>();
+#define X(i, W, P)                                                                  \
+  case i:                                                                           \
+    if (row_mode(rows) == kOdd) return info_fwd_xn_wide<W, P, kOdd>();              \
+    TT_LINES(info_fwd_xn_wide, (), W, P)
       TT_WIDE_LIST(X)
 #undef X
     }
@@ -167,19 +181,11 @@ inline KernelInfo lookup_fwd_xn(bool narrow, int idx, int rows) {
   return {nullptr, 0, 0, 0};
 }
 
-// Picks the instantiation of a wide kernel for the row mode `rows` (enum Rows).
-#define TT_ROWS(INFO, ...)                                     \
-  return rows == kFull     ? INFO<__VA_ARGS__, kFull>()        \
-         : rows == kRagged ? INFO<__VA_ARGS__, kRagged>()      \
-                           : INFO<__VA_ARGS__, kMasked>();
-#define TT_ROWS_ODD(INFO, ...)                           \
-  if (rows == kOdd) return INFO<__VA_ARGS__, kOdd>();    \
-  TT_ROWS(INFO, __VA_ARGS__)
 template <int KIND>
 KernelInfo lookup_fwd(bool narrow, int idx, int rows) {
   if (narrow) {
     switch (idx) {
-#define X(i, L) case i: return rows == kFull ? info_fwd_narrow<KIND, L, true>() : info_fwd_narrow<KIND, L, false>();
+#define X(i, L) case i: TT_LINES(info_fwd_narrow, (), KIND, L)
       TT_NARROW_LIST(X)
 #undef X
     }
@@ -196,7 +202,7 @@ template <int KIND>
 KernelInfo lookup_bwd(bool narrow, int idx, int rows) {
   if (narrow) {
     switch (idx) {
-#define X(i, L) case i: return rows == kFull ? info_bwd_narrow<KIND, L, true>() : info_bwd_narrow<KIND, L, false>();
+#define X(i, L) case i: TT_LINES(info_bwd_narrow, (), KIND, L)
       TT_NARROW_LIST(X)
 #undef X
     }
@@ -211,25 +217,25 @@ KernelInfo lookup_bwd(bool narrow, int idx, int rows) {
 }
 
 // RMSNorm with the rotary embedding fused behind it (wide rows only).
-template <int W, int P, bool FULL>
+template <int W, int P, int ROWS>
 KernelInfo info_fwd_rope_wide() {
   constexpr int R = fwd_wide_R(W, P), Q = fwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_fwd_wide<kRMS, W, P, R, Q, FULL ? kFull : kMasked, true>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_fwd_wide<kRMS, W, P, R, Q, kernel_rows(W, P, ROWS, false), true>), 64 * W * Q, Q * R, P * R};
 }
-template <int W, int P, bool FULL>
+template <int W, int P, int ROWS>
 KernelInfo info_bwd_rope_wide() {
   constexpr int R = bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&norm_bwd_wide<kRMS, W, P, R, Q, FULL ? kFull : kMasked, true>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&norm_bwd_wide<kRMS, W, P, R, Q, kernel_rows(W, P, ROWS, false), true>), 64 * W * Q, Q * R, P * R};
 }
-template <int L, bool FULL>
+template <int L, int ROWS>
 KernelInfo info_fwd_rope_narrow() {
   constexpr int R = kNarrowR, NW = kNarrowNW;
-  return {reinterpret_cast<const void*>(&norm_fwd_narrow<kRMS, L, R, NW, FULL, true>), 64 * NW, NW * R * (64 / L), R};
+  return {reinterpret_cast<const void*>(&norm_fwd_narrow<kRMS, L, R, NW, ROWS, 1>), 64 * NW, NW * R * (64 / L), R};
 }
-template <int L, bool FULL>
+template <int L, int ROWS>
 KernelInfo info_bwd_rope_narrow() {
   constexpr int R = kNarrowR, NW = kNarrowNW;
-  return {reinterpret_cast<const void*>(&norm_bwd_narrow<kRMS, L, R, NW, FULL, true>), 64 * NW, NW * R * (64 / L), R};
+  return {reinterpret_cast<const void*>(&norm_bwd_narrow<kRMS, L, R, NW, ROWS, 1>), 64 * NW, NW * R * (64 / L), R};
 }
 // Token mode of the narrow ROPE kernels (ROPE = 2: the rows a wave takes per tile are heads of one
 // token, so the (cos, sin) entries are loaded once per tile and lane).  R loads of 64 / L rows each have to
@@ -244,12 +250,12 @@ KernelInfo info_bwd_rope_narrow() {
 // CU and reach 259-265 us).
 constexpr int kRopeTokenMinL = 8, kRopeTokenMaxL = 16;
 constexpr int rope_token_NW(int R) { return R > 0 ? (24 + R / 2) / R : 0; }
-template <int L, int R, bool FULL>
+template <int L, int R, int ROWS>
 KernelInfo info_rope_token(bool backward) {
   constexpr int NW = rope_token_NW(R);
   if (backward)
-    return {reinterpret_cast<const void*>(&norm_bwd_narrow<kRMS, L, R, NW, FULL, 2>), 64 * NW, NW * R * (64 / L), R};
-  return {reinterpret_cast<const void*>(&norm_fwd_narrow<kRMS, L, R, NW, FULL, 2>), 64 * NW, NW * R * (64 / L), R};
+    return {reinterpret_cast<const void*>(&norm_bwd_narrow<kRMS, L, R, NW, ROWS, 2>), 64 * NW, NW * R * (64 / L), R};
+  return {reinterpret_cast<const void*>(&norm_fwd_narrow<kRMS, L, R, NW, ROWS, 2>), 64 * NW, NW * R * (64 / L), R};
 }
 // Loads per wave and tile in token mode, or 0 where `heads` rows per token do not allow it.
 inline int rope_token_R(int L, int64_t heads) {
@@ -258,33 +264,33 @@ inline int rope_token_R(int L, int64_t heads) {
     if (heads % (r * (64 / L)) == 0) return r;
   return 0;
 }
-template <int L, bool FULL>
+template <int L, int ROWS>
 KernelInfo lookup_rope_token(int R, bool backward) {
-  return R == 6   ? info_rope_token<L, 6, FULL>(backward)
-         : R == 4 ? info_rope_token<L, 4, FULL>(backward)
-                  : info_rope_token<L, 3, FULL>(backward);
+  return R == 6   ? info_rope_token<L, 6, ROWS>(backward)
+         : R == 4 ? info_rope_token<L, 4, ROWS>(backward)
+                  : info_rope_token<L, 3, ROWS>(backward);
 }
-inline KernelInfo lookup_rope(bool narrow, bool backward, int idx, bool full, int64_t heads) {
+inline KernelInfo lookup_rope(bool narrow, bool backward, int idx, int rows, int64_t heads) {
   if (const int r = narrow ? rope_token_R(kNarrowL[idx], heads) : 0) {
-    if (kNarrowL[idx] == 16) return full ? lookup_rope_token<16, true>(r, backward) : lookup_rope_token<16, false>(r, backward);
-    return full ? lookup_rope_token<8, true>(r, backward) : lookup_rope_token<8, false>(r, backward);
+    if (kNarrowL[idx] == 16) TT_LINES(lookup_rope_token, (r, backward), 16)
+    TT_LINES(lookup_rope_token, (r, backward), 8)
   }
   if (narrow) {
     switch (idx) {
-#define X(i, L)                                                                                       \
-  case i:                                                                                             \
-    return backward ? (full ? info_bwd_rope_narrow<L, true>() : info_bwd_rope_narrow<L, false>())     \
-                    : (full ? info_fwd_rope_narrow<L, true>() : info_fwd_rope_narrow<L, false>());
+#define X(i, L)                                         \
+  case i:                                               \
+    if (backward) TT_LINES(info_bwd_rope_narrow, (), L) \
+    TT_LINES(info_fwd_rope_narrow, (), L)
       TT_NARROW_LIST(X)
 #undef X
     }
     return {nullptr, 0, 0, 0};
   }
   switch (idx) {
-#define X(i, W, P)                                                                                  \
-  case i:                                                                                           \
-    return backward ? (full ? info_bwd_rope_wide<W, P, true>() : info_bwd_rope_wide<W, P, false>()) \
-                    : (full ? info_fwd_rope_wide<W, P, true>() : info_fwd_rope_wide<W, P, false>());
+#define X(i, W, P)                                       \
+  case i:                                                \
+    if (backward) TT_LINES(info_bwd_rope_wide, (), W, P) \
+    TT_LINES(info_fwd_rope_wide, (), W, P)
     TT_WIDE_LIST(X)
 #undef X
   }
@@ -294,18 +300,18 @@ inline KernelInfo lookup_rope(bool narrow, bool backward, int idx, bool full, in
 template <int MODE, int W, int P, int ROWS>
 KernelInfo info_gate_wide() {
   constexpr int R = bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
-  return {reinterpret_cast<const void*>(&gate_wide<MODE, W, P, R, Q, ROWS>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&gate_wide<MODE, W, P, R, Q, kernel_rows(W, P, ROWS, false)>), 64 * W * Q, Q * R, P * R};
 }
-template <int MODE, int L, bool FULL>
+template <int MODE, int L, int ROWS>
 KernelInfo info_gate_narrow() {
   constexpr int R = kNarrowR, NW = kNarrowNW;
-  return {reinterpret_cast<const void*>(&gate_narrow<MODE, L, R, NW, FULL>), 64 * NW, NW * R * (64 / L), R};
+  return {reinterpret_cast<const void*>(&gate_narrow<MODE, L, R, NW, ROWS>), 64 * NW, NW * R * (64 / L), R};
 }
 template <int MODE>
 KernelInfo lookup_gate(bool narrow, int idx, int rows) {
   if (narrow) {
     switch (idx) {
-#define X(i, L) case i: return rows == kFull ? info_gate_narrow<MODE, L, true>() : info_gate_narrow<MODE, L, false>();
+#define X(i, L) case i: TT_LINES(info_gate_narrow, (), MODE, L)
       TT_NARROW_LIST(X)
 #undef X
     }
@@ -339,25 +345,23 @@ constexpr int res_fwd_Q(int W, int P) {
 constexpr int res_bwd_Q(int W, int P, bool gated) {
   return res_waves_Q(W, P);
 }
-template <int W, int P, int ROWS, bool GATED>
+template <bool GATED, int W, int P, int ROWS>
 KernelInfo info_res_fwd() {
   constexpr int R = 1, Q = res_fwd_Q(W, P);
-  return {reinterpret_cast<const void*>(&resnorm_fwd_wide<W, P, R, Q, ROWS, GATED>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&resnorm_fwd_wide<W, P, R, Q, GATED ? row_mode(ROWS) : kernel_rows(W, P, ROWS, short_rows(W, P)), GATED>), 64 * W * Q, Q * R, P * R};
 }
-template <int W, int P, int ROWS, bool GATED>
+template <bool GATED, int W, int P, int ROWS>
 KernelInfo info_res_bwd() {
   constexpr int R = 1, Q = res_bwd_Q(W, P, GATED);
-  return {reinterpret_cast<const void*>(&resnorm_bwd_wide<W, P, R, Q, ROWS, GATED>), 64 * W * Q, Q * R, P * R};
+  return {reinterpret_cast<const void*>(&resnorm_bwd_wide<W, P, R, Q, GATED ? row_mode(ROWS) : kernel_rows(W, P, ROWS, short_rows(W, P)), GATED>), 64 * W * Q, Q * R, P * R};
 }
 template <bool GATED>
 KernelInfo lookup_res(bool backward, int idx, int rows) {
   switch (idx) {
-#define X(i, W, P)                                                                                            \
-  case i:                                                                                                     \
-    if (rows == kFull) return backward ? info_res_bwd<W, P, kFull, GATED>() : info_res_fwd<W, P, kFull, GATED>(); \
-    if (rows == kRagged)                                                                                      \
-      return backward ? info_res_bwd<W, P, kRagged, GATED>() : info_res_fwd<W, P, kRagged, GATED>();          \
-    return backward ? info_res_bwd<W, P, kMasked, GATED>() : info_res_fwd<W, P, kMasked, GATED>();
+#define X(i, W, P)                                          \
+  case i:                                                   \
+    if (backward) { TT_ROWS(info_res_bwd, GATED, W, P) }    \
+    TT_ROWS(info_res_fwd, GATED, W, P)
     TT_WIDE_LIST(X)
 #undef X
   }
@@ -365,16 +369,16 @@ KernelInfo lookup_res(bool backward, int idx, int rows) {
 }
 
 template <int KIND>
-KernelInfo lookup_bwd_saved(bool narrow, int idx, bool full) {
+KernelInfo lookup_bwd_saved(bool narrow, int idx, int rows) {
   if (narrow) {
     switch (idx) {
-#define X(i, L) case i: return full ? info_bwd_saved_narrow<KIND, L, true>() : info_bwd_saved_narrow<KIND, L, false>();
+#define X(i, L) case i: TT_LINES(info_bwd_saved_narrow, (), KIND, L)
       TT_NARROW_LIST(X)
 #undef X
     }
   } else {
     switch (idx) {
-#define X(i, W, P) case i: return full ? info_bwd_saved_wide<KIND, W, P, true>() : info_bwd_saved_wide<KIND, W, P, false>();
+#define X(i, W, P) case i: TT_LINES(info_bwd_saved_wide, (), KIND, W, P)
       TT_WIDE_LIST(X)
 #undef X
     }
@@ -389,9 +393,9 @@ KernelInfo adaln_fwd_xnorm_kernel(bool narrow, int idx, int rows);
 KernelInfo adaln_bwd_kernel(bool narrow, int idx, int rows);
 KernelInfo rms_fwd_kernel(bool narrow, int idx, int rows);
 KernelInfo rms_bwd_kernel(bool narrow, int idx, int rows);
-KernelInfo adaln_bwd_saved_kernel(bool narrow, int idx, bool full);
-KernelInfo rms_bwd_saved_kernel(bool narrow, int idx, bool full);
-KernelInfo rms_rope_kernel(bool narrow, bool backward, int idx, bool full, int64_t heads);
+KernelInfo adaln_bwd_saved_kernel(bool narrow, int idx, int rows);
+KernelInfo rms_bwd_saved_kernel(bool narrow, int idx, int rows);
+KernelInfo rms_rope_kernel(bool narrow, bool backward, int idx, int rows, int64_t heads);
 KernelInfo gate_fwd_kernel(bool narrow, int idx, int rows);
 KernelInfo gate_bwd_kernel(bool narrow, int idx, int rows);
 KernelInfo resnorm_plain_kernel(bool backward, int idx, int rows);

@@ -148,8 +148,10 @@ __device__ __forceinline__ u32x4 load_pack(const void* base, size_t elem_off, in
 }
 
 // XN: also store the normalised input before modulation (a.x_norm), paired with the y store.
-template <int KIND, int W, int P, int R, int Q, int ROWS, bool ROPE = false, bool XN = false>
+template <int KIND, int W, int P, int R, int Q, int RK, bool ROPE = false, bool XN = false>
 __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
+  constexpr int ROWS = row_mode(RK);
+  constexpr bool KEEP = keeps(RK);
   constexpr bool ADALN = (KIND == kAdaLN);
   constexpr bool FULL = ROWS == kFull, SHORT = short_rows(W, P), ODD = ROWS == kOdd;
   static_assert(!ROPE || KIND == kRMS, "rotary embedding is fused behind RMSNorm only");
@@ -231,7 +233,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
         if (r0 + r < S && act[p]) {
           const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
           if constexpr (ODD) raw[r][p] = load_any(a.x, off - (kPack - n[p]));
-          else               raw[r][p] = load_row<ROWS, SHORT>(a.x, off);
+          else               raw[r][p] = load_row<ROWS, SHORT, KEEP>(a.x, off);
         }
       }
   };
@@ -385,8 +387,10 @@ __device__ __forceinline__ void wide_write_partials(const float (&acc)[NACC][P][
 }
 
 // ============================================================================ wide backward
-template <int KIND, int W, int P, int R, int Q, int ROWS, bool ROPE = false>
+template <int KIND, int W, int P, int R, int Q, int RK, bool ROPE = false>
 __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
+  constexpr int ROWS = row_mode(RK);
+  constexpr bool KEEP = keeps(RK);
   constexpr bool ADALN = (KIND == kAdaLN);
   constexpr bool FULL = ROWS == kFull, SHORT = short_rows(W, P), ODD = ROWS == kOdd;
   static_assert(!ROPE || KIND == kRMS, "rotary embedding is fused behind RMSNorm only");
@@ -462,8 +466,8 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_wide(const BwdArgs a) {
             rawx[r][p] = load_any(a.x, off - (kPack - n[p]));
             rawd[r][p] = load_any(a.dy, off - (kPack - n[p]));
           } else {
-            rawx[r][p] = load_row<ROWS, SHORT>(a.x, off);
-            rawd[r][p] = load_row<ROWS, SHORT>(a.dy, off);
+            rawx[r][p] = load_row<ROWS, SHORT, KEEP>(a.x, off);
+            rawd[r][p] = load_row<ROWS, SHORT, KEEP>(a.dy, off);
           }
           if constexpr (ROPE)
             load_freq8(a.freqs, (size_t)(pos[r] * a.head_dim + fcol[p]), fr[r][p]);
@@ -597,8 +601,9 @@ struct RowPos {
 // ROPE: 0 none; 1 every row looks up its own position; 2 the R * 64/L rows a wave takes per tile
 // are heads of ONE token (the caller guarantees that R * 64/L divides rows_per_pos), so a lane
 // loads its (cos, sin) entries once per tile instead of once per row.
-template <int KIND, int L, int R, int NW, bool FULL, int ROPE = 0, bool XN = false>   // XN as in norm_fwd_wide
+template <int KIND, int L, int R, int NW, int RK, int ROPE = 0, bool XN = false>   // XN as in norm_fwd_wide
 __global__ __launch_bounds__(64 * NW) void norm_fwd_narrow(const FwdArgs a) {
+  constexpr bool FULL = row_mode(RK) == kFull, KEEP = keeps(RK);
   constexpr bool ADALN = (KIND == kAdaLN);
   static_assert(!ROPE || KIND == kRMS, "rotary embedding is fused behind RMSNorm only");
   static_assert(!XN || ADALN, "x_norm is an output of the AdaLN forward only");
@@ -653,7 +658,7 @@ __global__ __launch_bounds__(64 * NW) void norm_fwd_narrow(const FwdArgs a) {
         for (int j = 0; j < 8; ++j) fr[f][j] = 0.f;
       }
       if (rr < S && act) {
-        raw[r] = load_stream(a.x, (size_t)((b * S + rr) * C + col));
+        raw[r] = load_stream<KEEP>(a.x, (size_t)((b * S + rr) * C + col));
         if (table) load_freq8(a.freqs, (size_t)(rp[f].pos * a.head_dim + col), fr[f]);
       }
       if (table) rp[f].advance(a.rows_per_pos, a.seq_len);
@@ -758,8 +763,9 @@ __device__ __forceinline__ void narrow_write_partials(float (&acc0)[8], float (&
 }
 
 // ============================================================================ narrow backward
-template <int KIND, int L, int R, int NW, bool FULL, int ROPE = 0>   // ROPE as in norm_fwd_narrow
+template <int KIND, int L, int R, int NW, int RK, int ROPE = 0>   // ROPE as in norm_fwd_narrow
 __global__ __launch_bounds__(64 * NW) void norm_bwd_narrow(const BwdArgs a) {
+  constexpr bool FULL = row_mode(RK) == kFull, KEEP = keeps(RK);
   constexpr bool ADALN = (KIND == kAdaLN);
   static_assert(!ROPE || KIND == kRMS, "rotary embedding is fused behind RMSNorm only");
   constexpr int NF = ROPE == 1 ? R : 1;
@@ -813,8 +819,8 @@ __global__ __launch_bounds__(64 * NW) void norm_bwd_narrow(const BwdArgs a) {
       }
       if (rr < S && act) {
         const size_t off = (size_t)((b * S + rr) * C + col);
-        rawx[r] = load_stream(a.x, off);
-        rawd[r] = load_stream(a.dy, off);
+        rawx[r] = load_stream<KEEP>(a.x, off);
+        rawd[r] = load_stream<KEEP>(a.dy, off);
         if (table) load_freq8(a.freqs, (size_t)(rp[f].pos * a.head_dim + col), fr[f]);
       }
       if (table) rp[f].advance(a.rows_per_pos, a.seq_len);
@@ -902,8 +908,9 @@ struct BwdSavedArgs {
   float inv_cols;
 };
 
-template <int KIND, int W, int P, int R, int Q, bool FULL>
+template <int KIND, int W, int P, int R, int Q, int RK>
 __global__ __launch_bounds__(64 * W * Q) void norm_bwd_saved_wide(const BwdSavedArgs a) {
+  constexpr bool FULL = row_mode(RK) == kFull, KEEP = keeps(RK);
   constexpr bool ADALN = (KIND == kAdaLN);
   constexpr int NACC = ADALN ? 2 : 1;
   constexpr int NV = ADALN ? 2 : 1;
@@ -953,8 +960,8 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_saved_wide(const BwdSaved
         rawd[r][p] = u32x4{0, 0, 0, 0};
         if (ok && act[p]) {
           const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
-          rawx[r][p] = load_stream(a.xs, off);
-          rawd[r][p] = load_stream(a.dy, off);
+          rawx[r][p] = load_stream<KEEP>(a.xs, off);
+          rawd[r][p] = load_stream<KEEP>(a.dy, off);
         }
       }
     }
@@ -1022,8 +1029,9 @@ __global__ __launch_bounds__(64 * W * Q) void norm_bwd_saved_wide(const BwdSaved
   wide_write_partials<NACC, W, P, Q>(acc, a.partials, b, C, q, w, lane);
 }
 
-template <int KIND, int L, int R, int NW, bool FULL>
+template <int KIND, int L, int R, int NW, int RK>
 __global__ __launch_bounds__(64 * NW) void norm_bwd_saved_narrow(const BwdSavedArgs a) {
+  constexpr bool FULL = row_mode(RK) == kFull, KEEP = keeps(RK);
   constexpr bool ADALN = (KIND == kAdaLN);
   constexpr int RPW = 64 / L;
   const int lane = threadIdx.x & 63;
@@ -1062,8 +1070,8 @@ __global__ __launch_bounds__(64 * NW) void norm_bwd_saved_narrow(const BwdSavedA
       rs[r] = rr < S ? a.rstd[b * S + rr] : 0.f;
       if (rr < S && act) {
         const size_t off = (size_t)((b * S + rr) * C + col);
-        rawx[r] = load_stream(a.xs, off);
-        rawd[r] = load_stream(a.dy, off);
+        rawx[r] = load_stream<KEEP>(a.xs, off);
+        rawd[r] = load_stream<KEEP>(a.dy, off);
       }
     }
   };

@@ -67,8 +67,10 @@ struct ResBwdArgs {
 };
 
 // ============================================================================ forward
-template <int W, int P, int R, int Q, int ROWS, bool GATED>
+template <int W, int P, int R, int Q, int RK, bool GATED>
 __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs a) {
+  constexpr int ROWS = row_mode(RK);
+  constexpr bool KEEP = keeps(RK);
   constexpr bool FULL = ROWS == kFull, SHORT = !GATED && short_rows(W, P);
   __shared__ float red[2][Q][W * R];
 
@@ -116,8 +118,8 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs 
         rawr[r][p] = u32x4{0, 0, 0, 0};
         if (r0 + r < S && act[p]) {
           const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
-          rawx[r][p] = load_row<ROWS, SHORT>(a.x, off);
-          rawr[r][p] = load_row<ROWS, SHORT>(a.r, off);
+          rawx[r][p] = load_row<ROWS, SHORT, KEEP>(a.x, off);
+          rawr[r][p] = load_row<ROWS, SHORT, KEEP>(a.r, off);
         }
       }
   };
@@ -209,8 +211,10 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_fwd_wide(const ResFwdArgs 
 }
 
 // ============================================================================ backward
-template <int W, int P, int R, int Q, int ROWS, bool GATED>
+template <int W, int P, int R, int Q, int RK, bool GATED>
 __global__ __launch_bounds__(64 * W * Q) void resnorm_bwd_wide(const ResBwdArgs a) {
+  constexpr int ROWS = row_mode(RK);
+  constexpr bool KEEP = keeps(RK);
   constexpr bool FULL = ROWS == kFull, SHORT = !GATED && short_rows(W, P);
   constexpr int NACC = GATED ? 3 : 2;
   constexpr int NV = 3;
@@ -262,10 +266,10 @@ __global__ __launch_bounds__(64 * W * Q) void resnorm_bwd_wide(const ResBwdArgs 
         if constexpr (GATED) rawr[r][p] = u32x4{0, 0, 0, 0};
         if (r0 + r < S && act[p]) {
           const size_t off = (size_t)((b * S + r0 + r) * C + col[p]);
-          raws[r][p] = load_row<ROWS, SHORT>(a.s, off);
-          rawd[r][p] = load_row<ROWS, SHORT>(a.dy, off);
-          if (have_ds) rawg[r][p] = load_row<ROWS, SHORT>(a.ds_in, off);
-          if constexpr (GATED) rawr[r][p] = load_row<ROWS, SHORT>(a.r, off);
+          raws[r][p] = load_row<ROWS, SHORT, KEEP>(a.s, off);
+          rawd[r][p] = load_row<ROWS, SHORT, KEEP>(a.dy, off);
+          if (have_ds) rawg[r][p] = load_row<ROWS, SHORT, KEEP>(a.ds_in, off);
+          if constexpr (GATED) rawr[r][p] = load_row<ROWS, SHORT, KEEP>(a.r, off);
         }
       }
   };

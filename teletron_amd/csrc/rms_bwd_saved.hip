@@ -3,5 +3,5 @@
 #include "kernel_table.hpp"
 
 namespace tt {
-KernelInfo rms_bwd_saved_kernel(bool narrow, int idx, bool full) { return lookup_bwd_saved<kRMS>(narrow, idx, full); }
+KernelInfo rms_bwd_saved_kernel(bool narrow, int idx, int rows) { return lookup_bwd_saved<kRMS>(narrow, idx, rows); }
 }  // namespace tt
