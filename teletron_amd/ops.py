@@ -31,7 +31,10 @@ def _load_native():
     there and does not load (built for another torch) raises."""
     if importlib.util.find_spec(__package__ + ".native_ops") is None:
         return False
-    return importlib.import_module(__package__ + ".native_ops")
+    module = importlib.import_module(__package__ + ".native_ops")
+    if hasattr(module, "set_python_backwards"):
+        module.set_python_backwards(_BACKWARDS)
+    return module
 
 
 def native(x: torch.Tensor):
@@ -647,3 +650,33 @@ def residual_norm_backward(dy: torch.Tensor, ds_in: Optional[torch.Tensor], s: t
                   _ptr(residual if gate is not None else None), _ptr(gate), n_gate, scale.data_ptr(), n_param,
                   int(bool(affine)), ws, ws_bytes, rows, cols, rpb, float(eps), _stream(s))
     return dx, dr, dscale, dshift, dgate
+
+
+# Backward calls that the native nodes do not cover: (tensor gradients in the order of the operator's arguments).
+def _gate_backward_in_order(dout, gate, residual):
+    dres, dgate = gate_residual_backward(dout, gate, residual, BF16)
+    return None, dgate, dres
+
+
+def _rmsnorm_backward_any(dy, x, weight, freqs, eps, head_dim, heads, bf16):
+    dtype = BF16 if bf16 else torch.float32
+    if freqs is None:
+        return rmsnorm_backward(dy, x, weight, eps, dtype)
+    if heads:
+        return rmsnorm_rope_heads_backward(dy, x, weight, freqs, eps, dtype)
+    return rmsnorm_rope_backward(dy, x, weight, freqs, eps, head_dim, dtype)
+
+
+def _adaln_backward_in_order(dy, x, scale, eps):
+    dx, grads = adaln_backward_packed(dy, x, scale, eps, BF16)
+    return dx, grads[0], grads[1]
+
+
+def _residual_norm_backward_in_order(dy, ds, s, residual, gate, scale, eps, affine, direct):
+    dx, dr, dscale, dshift, dgate = residual_norm_backward(dy, ds, s, residual, gate, scale, eps, affine,
+                                                           BF16 if direct else torch.float32)
+    return dx, dr, dgate, dscale, dshift
+
+
+_BACKWARDS = {"adaln": _adaln_backward_in_order, "rmsnorm": _rmsnorm_backward_any, "gate": _gate_backward_in_order,
+              "residual_norm": _residual_norm_backward_in_order}

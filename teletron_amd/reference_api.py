@@ -12,13 +12,17 @@ from __future__ import annotations
 import torch
 from torch.autograd import Function
 
+from .functional import NativeFirst
+
 
 def _modules():
     from . import fused_adaln, fused_rmsnorm   # built by `python -m teletron_amd.build`
     return fused_adaln, fused_rmsnorm
 
 
-class AdaLNModelFunction(Function):
+class AdaLNModelFunction(NativeFirst):
+    _native = "adaln_saved"
+
     @staticmethod
     def forward(ctx, x, scale, shift, epsilon, cols):
         fused_adaln, _ = _modules()

@@ -1,0 +1,285 @@
+"""The operators as native autograd nodes against the Python Functions that they stand for: the same bits, and the same
+behaviour towards hooks, transforms, freed and changed tensors."""
+import threading
+
+import pytest
+import torch
+
+from test_gpu_parity import DEV, rand_bf16
+
+pytestmark = pytest.mark.gpu
+EPS, B, S, C, H = 1e-6, 2, 37, 1536, 12
+
+
+def leaf(*shape, seed, scale=1.0, dtype=torch.bfloat16):
+    return rand_bf16(*shape, seed=seed, scale=scale).to(DEV).to(dtype).requires_grad_(True)
+
+
+def cases():
+    """name -> (call, inputs): each operator in the forms that models use."""
+    import teletron_amd as T
+    from teletron_amd import reference_api as R
+    x, r = leaf(B, S, C, seed=0), leaf(B, S, C, seed=1)
+    mod = [t.detach().requires_grad_(True) for t in rand_bf16(B, 6, C, seed=2, scale=0.3).to(DEV).chunk(6, dim=1)[:3]]
+    one, two = leaf(C, seed=3, scale=0.3), leaf(C, seed=4, scale=0.3)
+    w32 = leaf(C, seed=5, dtype=torch.float32)
+    table = torch.randn(S, C // H // 2, 2, device=DEV, generator=torch.Generator(DEV).manual_seed(6))
+    heads = leaf(B, S, H, C // H, seed=7)
+    wh = leaf(C // H, seed=8)
+    return {
+        "adaln": (lambda: T.adaln_modulate(x, mod[0], mod[1], EPS), [x, mod[0], mod[1]]),
+        "adaln shared": (lambda: T.AdaLNModelFunction.apply(x, one, two, EPS, C), [x, one, two]),
+        "rmsnorm": (lambda: T.RMSNormModelFunction.apply(x, one, EPS, C), [x, one]),
+        "rmsnorm fp32": (lambda: T.RMSNormModelFunction.apply(x, w32, EPS, C), [x, w32]),
+        "rope": (lambda: T.RMSNormRopeFunction.apply(x, one, table, EPS, H), [x, one]),
+        "rope heads": (lambda: T.RMSNormRopeHeadsFunction.apply(heads, wh, table, EPS), [heads, wh]),
+        "rope heads view": (lambda: T.RMSNormRopeHeadsFunction.apply(heads.transpose(1, 2), wh, table, EPS), [heads, wh]),
+        "gate": (lambda: T.FusedGate()(x, mod[2], r), [x, mod[2], r]),
+        "residual": (lambda: T.residual_adaln(x, r, None, mod[0], mod[1], EPS), [x, r, mod[0], mod[1]]),
+        "gated residual": (lambda: T.residual_layer_norm(x, r, mod[2], one, two, EPS), [x, r, mod[2], one, two]),
+        "saved": (lambda: R.AdaLNModelFunction.apply(x, one, two, EPS, C), [x, one, two]),
+    }
+
+
+NAMES = ["adaln", "adaln shared", "rmsnorm", "rmsnorm fp32", "rope", "rope heads", "rope heads view", "gate", "residual",
+         "gated residual", "saved"]
+
+
+def outs(out):
+    return list(out) if isinstance(out, tuple) else [out]
+
+
+def both(monkeypatch, f):
+    """f() through the native nodes, then through the Python Functions."""
+    from teletron_amd import ops
+    a = f()
+    with monkeypatch.context() as m:
+        m.setattr(ops, "native", lambda x: None)
+        return a, f()
+
+
+def same(a, b):
+    assert len(a) == len(b)
+    for p, q in zip(a, b):
+        assert (p is None) == (q is None)
+        assert p is None or (torch.equal(p, q) and p.dtype == q.dtype and p.stride() == q.stride())
+
+
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("how", ["dense", "expanded", "misaligned"])
+def test_same_bits_for_any_gradient(monkeypatch, name, how):
+    def run():
+        call, inputs = cases()[name]
+        o = outs(call())
+        assert ("Function" in o[0].grad_fn.name())
+        g = []
+        for i, t in enumerate(o):
+            d = rand_bf16(*t.shape, seed=20 + i).to(DEV)
+            if how == "expanded":
+                d = d[:, :1].expand(t.shape)
+            elif how == "misaligned":
+                buf = torch.empty(d.numel() + 3, dtype=d.dtype, device=DEV)
+                buf[3:] = d.flatten()
+                d = buf[3:].view(d.shape)
+            g.append(d)
+        return o + list(torch.autograd.grad(o, inputs, g))
+
+    # (a gradient of the view is copied into the rows' order, and so aligned again)
+    if how == "misaligned" and name not in ("adaln", "adaln shared", "rmsnorm", "rmsnorm fp32", "rope heads view"):
+        with pytest.raises(Exception) as a:
+            run()
+        from teletron_amd import ops
+        monkeypatch.setattr(ops, "native", lambda x: None)
+        with pytest.raises(type(a.value)):
+            run()
+        return
+    native, python = both(monkeypatch, run)
+    same(native, python)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_each_input_alone_and_no_gradients(monkeypatch, name):
+    def run():
+        results = []
+        call, inputs = cases()[name]
+        for k in range(len(inputs)):
+            for i, t in enumerate(inputs):
+                t.requires_grad_(i == k)
+            o = outs(call())
+            used = [t for t in o if t.requires_grad]
+            results += o + list(torch.autograd.grad(used, [inputs[k]], [torch.ones_like(t) for t in used]))
+        with torch.no_grad():
+            results += outs(call())
+        with torch.inference_mode():
+            results += outs(call())
+        assert not any(t.requires_grad for t in results[-2:])
+        return results
+
+    same(*both(monkeypatch, run))
+
+
+@pytest.mark.parametrize("name", ["residual", "gated residual"])
+@pytest.mark.parametrize("which", [0, 1])
+def test_one_output_of_the_residual_norm(monkeypatch, name, which):
+    def run():
+        call, inputs = cases()[name]
+        o = call()[which]
+        return list(torch.autograd.grad(o, inputs, torch.ones_like(o), allow_unused=True))
+
+    same(*both(monkeypatch, run))
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_hooks_on_saved_tensors(monkeypatch, name):
+    def run():
+        call, inputs = cases()[name]
+        packed = []
+
+        def pack(t):
+            packed.append((tuple(t.shape), t.dtype))
+            return t.cpu()
+
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(DEV)):
+            o = outs(call())
+        return packed, o + list(torch.autograd.grad(o, inputs, [torch.ones_like(t) for t in o]))
+
+    (packed, a), (packed_python, b) = both(monkeypatch, run)
+    assert packed == packed_python and packed
+    if name != "rope heads view":            # a copy through the host loses the view's strides, and with them the bits' order
+        same(a, b)
+
+    class Stop(Exception):
+        pass
+
+    def stop(t):
+        raise Stop
+
+    with pytest.raises(Stop), torch.autograd.graph.saved_tensors_hooks(stop, lambda t: t):
+        cases()[name][0]()
+
+
+@pytest.mark.parametrize("reentrant", [False, True])
+@pytest.mark.parametrize("name", NAMES)
+def test_checkpointed(monkeypatch, name, reentrant):
+    from torch.utils.checkpoint import checkpoint
+
+    def run():
+        call, inputs = cases()[name]
+        o = outs(checkpoint(lambda *a: call(), *inputs, use_reentrant=reentrant))
+        torch.autograd.backward(o, [torch.ones_like(t) for t in o])
+        return o + [t.grad for t in inputs]
+
+    same(*both(monkeypatch, run))
+
+
+def raised(f):
+    try:
+        f()
+    except Exception as e:
+        return type(e)
+    return None
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_refusals_are_the_same(monkeypatch, name):
+    from torch.autograd import forward_ad
+    call, inputs = cases()[name]
+
+    def twice():
+        o = outs(call())
+        torch.autograd.backward(o, [torch.ones_like(t) for t in o])
+        torch.autograd.backward(o, [torch.ones_like(t) for t in o])
+
+    def changed():
+        o = outs(call())
+        with torch.no_grad():
+            for t in inputs:
+                t.mul_(1.0)
+        torch.autograd.backward(o, [torch.ones_like(t) for t in o])
+
+    def output_changed():
+        o = outs(call())
+        o[0].mul_(2.0)
+
+    def second_order():
+        o = outs(call())
+        g = torch.autograd.grad(o, inputs[:1], [torch.ones_like(t) for t in o], create_graph=True)
+        g[0].sum().backward()
+
+    def dual():
+        import teletron_amd as T
+        with forward_ad.dual_level():
+            x = forward_ad.make_dual(torch.ones(2, 8, C, device=DEV, dtype=torch.bfloat16), torch.ones(2, 8, C, device=DEV, dtype=torch.bfloat16))
+            w = inputs[0].new_ones(C)
+            return T.AdaLNModelFunction.apply(x, w, w, EPS, C)
+
+    def vmapped():
+        import teletron_amd as T
+        w = inputs[0].new_ones(C)
+        torch.func.vmap(lambda t: T.RMSNormModelFunction.apply(t, w, EPS, C))(torch.ones(2, 8, C, device=DEV, dtype=torch.bfloat16))
+
+    def functional_grad():
+        import teletron_amd as T
+        w = inputs[0].new_ones(C)
+        torch.func.grad(lambda t: T.RMSNormModelFunction.apply(t, w, EPS, C).float().sum())(torch.ones(8, C, device=DEV, dtype=torch.bfloat16))
+
+    for f in (twice, changed, output_changed, second_order, dual, vmapped, functional_grad):
+        a, b = both(monkeypatch, lambda: raised(f))
+        assert a == b, f.__name__
+        if f is twice:
+            assert a is RuntimeError
+
+
+def test_wrong_arguments_are_named_as_before():
+    import teletron_amd as T
+    x, w = leaf(2, 8, 64, seed=0), leaf(64, seed=1)
+    with pytest.raises(ValueError):
+        T.AdaLNModelFunction.apply(x, w, w, EPS, 32)
+    with pytest.raises(ValueError):
+        T.AdaLNModelFunction.apply(x, leaf(1, 8, 64, seed=2), leaf(1, 8, 64, seed=3), EPS, 64)
+    with pytest.raises(TypeError):
+        T.RMSNormModelFunction.apply(x.float(), w, EPS, 64)
+    with pytest.raises(TypeError):
+        T.RMSNormModelFunction.apply(x, w, EPS)
+    with pytest.raises(ValueError):
+        T.RMSNormModelFunction.apply(x.cpu(), w.cpu(), EPS, 64)
+
+
+def test_subclasses_keep_their_own_forward():
+    import teletron_amd as T
+
+    class Mine(T.RMSNormModelFunction):
+        @staticmethod
+        def forward(ctx, x, weight, epsilon, cols):
+            return x.clone()
+
+    x, w = leaf(4, 64, seed=0), leaf(64, seed=1)
+    assert torch.equal(Mine.apply(x, w, EPS, 64), x)
+
+
+def test_threads_and_streams():
+    """Passes of several threads, each on a stream of its own, give what one alone gives."""
+    want = {n: [t.clone() for t in step(n)] for n in NAMES}
+    failed = []
+
+    def work(n):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(10):
+                    got = step(n)
+                    torch.cuda.current_stream().synchronize()
+                    same(got, want[n])
+        except BaseException as e:
+            failed.append((n, e))
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(n,)) for n in NAMES]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not failed, failed
+
+
+def step(name):
+    call, inputs = cases()[name]
+    o = outs(call())
+    return o + list(torch.autograd.grad(o, inputs, [torch.ones_like(t) for t in o]))
