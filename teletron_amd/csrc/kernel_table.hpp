@@ -222,9 +222,14 @@ KernelInfo info_fwd_rope_wide() {
   constexpr int R = fwd_wide_R(W, P), Q = fwd_wide_Q(W, P);
   return {reinterpret_cast<const void*>(&norm_fwd_wide<kRMS, W, P, R, Q, kernel_rows(W, P, ROWS, false), true>), 64 * W * Q, Q * R, P * R};
 }
+// Twelve waves where a lane holds two packs: the table's 64 bytes a pack make a lane's loads slower to come back than
+// those of the plain backward, whose six to eight waves stream its x and dy (3072 columns 355 us with six, 372 with
+// twelve).  us, bwd_wide_Q -> this: 60000 x 3072 191.6 -> 177.4, 86646 x 3072 273.8 -> 258.3, 40000 x 4096 163.5 ->
+// 158.7, 40000 x 6144 252.7 -> 239.2; 5120 columns have ten either way.  One pack a lane is as fast or slower with other counts.
+constexpr int bwd_rope_wide_Q(int W, int P) { return P == 2 && W <= 12 ? 12 / W : bwd_wide_Q(W, P); }
 template <int W, int P, int ROWS>
 KernelInfo info_bwd_rope_wide() {
-  constexpr int R = bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
+  constexpr int R = bwd_wide_R(W, P), Q = bwd_rope_wide_Q(W, P);
   return {reinterpret_cast<const void*>(&norm_bwd_wide<kRMS, W, P, R, Q, kernel_rows(W, P, ROWS, false), true>), 64 * W * Q, Q * R, P * R};
 }
 template <int L, int ROWS>

@@ -1,0 +1,26 @@
+"""Widths whose workgroups hold more row groups than the others of their kernels: rows that are no multiple of a tile,
+one row, several tiles a workgroup."""
+import pytest
+import torch
+
+from test_gpu_parity import DEV, check_adaln, check_rmsnorm, rand_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+# 3, 4 and 6 waves of two packs: full rows and ones with idle lanes
+@pytest.mark.parametrize("heads", [17, 20, 24, 25, 32, 41, 48])
+@pytest.mark.parametrize("b,s", [(1, 1), (3, 7), (2, 1601)])
+def test_rotary_backward(heads, b, s):
+    from oracle import norm_oracle as O
+    from teletron_amd import ops
+    from test_gpu_parity import assert_bf16_close, assert_grad_close
+    c = heads * 128
+    x, dy = rand_bf16(b, s, c, seed=heads), rand_bf16(b, s, c, seed=heads + 1)
+    w = rand_bf16(c, seed=heads + 2, scale=0.1, offset=1.0)
+    ang = 3.0 * torch.randn(s, 64, generator=torch.Generator().manual_seed(s))
+    table = torch.stack([ang.cos(), ang.sin()], dim=-1)
+    dx, dw = ops.rmsnorm_rope_backward(dy.to(DEV), x.to(DEV), w.to(DEV), table.to(DEV), 1e-6, 128)
+    dxo, dwo = O.rmsnorm_rope_backward(dy, x, w, table, 1e-6, 128)
+    assert_bf16_close(dx, dxo, "dx")
+    assert_grad_close(dw, dwo, b * s, "dweight")
