@@ -79,6 +79,28 @@ constexpr int bwd_wide_Q(int W, int P) {
   return q;
 }
 
+// Ragged rows (kRagged): their stores and the lines that they share are slower, and more row groups a workgroup
+// hide it on these variants.  us at the groups of whole-line rows -> with these, 400 MB tensors:
+//   AdaLN / RMSNorm forward    1000 columns 140 / 137 -> 136 / 135,  1912: 149 / 148 -> 137 / 137;  AdaLN 4600: 139 -> 128
+//   and backward               3080: 226 / 201 -> 193 / 191,  3536: 204 / 200 -> 188 / 189,  4088: 197 / 195 -> 190 / 187
+//   gate, either way           2200: 210 -> 190,  2600: 200 -> 188,  3080: 198 -> 189,  3536: 198 -> 189,  4088: 193 -> 188
+//   residual + norm forward    1912 columns, ungated (267 MB) / gated (200 MB) 199 / 140 -> 183 / 133,  1416 gated 138 -> 134
+// and in the caches as before or faster (6 MB, forward: AdaLN 4600 7.3 -> 5.5, RMSNorm 1000 5.5 -> 4.6).  Not taken: forward and
+// AdaLN backward of 2056 to 3064 columns (2200: 233 -> 217, but 2600: 205 -> 223); residual + norm forward with two packs a
+// lane (4600: 187 -> 175, but 6 MB 6.4 -> 8.6); one pack a lane in the other backward kernels (no gain); residual backward
+// (170 registers and more).
+constexpr int ragged_fwd_Q(Kind kind, int W, int P, int rows) {
+  if (row_mode(rows) != kRagged) return fwd_wide_Q(W, P);
+  return P == 1 && W == 2 ? 8 : P == 1 && W == 4 ? 4 : kind == kAdaLN && P == 2 && W == 5 ? 3 : fwd_wide_Q(W, P);
+}
+constexpr int ragged_bwd_Q(Kind kind, int W, int P, int rows) {
+  if (row_mode(rows) != kRagged) return bwd_wide_Q(W, P);
+  return P == 2 && W == 4 ? 3 : kind == kRMS && P == 1 && W == 2 ? 8 : bwd_wide_Q(W, P);
+}
+constexpr int ragged_gate_Q(int W, int P, int rows) {
+  return row_mode(rows) == kRagged && P == 2 && (W == 3 || W == 4) ? 12 / W : bwd_wide_Q(W, P);
+}
+
 // Index of the wide variant for `packs` (> kNarrowMaxPacks), or -1.
 inline int select_wide(int packs) {
   int best = -1, best_slots = 1 << 30;
@@ -97,12 +119,12 @@ inline int select_narrow(int packs) {
 
 template <int KIND, int W, int P, int ROWS>
 KernelInfo info_fwd_wide() {
-  constexpr int R = fwd_wide_R(W, P), Q = fwd_wide_Q(W, P);
+  constexpr int R = fwd_wide_R(W, P), Q = ragged_fwd_Q(static_cast<Kind>(KIND), W, P, ROWS);
   return {reinterpret_cast<const void*>(&norm_fwd_wide<KIND, W, P, R, Q, kernel_rows(W, P, ROWS, short_rows(W, P))>), 64 * W * Q, Q * R, P * R};
 }
 template <int KIND, int W, int P, int ROWS>
 KernelInfo info_bwd_wide() {
-  constexpr int R = KIND == kAdaLN ? adaln_bwd_wide_R(W, P, ROWS) : bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
+  constexpr int R = KIND == kAdaLN ? adaln_bwd_wide_R(W, P, ROWS) : bwd_wide_R(W, P), Q = ragged_bwd_Q(static_cast<Kind>(KIND), W, P, ROWS);
   return {reinterpret_cast<const void*>(&norm_bwd_wide<KIND, W, P, R, Q, kernel_rows(W, P, ROWS, short_rows(W, P))>), 64 * W * Q, Q * R, P * R};
 }
 template <int KIND, int W, int P, int ROWS>
@@ -304,7 +326,7 @@ inline KernelInfo lookup_rope(bool narrow, bool backward, int idx, int rows, int
 
 template <int MODE, int W, int P, int ROWS>
 KernelInfo info_gate_wide() {
-  constexpr int R = bwd_wide_R(W, P), Q = bwd_wide_Q(W, P);
+  constexpr int R = bwd_wide_R(W, P), Q = ragged_gate_Q(W, P, ROWS);
   return {reinterpret_cast<const void*>(&gate_wide<MODE, W, P, R, Q, kernel_rows(W, P, ROWS, false)>), 64 * W * Q, Q * R, P * R};
 }
 template <int MODE, int L, int ROWS>
@@ -350,9 +372,13 @@ constexpr int res_fwd_Q(int W, int P) {
 constexpr int res_bwd_Q(int W, int P, bool gated) {
   return res_waves_Q(W, P);
 }
+constexpr int ragged_res_fwd_Q(int W, int P, int rows, bool gated) {   // see ragged_fwd_Q
+  if (row_mode(rows) != kRagged || P != 1) return res_fwd_Q(W, P);
+  return W == 4 ? 4 : gated && W == 3 ? 5 : res_fwd_Q(W, P);
+}
 template <bool GATED, int W, int P, int ROWS>
 KernelInfo info_res_fwd() {
-  constexpr int R = 1, Q = res_fwd_Q(W, P);
+  constexpr int R = 1, Q = ragged_res_fwd_Q(W, P, ROWS, GATED);
   return {reinterpret_cast<const void*>(&resnorm_fwd_wide<W, P, R, Q, GATED ? row_mode(ROWS) : kernel_rows(W, P, ROWS, short_rows(W, P)), GATED>), 64 * W * Q, Q * R, P * R};
 }
 template <bool GATED, int W, int P, int ROWS>

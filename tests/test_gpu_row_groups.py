@@ -24,3 +24,18 @@ def test_rotary_backward(heads, b, s):
     dxo, dwo = O.rmsnorm_rope_backward(dy, x, w, table, 1e-6, 128)
     assert_bf16_close(dx, dxo, "dx")
     assert_grad_close(dw, dwo, b * s, "dweight")
+
+
+# ragged rows: the shortest and the longest of the variants of 2, 3 and 4 waves of one pack, 3, 4 and 5 of two
+@pytest.mark.parametrize("cols", [520, 1000, 1032, 1528, 1544, 2040, 2056, 3064, 3080, 4088, 4104, 5112])
+@pytest.mark.parametrize("nb,rpb", [(1, 1), (2, 31), (1, 1901)])
+def test_ragged_rows(cols, nb, rpb):
+    from test_gpu_gate import test_gate_residual_shapes as check_gate
+    from test_gpu_resnorm import run_case as check_residual
+    x, dy = rand_bf16(nb, rpb, cols, seed=cols), rand_bf16(nb, rpb, cols, seed=cols + 1)
+    p = [rand_bf16(nb, 1, cols, seed=cols + 2 + i, scale=0.2) for i in range(2)]
+    check_adaln(x, p[0], p[1], dy, 1e-6, nb, f"cols {cols}")
+    check_rmsnorm(x, 1 + p[0][0, 0], dy, 1e-6, f"cols {cols}")
+    check_gate(cols, nb, rpb)
+    for gated in (False, True):
+        check_residual(cols, nb, rpb, gated, affine=False)
