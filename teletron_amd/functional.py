@@ -80,6 +80,9 @@ def _adaln_backward(ctx, grad_output, grad_reduce=None):
     return dx, dscale, dshift
 
 
+_python_apply = Function.apply.__func__    # torch.compile follows this call, but not super() of a Function
+
+
 class NativeFirst(Function):
     """A Function whose ``apply`` is one native call (csrc/torch_ext/native_ops.cpp) where its arguments are what a model
     passes in earnest: forward and graph node there, backward on the engine's thread without the interpreter.  What
@@ -87,22 +90,24 @@ class NativeFirst(Function):
     classes), takes ``forward`` and ``backward`` below, which do the same.
 
     A short pass is host time.  us of one through the Python classes -> through native nodes, of which the engine's
-    hand-over to its thread and back takes about 25: RMSNorm 512 x 5120 75 -> 58, 2 x 4096 x 1536 77 -> 60, AdaLN
-    3 x 5000 x 1000 86 -> 65, gated residual + norm 4 x 1000 x 2048 123 -> 84; AdaLN 256 x 3072 without gradients
-    10.4 -> 7.0."""
+    hand-over to its thread and back takes about 25: RMSNorm 512 x 5120 78 -> 56, 2 x 4096 x 1536 80 -> 60, AdaLN
+    3 x 5000 x 1000 87 -> 67, gate 512 x 5120 80 -> 60, gated residual + norm 512 x 5120 119 -> 90; AdaLN 256 x 3072
+    without gradients 10.6 -> 6.7."""
 
     _native = None      # name of the native function, of the class that names it and not of its subclasses
 
     @classmethod
     def apply(cls, *args):
+        if torch.compiler.is_compiling():
+            return _python_apply(cls, *args)
         name = cls.__dict__.get("_native")
-        if name and args and not (torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active()):
+        if name and args and not torch._C._are_functorch_transforms_active():
             native = ops.native(args[0])
             if native:
                 out = getattr(native, name)(*args)
                 if out is not None:
                     return out
-        return super().apply(*args)
+        return _python_apply(cls, *args)
 
 
 class AdaLNModelFunction(NativeFirst):

@@ -283,3 +283,21 @@ def step(name):
     call, inputs = cases()[name]
     o = outs(call())
     return o + list(torch.autograd.grad(o, inputs, [torch.ones_like(t) for t in o]))
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_compiled(name):
+    """torch.compile goes round the operators: the same results as without it."""
+    call, inputs = cases()[name]
+
+    def step():
+        return [2 * t for t in outs(call())]
+
+    want = step()
+    grads = [rand_bf16(*t.shape, seed=20 + i).to(DEV) for i, t in enumerate(want)]
+    want += torch.autograd.grad(want, inputs, grads)
+    torch._dynamo.reset()
+    compiled = torch.compile(step, backend="eager")
+    for _ in range(2):
+        got = compiled()
+        same([*got, *torch.autograd.grad(got, inputs, grads)], want)
