@@ -192,7 +192,7 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   // throughput peaks near kFwdLoadsPerCu / kBwdLoadsPerCu outstanding 128-bit loads per lane
   // column of a CU (waves x loads per lane) and streamed tensor, falls off by 10-20 % at full
   // occupancy, and is a few percent better with one CU in 32 left without a workgroup.
-  // Tensors that fit the caches just take the whole machine.
+  // Tensors that fit the caches take what fits a CU, or one workgroup (max_x below).
   int usable_cus = cus;
   if (!cache_resident) {
     const int per_wg = (k.threads / kWave) * k.lane_loads;

@@ -15,7 +15,7 @@ constexpr int kWave = 64;   // CDNA wavefront width
 constexpr int kPack = 8;    // bf16 elements per 128-bit pack
 
 // ---------------------------------------------------------------- memory
-// Streaming tensors are touched exactly once, so they bypass cache retention: "nt" global
+// A kernel touches each value of a streaming tensor once, so tensors beyond the caches bypass their retention: "nt" global
 // loads, and stores with system scope on top ("sc0 sc1 nt": written through instead of being
 // kept in L2), which measured 1-2 % faster than plain "nt" stores under the 2-reads-1-write mix
 // of the backward kernels.  The compiler's builtin only offers "nt", hence the asm for stores;
