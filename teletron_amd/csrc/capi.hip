@@ -572,8 +572,10 @@ int reduce(void* out0, void* out1, const void* workspace, int n_batches, int n_p
       cols > TT_MAX_COLS || n_acc < 1 || n_acc > 3 || (n_acc >= 2 && !out1) || (n_acc == 3 && !out2))
     return TT_ERR_INVALID_ARGUMENT;
   // 32 columns a workgroup where 64 would leave CUs without one (see reduce_partials); with many batches, which have
-  // few partials each, it would only double the idle waves (300 batches of 5120 columns 58 -> 118 us).
-  const bool wide = (cols + 63) / 64 * n_batches >= 256;
+  // few partials each, it would only double the idle waves (300 batches of 5120 columns 58 -> 118 us).  Up to 128 partials
+  // are one round of loads at 64 columns as well: us at 32 -> 64, three sums each, 85 partials of 3 x 5120 6.3 -> 4.8, 82 of
+  // 3 x 3072 6.0 -> 4.7, 62 of 4 x 3072 6.0 -> 4.7, 50 of 2 x 5120 6.5 -> 4.3; one batch or fewer sums 0.0 to 0.2 faster.
+  const bool wide = (cols + 63) / 64 * n_batches >= 256 || n_partials <= 128;
   const int lc = wide ? 64 : 32;
   const dim3 grid((unsigned)((cols + lc - 1) / lc), (unsigned)n_batches, 1);
   using Kernel = void (*)(void*, void*, void*, const float*, int, int, int);
