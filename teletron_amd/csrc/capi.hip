@@ -215,9 +215,18 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   // RMSNorm 3000 x 3072 15.3 + 3.8 -> 13.6 + 3.8, with the rotary embedding 5000 x 3072 23.7 + 3.9 -> 21.2 + 3.9.
   // Not where over a quarter of the lanes are idle: one workgroup then has too little in flight (RMSNorm 19660 x 640
   // 17.9 -> 19.7 with the reduction), nor for narrow rows, whose partial sums are small (40 heads of 128 x 3000 17 -> 22).
+  // Nor where the batches divide the CUs so badly that over a quarter of them would go without a workgroup.  Backward +
+  // reduction, as many as fit | whole workgroups a batch up to one a CU | rounded up to one a CU:
+  //   140 x 60 x 3072 (140 of 256 CUs): residual + norm 46.3 + 18.2 | 52.4 + 17.8 | 62.1 + 18.2, gate 24.8 + 14.4 | 31.7 + 13.3 | 26.4 + 14.1
+  //   86 x 90 x 3072 (172): residual + norm 40.6 + 13.2 | 43.1 + 11.8 | 58.4 + 12.5, gate 23.2 + 9.8 | 24.0 + 9.2 | 24.9 + 9.5
+  //   100 x 50 x 3072 (200): residual + norm 28.5 + 14.9 | 29.5 + 13.3 | 36.4 + 13.4, gate 15.9 + 10.9 | 14.8 + 10.4 | 16.5 + 10.6
+  //   43 x 45 x 3072 (215): residual + norm 15.0 + 9.2 | 13.3 + 7.2, gate 7.5 + 7.5 | 7.7 + 6.3;  AdaLN within 2 % everywhere
+  // (Rounded up, a few CUs have two workgroups, and all the others wait for them.)
   // Workspaces stay sized for grid_x, so that sizes asked for once hold.
-  if (ov <= 0 && cache_resident && !narrow && (dir == kBwd || dir == kBwdSaved) && packs * 4 >= slots * 3)
-    plan->max_x = rows / rows_per_batch < cus ? (int)(cus / (rows / rows_per_batch)) : 1;
+  const int64_t groups = rows / rows_per_batch, per_group = groups <= cus ? cus / groups : 0;
+  if (ov <= 0 && cache_resident && !narrow && (dir == kBwd || dir == kBwdSaved) && packs * 4 >= slots * 3 &&
+      per_group * groups * 4 >= (int64_t)cus * 3)
+    plan->max_x = (int)per_group;
 
   // Tensors that fit the caches are read with ordinary loads (kKeep; the plan is that of the other kernel).  As fast
   // as streaming loads on inputs that no cache holds, and the next kernel to read them finds them there (forward, then

@@ -14,18 +14,40 @@ def test_residual_norm_backward_keeps_one_workgroup_a_cu(lib, rows, cols):
     assert lib.tt_residual_norm_backward_workspace_bytes(rows, cols, rows, 0) == cus * 2 * cols * 4
 
 
-@pytest.mark.parametrize("rows,cols,nb", [(2000, 3072, 1), (9000, 3072, 3), (1200, 5128, 1), (3000, 1536, 2), (600, 512, 600)])
-def test_cached_backward_of_wide_rows_runs_one_workgroup_a_cu(lib, rows, cols, nb):
-    """... and no more than the size query's answer; rows with over a quarter of their lanes idle keep theirs."""
+def partials_a_batch(lib, rows, cols, nb, op="adaln"):
+    """Workgroups a batch that the backward of a norm launches, and the size query's answer."""
     import ctypes
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
     x, dy, dx = (torch.ones(rows, cols, dtype=torch.bfloat16, device="cuda:0") for _ in range(3))
     p = torch.ones(nb, cols, dtype=torch.bfloat16, device="cuda:0")
-    need = lib.tt_adaln_backward_workspace_bytes(rows, cols, rows // nb)
+    shape = [rows, cols, rows // nb] if op == "adaln" else [rows, cols]
+    need = getattr(lib, f"tt_{op}_backward_workspace_bytes")(*shape)
     ws = torch.empty(need, dtype=torch.uint8, device="cuda:0")
     n = ctypes.c_int(0)
-    args = [dx.data_ptr(), dy.data_ptr(), x.data_ptr(), p.data_ptr(), ws.data_ptr()]
-    tail = [rows, cols, rows // nb, 1e-6, torch.cuda.current_stream().cuda_stream]
-    assert lib.tt_adaln_backward_partials(*args, need, ctypes.byref(n), *tail) == 0
+    args = [dx.data_ptr(), dy.data_ptr(), x.data_ptr(), p.data_ptr(), ws.data_ptr(), need, ctypes.byref(n)]
+    assert getattr(lib, f"tt_{op}_backward_partials")(*args, *shape, 1e-6, torch.cuda.current_stream().cuda_stream) == 0
     torch.cuda.synchronize()
-    assert 1 <= n.value <= max(1, cus // nb) and n.value * nb * 2 * cols * 4 <= need
+    return n.value, need
+
+
+@pytest.mark.parametrize("rows,cols,nb", [(2000, 3072, 1), (9000, 3072, 3), (1200, 5128, 1), (3000, 1536, 2), (4300, 3072, 43),
+                                          (60 * 200, 1536, 200)])
+def test_cached_backward_of_wide_rows_runs_one_workgroup_a_cu(lib, rows, cols, nb):
+    """... and no more than the size query's answer, at most a quarter of the CUs going without."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n, need = partials_a_batch(lib, rows, cols, nb)
+    assert n == cus // nb and n * nb * 4 >= cus * 3 and n * nb * 2 * cols * 4 <= need
+
+
+@pytest.mark.parametrize("nb", [86, 129, 140, 190, 300])
+def test_batches_that_divide_the_cus_badly_keep_every_cu(lib, nb):
+    """One workgroup a CU in whole workgroups a batch would leave over a quarter of the CUs without one."""
+    cus, cols, rpb = torch.cuda.get_device_properties(0).multi_processor_count, 2312, 20
+    assert cus // nb * nb * 4 < cus * 3
+    n, need = partials_a_batch(lib, rpb * nb, cols, nb)
+    assert n * nb >= cus * 3 // 4 and n * nb * 2 * cols * 4 <= need
+
+
+def test_rows_with_idle_lanes_keep_their_workgroups(lib):
+    """Over a quarter of the lanes without a pack: as many workgroups as fit a CU."""
+    n, _ = partials_a_batch(lib, 19660, 640, 1, "rmsnorm")
+    assert n > torch.cuda.get_device_properties(0).multi_processor_count
