@@ -205,6 +205,7 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
     if (cus >= 32) usable_cus = cus - cus / 32;
   }
   const int ov = g_wgs_per_cu_override.load(std::memory_order_relaxed);
+  const int gov = g_grid_override.load(std::memory_order_relaxed);
   if (ov > 0) per_cu = ov;
   if (per_cu > kMaxWgsPerCu) per_cu = kMaxWgsPerCu;
 
@@ -224,7 +225,7 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   // (Rounded up, a few CUs have two workgroups, and all the others wait for them.)
   // Workspaces stay sized for grid_x, so that sizes asked for once hold.
   const int64_t groups = rows / rows_per_batch, per_group = groups <= cus ? cus / groups : 0;
-  if (ov <= 0 && cache_resident && !narrow && (dir == kBwd || dir == kBwdSaved) && packs * 4 >= slots * 3 &&
+  if (ov <= 0 && gov <= 0 && cache_resident && !narrow && (dir == kBwd || dir == kBwdSaved) && packs * 4 >= slots * 3 &&
       per_group * groups * 4 >= (int64_t)cus * 3)
     plan->max_x = (int)per_group;
 
@@ -244,7 +245,6 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   if (plan->n_batches > 65535) return TT_ERR_UNSUPPORTED;
   int64_t gx = (int64_t)per_cu * usable_cus / plan->n_batches;
   if (gx < 1) gx = 1;
-  const int gov = g_grid_override.load(std::memory_order_relaxed);
   if (gov > 0 && gov <= kMaxWgsPerCu * cus) gx = gov / plan->n_batches > 0 ? gov / plan->n_batches : 1;
   if (gx > plan->n_tiles) gx = plan->n_tiles;
   plan->grid_x = static_cast<int>(gx);
