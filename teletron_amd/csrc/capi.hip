@@ -584,7 +584,10 @@ int reduce(void* out0, void* out1, const void* workspace, int n_batches, int n_p
   // few partials each, it would only double the idle waves (300 batches of 5120 columns 58 -> 118 us).  Up to 128 partials
   // are one round of loads at 64 columns as well: us at 32 -> 64, three sums each, 85 partials of 3 x 5120 6.3 -> 4.8, 82 of
   // 3 x 3072 6.0 -> 4.7, 62 of 4 x 3072 6.0 -> 4.7, 50 of 2 x 5120 6.5 -> 4.3; one batch or fewer sums 0.0 to 0.2 faster.
-  const bool wide = (cols + 63) / 64 * n_batches >= 256 || n_partials <= 128;
+  int cus = 0;
+  const int rc = current_device_cus(&cus);
+  if (rc != TT_OK) return rc;
+  const bool wide = (cols + 63) / 64 * n_batches >= cus || n_partials <= 128;
   const int lc = wide ? 64 : 32;
   const dim3 grid((unsigned)((cols + lc - 1) / lc), (unsigned)n_batches, 1);
   using Kernel = void (*)(void*, void*, void*, const float*, int, int, int);
