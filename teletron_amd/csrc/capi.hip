@@ -584,10 +584,13 @@ int reduce(void* out0, void* out1, const void* workspace, int n_batches, int n_p
   // few partials each, it would only double the idle waves (300 batches of 5120 columns 58 -> 118 us).  Up to 128 partials
   // are one round of loads at 64 columns as well: us at 32 -> 64, three sums each, 85 partials of 3 x 5120 6.3 -> 4.8, 82 of
   // 3 x 3072 6.0 -> 4.7, 62 of 4 x 3072 6.0 -> 4.7, 50 of 2 x 5120 6.5 -> 4.3; one batch or fewer sums 0.0 to 0.2 faster.
+  // So do long rows of partial sums that are no whole lines, which two workgroups of 32 columns share: 256 partials, three |
+  // two sums, 32 -> 64 columns, 4616 columns 5.7 -> 5.8 | 4.8 -> 4.2, 5640: 6.4 -> 5.9 | 4.8 -> 4.2, 8184: 8.3 -> 7.1 | 5.8 -> 5.0;
+  // the other way round at 4104 (5.4 -> 5.6 | 4.1 -> 4.6) and 3080 (4.7 -> 5.6 | 4.0 -> 4.1).
   int cus = 0;
   const int rc = current_device_cus(&cus);
   if (rc != TT_OK) return rc;
-  const bool wide = (cols + 63) / 64 * n_batches >= cus || n_partials <= 128;
+  const bool wide = (cols + 63) / 64 * n_batches >= cus || n_partials <= 128 || (cols % 32 != 0 && cols > 4608);
   const int lc = wide ? 64 : 32;
   const dim3 grid((unsigned)((cols + lc - 1) / lc), (unsigned)n_batches, 1);
   using Kernel = void (*)(void*, void*, void*, const float*, int, int, int);

@@ -57,7 +57,7 @@ def test_gate_and_residual_gradients(cols):
 
 # rounds of 8 x 16 and 8 x 32 partials, a last one of a single partial, column counts beside whole workgroups of 32 and 64
 @pytest.mark.parametrize("n_partials", [1, 31, 33, 128, 129, 256, 257, 777])
-@pytest.mark.parametrize("n_batches,cols", [(1, 1), (1, 33), (1, 128), (1, 5128), (2, 8191), (3, 5120), (300, 72), (70, 300)])
+@pytest.mark.parametrize("n_batches,cols", [(1, 1), (1, 33), (1, 128), (1, 4600), (1, 4616), (1, 5128), (2, 8191), (3, 5120), (300, 72), (70, 300)])
 @pytest.mark.parametrize("n_acc", [1, 2])
 def test_reduction(lib, n_partials, n_batches, cols, n_acc):
     """Any order of n additions is off by at most n 2^-24 sum |x|."""
