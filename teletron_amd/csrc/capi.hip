@@ -216,6 +216,10 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   // RMSNorm 3000 x 3072 15.3 + 3.8 -> 13.6 + 3.8, with the rotary embedding 5000 x 3072 23.7 + 3.9 -> 21.2 + 3.9.
   // Not where over a quarter of the lanes are idle: one workgroup then has too little in flight (RMSNorm 19660 x 640
   // 17.9 -> 19.7 with the reduction), nor for narrow rows, whose partial sums are small (40 heads of 128 x 3000 17 -> 22).
+  // Nor, beyond 12 MiB, where over a sixteenth of them are, with one pack a lane and two tensors to read: RMSNorm
+  // 1664 columns 15 / 20 / 60 MB 12.0 / 14.4 / 34.9 -> 13.6 / 15.9 / 37.2, 1544: 48 / 60 MB 30.1 / 35.5 -> 31.5 / 38.0, with the
+  // rotary embedding 896: 20 / 60 MB 17.4 / 36.7 -> 18.4 / 39.1, saved AdaLN 392: 33 / 60 MB 24.9 / 41.7 -> 26.6 / 43.8, gate 1160:
+  // 20 MB 14.3 -> 15.2 (up to 8 MB, or with every lane in use, one is the faster there too: RMSNorm 1544 11.4 -> 10.5, 1536 10.4 -> 9.9).
   // Nor where the batches divide the CUs so badly that over a quarter of them would go without a workgroup.  Backward +
   // reduction, as many as fit | whole workgroups a batch up to one a CU | rounded up to one a CU:
   //   140 x 60 x 3072 (140 of 256 CUs): residual + norm 46.3 + 18.2 | 52.4 + 17.8 | 62.1 + 18.2, gate 24.8 + 14.4 | 31.7 + 13.3 | 26.4 + 14.1
@@ -226,6 +230,7 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   // Workspaces stay sized for grid_x, so that sizes asked for once hold.
   const int64_t groups = rows / rows_per_batch, per_group = groups <= cus ? cus / groups : 0;
   if (ov <= 0 && gov <= 0 && cache_resident && !narrow && (dir == kBwd || dir == kBwdSaved) && packs * 4 >= slots * 3 &&
+      (res || kWideP[idx] > 1 || packs * 16 >= slots * 15 || rows * cols * 2 < (int64_t)12 << 20) &&
       per_group * groups * 4 >= (int64_t)cus * 3)
     plan->max_x = (int)per_group;
 
