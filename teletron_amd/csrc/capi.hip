@@ -143,9 +143,11 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   if (idx < 0) return TT_ERR_UNSUPPORTED;
   const int slots = narrow ? kNarrowL[idx] : 64 * kWideW[idx] * kWideP[idx];
   const bool full = (slots == packs);
-  // a row of whole 128-byte lines or not: see enum Rows
-  const int mode = odd ? kOdd : full ? kFull : (cols * 2) % 128 == 0 || force == kMasked ? kMasked : kRagged;
   const bool cache_resident = rows * cols * 2 < (int64_t)64 << 20;
+  // a row of whole 128-byte lines or not: see enum Rows
+  int mode = odd ? kOdd : full ? kFull : (cols * 2) % 128 == 0 || force == kMasked ? kMasked : kRagged;
+  if (mode == kRagged)
+    mode |= (cache_resident ? kCached : 0) | (packs * 4 < slots * 3 ? kIdle : packs * 16 >= slots * 15 ? kDense : 0);
   if (res && (narrow || kind != kAdaLN || dir == kBwdSaved || dir == kFwdXn)) return TT_ERR_UNSUPPORTED;
   if (rope) {
     if (kind != kRMS || dir == kBwdSaved || dir == kFwdXn) return TT_ERR_UNSUPPORTED;

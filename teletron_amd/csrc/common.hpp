@@ -61,6 +61,11 @@ enum Rows : int {
   // Added to the others (and to kFull / kMasked of the narrow kernels): the activations are read with ordinary loads,
   // so that tensors which fit the caches stay there for the next kernel that reads them.
   kKeep = 4,
+  // Added to kRagged, for the row groups a workgroup (ragged_fwd_Q and the rules after it): the tensor fits the caches;
+  // over a quarter, or at most a sixteenth, of the lane slots hold no pack.
+  kCached = 8,
+  kIdle = 16,
+  kDense = 32,
 };
 constexpr int row_mode(int rows) { return rows & 3; }
 constexpr bool keeps(int rows) { return (rows & kKeep) != 0; }
@@ -82,7 +87,8 @@ constexpr bool keeps(int rows) { return (rows & kKeep) != 0; }
 constexpr bool short_rows(int W, int P) { return W * P <= 6; }
 // The instantiation that stands for `rows`: kKeep goes where the loads are ordinary ones anyway, and above 6144 columns.
 constexpr int kernel_rows(int W, int P, int rows, bool is_short) {
-  return W * P > 12 || (row_mode(rows) == kRagged && is_short) || row_mode(rows) == kOdd ? row_mode(rows) : rows;
+  return W * P > 12 || (row_mode(rows) == kRagged && is_short) || row_mode(rows) == kOdd ? row_mode(rows)
+                                                                                          : row_mode(rows) | (rows & kKeep);
 }
 
 template <int ROWS, bool SHORT, bool KEEP>

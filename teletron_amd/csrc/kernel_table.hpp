@@ -80,22 +80,33 @@ constexpr int bwd_wide_Q(int W, int P) {
 }
 
 // Ragged rows (kRagged): their stores and the lines that they share are slower, and more row groups a workgroup
-// hide it on these variants.  us at the groups of whole-line rows -> with these, 400 MB tensors:
-//   AdaLN / RMSNorm forward    1000 columns 140 / 137 -> 136 / 135,  1912: 149 / 148 -> 137 / 137;  AdaLN 4600: 139 -> 128
-//   and backward               3080: 226 / 201 -> 193 / 191,  3536: 204 / 200 -> 188 / 189,  4088: 197 / 195 -> 190 / 187
-//   gate, either way           2200: 210 -> 190,  2600: 200 -> 188,  3080: 198 -> 189,  3536: 198 -> 189,  4088: 193 -> 188
-//   residual + norm forward    1912 columns, ungated (267 MB) / gated (200 MB) 199 / 140 -> 183 / 133,  1416 gated 138 -> 134
-// and in the caches as before or faster (6 MB, forward: AdaLN 4600 7.3 -> 5.5, RMSNorm 1000 5.5 -> 4.6).  Not taken: forward and
-// AdaLN backward of 2056 to 3064 columns (2200: 233 -> 217, but 2600: 205 -> 223); residual + norm forward with two packs a
-// lane (4600: 187 -> 175, but 6 MB 6.4 -> 8.6); one pack a lane in the other backward kernels (no gain); residual backward
-// (170 registers and more).
+// hide it on these variants.  us at the groups of whole-line rows -> with these, 400 MB tensors unless stated:
+//   AdaLN forward      520 columns 211 -> 195,  776: 152 -> 148,  904: 138 -> 138,  1016: 146 -> 135 (eight groups of two waves);
+//                      4104: 152 -> 124,  4616: 142 -> 126,  5112: 133 -> 125 (three of five)
+//   RMSNorm forward    1016: 147 -> 136, and in the caches 520 (20 MB) 11.5 -> 9.3, 904 8.8 -> 8.0; beyond them shorter rows lose
+//                      (520: 167 -> 191, 776: 142 -> 145, 968: 136 -> 138)
+//   AdaLN and RMSNorm forward, four groups of four waves: 1928 columns 149 / 142 -> 136 / 133,  2040: 153 / 150 -> 138 / 135; with more
+//                      lanes idle they lose, most at 80 MB (1544: 29.3 / 28.6 -> 32.8 / 31.6, 1800: 29.7 / 28.8 -> 31.2 / 29.9)
+//   and backward       3080: 226 / 201 -> 193 / 191,  3536: 204 / 200 -> 188 / 189,  4088: 197 / 195 -> 190 / 187
+//   RMSNorm backward   520 (200 MB) 131 -> 115,  648: 114 -> 103,  776: 104 -> 99,  1016: 99 -> 100,  968 (12 MB) 9.0 -> 8.2; in the caches
+//                      with over a quarter of the lanes idle two smaller workgroups a CU are better (520, 31 MB: 18.6 -> 20.6)
+//   gate, either way   2200: 210 -> 190,  2600: 200 -> 188,  3080: 198 -> 189,  3536: 198 -> 189,  4088: 193 -> 188
+//   residual + norm forward beyond the caches: 1544 columns, ungated / gated 272 / 261 -> 278 / 265,  1736: 279 -> 268,
+//                      1928: 269 / 261 -> 260 / 251;  gated 1032: 328 -> 268,  1288: 281 -> 263,  1528: 269 -> 269; in the caches they
+//                      lose (gated 1032, 6 / 20 MB 8.2 / 17.5 -> 8.9 / 18.3; 1864, 20 MB 15.4 -> 16.6)
+// Not taken: forward and AdaLN backward of 2056 to 3064 columns (2200: 233 -> 217, but 2600: 205 -> 223); residual + norm forward
+// with two packs a lane (4600: 187 -> 175, but 6 MB 6.4 -> 8.6); one pack a lane in the other backward kernels (no gain);
+// residual backward (170 registers and more).
 constexpr int ragged_fwd_Q(Kind kind, int W, int P, int rows) {
   if (row_mode(rows) != kRagged) return fwd_wide_Q(W, P);
-  return P == 1 && W == 2 ? 8 : P == 1 && W == 4 ? 4 : kind == kAdaLN && P == 2 && W == 5 ? 3 : fwd_wide_Q(W, P);
+  if (P == 1 && W == 2) return kind == kAdaLN || (rows & (kCached | kDense)) ? 8 : fwd_wide_Q(W, P);
+  if (P == 1 && W == 4) return rows & kDense ? 4 : fwd_wide_Q(W, P);
+  return kind == kAdaLN && P == 2 && W == 5 ? 3 : fwd_wide_Q(W, P);
 }
 constexpr int ragged_bwd_Q(Kind kind, int W, int P, int rows) {
   if (row_mode(rows) != kRagged) return bwd_wide_Q(W, P);
-  return P == 2 && W == 4 ? 3 : kind == kRMS && P == 1 && W == 2 ? 8 : bwd_wide_Q(W, P);
+  if (kind == kRMS && P == 1 && W == 2) return (rows & kCached) && (rows & kIdle) ? bwd_wide_Q(W, P) : 8;
+  return P == 2 && W == 4 ? 3 : bwd_wide_Q(W, P);
 }
 constexpr int ragged_gate_Q(int W, int P, int rows) {
   return row_mode(rows) == kRagged && P == 2 && (W == 3 || W == 4) ? 12 / W : bwd_wide_Q(W, P);
@@ -155,9 +166,15 @@ KernelInfo info_bwd_narrow() {
          : rows == (kFull | kKeep) ? INFO<__VA_ARGS__, kFull | kKeep> CALL    \
          : keeps(rows)             ? INFO<__VA_ARGS__, kMasked | kKeep> CALL  \
                                    : INFO<__VA_ARGS__, kMasked> CALL;
-#define TT_ROWS(INFO, ...)                                          \
-  if (rows == kRagged) return INFO<__VA_ARGS__, kRagged>();         \
-  if (rows == (kRagged | kKeep)) return INFO<__VA_ARGS__, kRagged | kKeep>(); \
+#define TT_LANES(INFO, ROWS, ...)                           \
+  (rows & kIdle    ? INFO<__VA_ARGS__, (ROWS) | kIdle>()    \
+   : rows & kDense ? INFO<__VA_ARGS__, (ROWS) | kDense>()   \
+                   : INFO<__VA_ARGS__, (ROWS)>())
+#define TT_ROWS(INFO, ...)                                                             \
+  if (row_mode(rows) == kRagged)                                                       \
+    return keeps(rows)      ? TT_LANES(INFO, kRagged | kKeep | kCached, __VA_ARGS__)   \
+           : rows & kCached ? TT_LANES(INFO, kRagged | kCached, __VA_ARGS__)           \
+                            : TT_LANES(INFO, kRagged, __VA_ARGS__);                    \
   TT_LINES(INFO, (), __VA_ARGS__)
 #define TT_ROWS_ODD(INFO, ...)                                      \
   if (row_mode(rows) == kOdd) return INFO<__VA_ARGS__, kOdd>();     \
@@ -373,7 +390,7 @@ constexpr int res_bwd_Q(int W, int P, bool gated) {
   return res_waves_Q(W, P);
 }
 constexpr int ragged_res_fwd_Q(int W, int P, int rows, bool gated) {   // see ragged_fwd_Q
-  if (row_mode(rows) != kRagged || P != 1) return res_fwd_Q(W, P);
+  if (row_mode(rows) != kRagged || P != 1 || (rows & kCached)) return res_fwd_Q(W, P);
   return W == 4 ? 4 : gated && W == 3 ? 5 : res_fwd_Q(W, P);
 }
 template <bool GATED, int W, int P, int ROWS>

@@ -8,8 +8,8 @@ pytestmark = pytest.mark.gpu
 EPS = 1e-6
 
 
-# full rows, masked ones of whole cache lines, ragged ones past the short variants, narrow rows
-@pytest.mark.parametrize("cols", [512, 2176, 3080, 5120, 128])
+# full rows, masked ones of whole cache lines, ragged ones (with many, some and few idle lanes, and past the short variants), narrow rows
+@pytest.mark.parametrize("cols", [512, 520, 776, 1000, 1288, 1544, 1928, 2176, 3080, 5120, 128])
 def test_same_bits_on_both_sides_of_the_limit(lib, cols):
     from teletron_amd import ops
     rows, part = (66 << 20) // (2 * cols) + 1, 4 * 211

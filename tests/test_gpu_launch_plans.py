@@ -47,7 +47,7 @@ def test_batches_that_divide_the_cus_badly_keep_every_cu(lib, nb):
     assert n * nb >= cus * 3 // 4 and n * nb * 2 * cols * 4 <= need
 
 
-@pytest.mark.parametrize("rows,cols,capped", [(19660, 640, False), (6009, 1664, False), (2403, 1664, True), (5208, 1920, True),
+@pytest.mark.parametrize("rows,cols,capped", [(19660, 640, False), (19660, 648, False), (6009, 1664, False), (2403, 1664, True), (5208, 1920, True),
                                               (6475, 1544, False), (6510, 1536, True)])
 def test_rows_with_idle_lanes_keep_their_workgroups(lib, rows, cols, capped):
     """Over a quarter of the lanes without a pack, or over a sixteenth beyond 12 MiB: as many workgroups as fit a CU."""
