@@ -242,12 +242,13 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   // -> 6.6 / 11.0, 5000 x 4096 16.1 / 24.5 -> 12.9 / 21.8, RMSNorm 5000 x 1536 7.6 / 11.6 -> 6.2 / 9.4, gate 2500 x 3072 10.4 / 10.4
   // -> 8.8 / 6.2, residual + norm 2000 x 3072 11.9 / 17.0 -> 9.4 / 14.1.  With more tensors a call the limit is lower (means
   // over 28 widths, streaming / kept): residual + norm forward 16 MB 1.11, 17.5 MB 1.02, 20 MB 1.00 (down to 0.94: 2441 x 4096 15.5 -> 16.3,
-  // 1627 x 6144 16.8 -> 17.9), gate forward 48 MB 1.08, 54 MB 1.00, 60 MB 0.97 (25862 x 1160 30.1 -> 33.0; its backward goes with
-  // it: behind a streaming forward 60 MB are 36.2 streaming, 40.5 kept, behind a keeping one 35.0 kept); x_norm
+  // 1627 x 6144 16.8 -> 17.9), gate forward with idle lanes 48 MB 1.05, 53 MB 1.00, 60 MB 0.95 (25862 x 1160 30.1 ->
+  // 33.0; its backward goes with it: behind a streaming forward 36.2 streaming, 40.5 kept, behind a keeping one 35.0 kept), with
+  // every lane in use 60 MB 0.99 and its backward 1.10 (19531 x 1536 31.2 / 32.0 -> 30.6 / 27.0); x_norm
   // forward and its backward 4972 x 3072 18.1 / 21.8 -> 17.0 / 20.9, 9000 x 3072 31.0 / 32.4 -> 30.8 / 33.4; gated, 4000 x 3072
   // 18.8 / 29.1 -> 18.6 / 29.1.  Beyond the caches streaming is the faster (75600 x 5120 374 -> 410).
   const int64_t keep_mib = res == 2 ? 0 : res ? 18 : dir == kFwdXn || dir == kBwdSaved ? 40
-                         : kind == kGateKind ? 52 : 64;
+                         : kind == kGateKind && !full ? 52 : 64;
   plan->k = rows * cols * 2 < keep_mib << 20 ? pick(mode | kKeep) : k;
   plan->packs = packs;
   plan->n_batches = rows / rows_per_batch;
