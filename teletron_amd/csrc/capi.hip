@@ -222,18 +222,19 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   // 1664 columns 15 / 20 / 60 MB 12.0 / 14.4 / 34.9 -> 13.6 / 15.9 / 37.2, 1544: 48 / 60 MB 30.1 / 35.5 -> 31.5 / 38.0, with the
   // rotary embedding 896: 20 / 60 MB 17.4 / 36.7 -> 18.4 / 39.1, saved AdaLN 392: 33 / 60 MB 24.9 / 41.7 -> 26.6 / 43.8, gate 1160:
   // 20 MB 14.3 -> 15.2 (up to 8 MB, or with every lane in use, one is the faster there too: RMSNorm 1544 11.4 -> 10.5, 1536 10.4 -> 9.9).
-  // Nor where the batches divide the CUs so badly that over a quarter of them would go without a workgroup.  Backward +
+  // Nor where the batches divide the CUs so badly that over a third of them would go without a workgroup.  Backward +
   // reduction, as many as fit | whole workgroups a batch up to one a CU | rounded up to one a CU:
   //   140 x 60 x 3072 (140 of 256 CUs): residual + norm 46.3 + 18.2 | 52.4 + 17.8 | 62.1 + 18.2, gate 24.8 + 14.4 | 31.7 + 13.3 | 26.4 + 14.1
-  //   86 x 90 x 3072 (172): residual + norm 40.6 + 13.2 | 43.1 + 11.8 | 58.4 + 12.5, gate 23.2 + 9.8 | 24.0 + 9.2 | 24.9 + 9.5
+  //   86 x 90 x 3072 (172): residual + norm 40.5 + 13.3 | 41.6 + 12.0 | 58.4 + 12.5, gate 23.2 + 9.8 | 24.0 + 9.2 | 24.9 + 9.5, AdaLN
+  //     86 x 34 x 2696 16.6 + 12.0 | 15.7 + 11.0
   //   100 x 50 x 3072 (200): residual + norm 28.5 + 14.9 | 29.5 + 13.3 | 36.4 + 13.4, gate 15.9 + 10.9 | 14.8 + 10.4 | 16.5 + 10.6
-  //   43 x 45 x 3072 (215): residual + norm 15.0 + 9.2 | 13.3 + 7.2, gate 7.5 + 7.5 | 7.7 + 6.3;  AdaLN within 2 % everywhere
+  //   43 x 45 x 3072 (215): residual + norm 15.0 + 9.2 | 13.3 + 7.2, gate 7.5 + 7.5 | 7.7 + 6.3
   // (Rounded up, a few CUs have two workgroups, and all the others wait for them.)
   // Workspaces stay sized for grid_x, so that sizes asked for once hold.
   const int64_t groups = rows / rows_per_batch, per_group = groups <= cus ? cus / groups : 0;
   if (ov <= 0 && gov <= 0 && cache_resident && !narrow && (dir == kBwd || dir == kBwdSaved) && packs * 4 >= slots * 3 &&
       (res || kWideP[idx] > 1 || packs * 16 >= slots * 15 || rows * cols * 2 < (int64_t)12 << 20) &&
-      per_group * groups * 4 >= (int64_t)cus * 3)
+      per_group * groups * 3 >= (int64_t)cus * 2)
     plan->max_x = (int)per_group;
 
   // Tensors that fit the caches are read with ordinary loads (kKeep; the plan is that of the other kernel).  As fast

@@ -29,22 +29,22 @@ def partials_a_batch(lib, rows, cols, nb, op="adaln"):
     return n.value, need
 
 
-@pytest.mark.parametrize("rows,cols,nb", [(2000, 3072, 1), (9000, 3072, 3), (1200, 5128, 1), (3000, 1536, 2), (4300, 3072, 43),
+@pytest.mark.parametrize("rows,cols,nb", [(2000, 3072, 1), (9000, 3072, 3), (1200, 5128, 1), (3000, 1536, 2), (4300, 3072, 43), (86 * 34, 2696, 86),
                                           (60 * 200, 1536, 200)])
 def test_cached_backward_of_wide_rows_runs_one_workgroup_a_cu(lib, rows, cols, nb):
-    """... and no more than the size query's answer, at most a quarter of the CUs going without."""
+    """... and no more than the size query's answer, at most a third of the CUs going without."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     n, need = partials_a_batch(lib, rows, cols, nb)
-    assert n == cus // nb and n * nb * 4 >= cus * 3 and n * nb * 2 * cols * 4 <= need
+    assert n == cus // nb and n * nb * 3 >= cus * 2 and n * nb * 2 * cols * 4 <= need
 
 
-@pytest.mark.parametrize("nb", [86, 129, 140, 190, 300])
+@pytest.mark.parametrize("nb", [129, 140, 168, 300])
 def test_batches_that_divide_the_cus_badly_keep_every_cu(lib, nb):
-    """One workgroup a CU in whole workgroups a batch would leave over a quarter of the CUs without one."""
+    """One workgroup a CU in whole workgroups a batch would leave over a third of the CUs without one."""
     cus, cols, rpb = torch.cuda.get_device_properties(0).multi_processor_count, 2312, 20
-    assert cus // nb * nb * 4 < cus * 3
+    assert cus // nb * nb * 3 < cus * 2
     n, need = partials_a_batch(lib, rpb * nb, cols, nb)
-    assert n * nb >= cus * 3 // 4 and n * nb * 2 * cols * 4 <= need
+    assert n * nb * 3 >= cus * 2 and n * nb * 2 * cols * 4 <= need
 
 
 @pytest.mark.parametrize("rows,cols,capped", [(19660, 640, False), (19660, 648, False), (6009, 1664, False), (2403, 1664, True), (5208, 1920, True),
