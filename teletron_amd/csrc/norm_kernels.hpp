@@ -350,7 +350,7 @@ __global__ __launch_bounds__(64 * W * Q) void norm_fwd_wide(const FwdArgs a) {
 // which reduce_partials reads it next.  Backward + reduction, us, one group storing 32 bytes a lane with plain stores ->
 // this: AdaLN 512 x 5120 11.4 + 4.6 -> 9.2 + 4.4, 1500 x 5120 15.9 + 4.2 -> 14.1 + 4.0, RMSNorm 512 x 5120 7.2 + 3.6 ->
 // 6.2 + 3.6, residual + norm 1300 x 3072 16.6 + 6.2 -> 14.3 + 5.4.  Laid out like this but with plain stores 10.4 + 3.8,
-// with non-temporal ones ("sc1 nt") 9.2 + 5.7 in the first of these.
+// with "nt" ones 9.4 + 5.6 and with "sc1 nt" 9.2 + 5.7 in the first of these.
 template <int NACC, int W, int P, int Q, bool ODD = false>
 __device__ __forceinline__ void wide_write_partials(const float (&acc)[NACC][P][8], float* partials, int64_t b, int C,
                                                     int q, int w, int lane) {

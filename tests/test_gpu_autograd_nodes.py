@@ -83,6 +83,26 @@ def test_the_native_node_runs(monkeypatch, name):
         call()
 
 
+def test_what_the_graph_shows():
+    """Edges, hooks and names of a native node as of any other; a subclass has the Python node with what Python keeps there."""
+    import teletron_amd as T
+    x, w = leaf(B, S, C, seed=0), leaf(C, seed=1)
+    y = T.RMSNormModelFunction.apply(x, w, EPS, C)
+    node, seen = y.grad_fn, []
+    assert "RMSNormModelFunction" in node.name() and len(node.next_functions) == 2 and node.metadata == {}
+    assert not hasattr(node, "saved_tensors")
+    node.register_prehook(lambda g: seen.append(g[0].shape))
+    node.register_hook(lambda gi, go: seen.append(len(gi)))
+    y.sum().backward()
+    assert seen == [y.shape, 2]
+
+    class Mine(T.RMSNormModelFunction):
+        pass
+
+    z = Mine.apply(x, w, EPS, C)
+    assert torch.equal(z, y) and [t.shape for t in z.grad_fn.saved_tensors] == [x.shape, w.shape]
+
+
 @pytest.mark.parametrize("name", NAMES)
 @pytest.mark.parametrize("how", ["dense", "expanded", "misaligned"])
 def test_same_bits_for_any_gradient(monkeypatch, name, how):
