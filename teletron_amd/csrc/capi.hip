@@ -144,13 +144,21 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   const int slots = narrow ? kNarrowL[idx] : 64 * kWideW[idx] * kWideP[idx];
   const bool full = (slots == packs);
   const bool cache_resident = rows * cols * 2 < (int64_t)64 << 20;
+  if (res && (narrow || kind != kAdaLN || dir == kBwdSaved || dir == kFwdXn)) return TT_ERR_UNSUPPORTED;
+  if (rope && (kind != kRMS || dir == kBwdSaved || dir == kFwdXn)) return TT_ERR_UNSUPPORTED;
+  if (dir == kFwdXn && kind != kAdaLN) return TT_ERR_UNSUPPORTED;
   // a row of whole 128-byte lines or not: see enum Rows
   int mode = odd ? kOdd : full ? kFull : (cols * 2) % 128 == 0 || force == kMasked ? kMasked : kRagged;
+  int cus = 0, per_cu = 0;
+  int rc = current_device_cus(&cus);
+  if (rc != TT_OK) return rc;
+  // beyond the caches one CU in 32 is left without a workgroup
+  const int usable_cus = !cache_resident && cus >= 32 ? cus - cus / 32 : cus;
+  const int64_t groups = rows / rows_per_batch;
+  const bool uneven = !cache_resident && usable_cus / groups * groups * 20 < (int64_t)usable_cus * 19;
   if (mode == kRagged)
-    mode |= (cache_resident ? kCached : 0) | (packs * 4 < slots * 3 ? kIdle : packs * 16 >= slots * 15 ? kDense : 0);
-  if (res && (narrow || kind != kAdaLN || dir == kBwdSaved || dir == kFwdXn)) return TT_ERR_UNSUPPORTED;
+    mode |= (cache_resident ? kCached : uneven ? kUneven : 0) | (packs * 4 < slots * 3 ? kIdle : packs * 16 >= slots * 15 ? kDense : 0);
   if (rope) {
-    if (kind != kRMS || dir == kBwdSaved || dir == kFwdXn) return TT_ERR_UNSUPPORTED;
     // Token mode saves table look-ups, but its tiles are three times those of the look-up per row: on tensors
     // that the caches hold, its forward waits for one tile a CU, and with four loads a wave it is slower
     // throughout; its backward has fewer waves resident (237 registers against 138).  Kernel us per token | per row:
@@ -161,14 +169,10 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
     //            16 of 128,         1: 5.5 | 4.7      4: 5.6 | 5.2    12: 9.7 | 8.3    32: 19.7 | 17.5    63: 35.7 | 35.6
     // (48 heads of 128 as 24; 64 columns as 128 with half the heads.  Beyond the caches: see rope_token_R.)
     if (narrow && rope_heads > 0 && cache_resident) {
-      int cus = 0;
-      const int rc = current_device_cus(&cus);
-      if (rc != TT_OK) return rc;
       const int r = rope_token_R(kNarrowL[idx], rope_heads);
       if (dir == kBwd || r == 4 || rows < (int64_t)cus * rope_token_NW(r) * r * (kWave / kNarrowL[idx])) rope_heads = 0;
     }
   }
-  if (dir == kFwdXn && kind != kAdaLN) return TT_ERR_UNSUPPORTED;
   const auto pick = [&](int rows_kind) -> KernelInfo {
     if (res == 2) return resnorm_gated_kernel(dir == kBwd, idx, rows_kind);
     if (res) return resnorm_plain_kernel(dir == kBwd, idx, rows_kind);
@@ -185,9 +189,6 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   const KernelInfo k = pick(mode);
   if (!k.fn) return TT_ERR_UNSUPPORTED;
 
-  int cus = 0, per_cu = 0;
-  int rc = current_device_cus(&cus);
-  if (rc != TT_OK) return rc;
   rc = resident_wgs_per_cu(k, &per_cu);
   if (rc != TT_OK) return rc;
   // HBM streams fastest with a modest number of requests in flight: measured on MI355X,
@@ -195,7 +196,6 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   // column of a CU (waves x loads per lane) and streamed tensor, falls off by 10-20 % at full
   // occupancy, and is a few percent better with one CU in 32 left without a workgroup.
   // Tensors that fit the caches take what fits a CU, or one workgroup (max_x below).
-  int usable_cus = cus;
   if (!cache_resident) {
     const int per_wg = (k.threads / kWave) * k.lane_loads;
     // two streamed inputs (backward kernels, both gate kernels) or one (normalisation forward)
@@ -204,7 +204,6 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
     int want = (2 * target + per_wg) / (2 * per_wg);
     if (want < 1) want = 1;
     if (want < per_cu) per_cu = want;
-    if (cus >= 32) usable_cus = cus - cus / 32;
   }
   const int ov = g_wgs_per_cu_override.load(std::memory_order_relaxed);
   const int gov = g_grid_override.load(std::memory_order_relaxed);
@@ -231,7 +230,7 @@ int make_plan(int kind, Dir dir, int64_t rows, int64_t cols, int64_t rows_per_ba
   //   43 x 45 x 3072 (215): residual + norm 15.0 + 9.2 | 13.3 + 7.2, gate 7.5 + 7.5 | 7.7 + 6.3
   // (Rounded up, a few CUs have two workgroups, and all the others wait for them.)
   // Workspaces stay sized for grid_x, so that sizes asked for once hold.
-  const int64_t groups = rows / rows_per_batch, per_group = groups <= cus ? cus / groups : 0;
+  const int64_t per_group = cus / groups;
   if (ov <= 0 && gov <= 0 && cache_resident && !narrow && (dir == kBwd || dir == kBwdSaved) && packs * 4 >= slots * 3 &&
       (res || kWideP[idx] > 1 || packs * 16 >= slots * 15 || rows * cols * 2 < (int64_t)12 << 20) &&
       per_group * groups * 3 >= (int64_t)cus * 2)

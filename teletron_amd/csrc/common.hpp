@@ -62,10 +62,12 @@ enum Rows : int {
   // so that tensors which fit the caches stay there for the next kernel that reads them.
   kKeep = 4,
   // Added to kRagged, for the row groups a workgroup (ragged_fwd_Q and the rules after it): the tensor fits the caches;
-  // over a quarter, or at most a sixteenth, of the lane slots hold no pack.
+  // over a quarter, or at most a sixteenth, of the lane slots hold no pack; it is beyond the caches, and one workgroup
+  // a CU is not to be had in whole workgroups a batch.
   kCached = 8,
   kIdle = 16,
   kDense = 32,
+  kUneven = 64,
 };
 constexpr int row_mode(int rows) { return rows & 3; }
 constexpr bool keeps(int rows) { return (rows & kKeep) != 0; }

@@ -87,6 +87,8 @@ constexpr int bwd_wide_Q(int W, int P) {
 //                      (520: 167 -> 191, 776: 142 -> 145, 968: 136 -> 138)
 //   AdaLN and RMSNorm forward, four groups of four waves: 1928 columns 149 / 142 -> 136 / 133,  2040: 153 / 150 -> 138 / 135; with more
 //                      lanes idle they lose, most at 80 MB (1544: 29.3 / 28.6 -> 32.8 / 31.6, 1800: 29.7 / 28.8 -> 31.2 / 29.9)
+//                      Neither of the last with batches that leave CUs idle when each has whole workgroups of this size: 150 MB, 86 / 140
+//                      batches, 600 columns 82 / 85 -> 97 / 115, 1992: 64 / 60 -> 69 / 77 (residual + norm 1992 125 / 124 -> 132 / 130)
 //   and backward       3080: 226 / 201 -> 193 / 191,  3536: 204 / 200 -> 188 / 189,  4088: 197 / 195 -> 190 / 187
 //   RMSNorm backward   520 (200 MB) 131 -> 115,  648: 114 -> 103,  776: 104 -> 99,  1016: 99 -> 100,  968 (12 MB) 9.0 -> 8.2; in the caches
 //                      with over a quarter of the lanes idle two smaller workgroups a CU are better (520, 31 MB: 18.6 -> 20.6)
@@ -99,6 +101,7 @@ constexpr int bwd_wide_Q(int W, int P) {
 // residual backward (170 registers and more).
 constexpr int ragged_fwd_Q(Kind kind, int W, int P, int rows) {
   if (row_mode(rows) != kRagged) return fwd_wide_Q(W, P);
+  if (P == 1 && (W == 2 || W == 4) && (rows & kUneven)) return fwd_wide_Q(W, P);
   if (P == 1 && W == 2) return kind == kAdaLN || (rows & (kCached | kDense)) ? 8 : fwd_wide_Q(W, P);
   if (P == 1 && W == 4) return rows & kDense ? 4 : fwd_wide_Q(W, P);
   return kind == kAdaLN && P == 2 && W == 5 ? 3 : fwd_wide_Q(W, P);
@@ -174,6 +177,7 @@ KernelInfo info_bwd_narrow() {
   if (row_mode(rows) == kRagged)                                                       \
     return keeps(rows)      ? TT_LANES(INFO, kRagged | kKeep | kCached, __VA_ARGS__)   \
            : rows & kCached ? TT_LANES(INFO, kRagged | kCached, __VA_ARGS__)           \
+           : rows & kUneven ? TT_LANES(INFO, kRagged | kUneven, __VA_ARGS__)           \
                             : TT_LANES(INFO, kRagged, __VA_ARGS__);                    \
   TT_LINES(INFO, (), __VA_ARGS__)
 #define TT_ROWS_ODD(INFO, ...)                                      \
@@ -391,7 +395,8 @@ constexpr int res_bwd_Q(int W, int P, bool gated) {
 }
 constexpr int ragged_res_fwd_Q(int W, int P, int rows, bool gated) {   // see ragged_fwd_Q
   if (row_mode(rows) != kRagged || P != 1 || (rows & kCached)) return res_fwd_Q(W, P);
-  return W == 4 ? 4 : gated && W == 3 ? 5 : res_fwd_Q(W, P);
+  if (!gated) return W == 4 && !(rows & kUneven) ? 4 : res_fwd_Q(W, P);
+  return W == 4 ? 4 : W == 3 ? 5 : res_fwd_Q(W, P);
 }
 template <bool GATED, int W, int P, int ROWS>
 KernelInfo info_res_fwd() {

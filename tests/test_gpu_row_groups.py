@@ -39,3 +39,15 @@ def test_ragged_rows(cols, nb, rpb):
     check_gate(cols, nb, rpb)
     for gated in (False, True):
         check_residual(cols, nb, rpb, gated, affine=False)
+
+
+@pytest.mark.parametrize("cols", [1000, 1992])
+def test_same_rows_with_batches_that_divide_the_cus_badly(cols):
+    """Beyond the caches their workgroups hold fewer row groups: the same bits a row as with one batch."""
+    from teletron_amd import ops
+    nb = 140
+    rpb = (70 << 20) // (2 * cols * nb) + 1
+    x = torch.randn(nb * rpb, cols, generator=torch.Generator(DEV).manual_seed(cols), device=DEV).to(torch.bfloat16)
+    a, b = (rand_bf16(1, cols, seed=i, scale=0.3).to(DEV) for i in range(2))
+    one = ops.adaln_forward(x, a, b, 1e-6)
+    assert torch.equal(ops.adaln_forward(x, a.expand(nb, cols).contiguous(), b.expand(nb, cols).contiguous(), 1e-6), one)
